@@ -205,7 +205,7 @@ namespace qcore
             fused_->set_stage_stream(stage_stream_ != 0);
             fused_->set_check(planner_check_ != 0);
         }
-        work_len_ = qsv::reduce_workspace(count) + 16;
+        work_len_ = std::max(qsv::reduce_workspace(count), qsv::expz_workspace(count)) + 16;
         qsv::check(hipMalloc((void **)&work_, work_len_ * sizeof(double)), "hipMalloc workspace");
         allocated_ = true;
         set_zero_state();
@@ -877,7 +877,7 @@ namespace qcore
         need_alloc();
         flush();
         prof_begin(QCS_EXT_K_REDUCE, (c64_state() ? 8.0 : 16.0) * (1ull << n_));
-        with_state([&](auto *st) { qsv::reduce_probs(stream_, st, uint64_t(1) << n_, 0, work_, pinned_); });
+        with_state([&](auto *st) { qsv::reduce_probs(stream_, st, uint64_t(1) << n_, work_, pinned_); });
         prof_end();
         return pinned_[0];
     }
@@ -888,13 +888,11 @@ namespace qcore
         flush();
         if (count < 0 || count > n_ || (count > 0 && out == nullptr))
             throw std::runtime_error("expect_z count out of range");
-        for (int q = 0; q < count; ++q)
-        {
-            prof_begin(QCS_EXT_K_REDUCE, (c64_state() ? 8.0 : 16.0) * (1ull << n_));
-            with_state([&](auto *st) { qsv::reduce_probs(stream_, st, uint64_t(1) << n_, uint64_t(1) << l2p_[q], work_, pinned_); });
-            prof_end();
-            out[q] = pinned_[0];
-        }
+        if (count == 0)
+            return;
+        prof_begin(QCS_EXT_K_REDUCE, (c64_state() ? 8.0 : 16.0) * (1ull << n_));
+        with_state([&](auto *st) { qsv::expect_z(stream_, st, n_, work_, pinned_, l2p_.data(), count, out); });
+        prof_end();
     }
 
     void Simulator::set_local_qubits(int nl)

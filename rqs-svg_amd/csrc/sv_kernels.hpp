@@ -102,9 +102,15 @@ namespace qsv
     // {p0,p1} over the subspace `sub` (p1 at index | tbit); host out[2], stream synchronised.
     template <class A>
     void reduce_pair_probs(hipStream_t s, const A *state, const Subspace &sub, uint64_t tbit, uint64_t nitems, double *work, double out[2]);
-    // canonical sum of p(i) (negated where bit `zbit` is set, if zbit != 0) over all amplitudes
+    // canonical sum of p(i) over all amplitudes
     template <class A>
-    void reduce_probs(hipStream_t s, const A *state, uint64_t count, uint64_t zbit, double *work, double *out);
+    void reduce_probs(hipStream_t s, const A *state, uint64_t count, double *work, double *out);
+    // out[i] = canonical sum of p negated where physical bit bits[i] is set, i < nbits, all
+    // from one read of the 2^n amplitudes; work holds expz_workspace(2^n) doubles, pinned 64
+    // doubles of pinned host memory (the last kernel writes there).  Synchronises `s`.
+    uint64_t expz_workspace(uint64_t count);
+    template <class A>
+    void expect_z(hipStream_t s, const A *state, int n, double *work, double *pinned, const int *bits, int nbits, double *out);
     // out[0..1] = <a|b> (canonical tree per component), out[2] = max |a_i - b_i|
     uint64_t overlap_workspace(uint64_t count);
     template <class A, class B>
