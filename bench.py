@@ -1,5 +1,5 @@
 #!/usr/bin/env python3
-"""Benchmark: 30-qubit complex128 brick circuit on one MI355X (plain per-gate method).
+"""Benchmark: 30-qubit complex128 brick circuit on one MI355X (plain method).
 
 One step = zero state + 24 brick layers (U3 on all 30 qubits, CZ on even/odd neighbour
 pairs alternating) with 4 three-control X gates (at least one operand among the top 6
@@ -8,16 +8,17 @@ calls on a 16 GiB state.  `value` is gates per second over the timed steps; the 
 resident in HBM throughout.
 
 Also reported:
-  roofline      -- the dominant kernel (the 2x2 pair kernel that runs U3 and MCX), its
-                   algorithmic bytes per launch (2 * 16 B * amplitudes it may change) over
-                   its average duration from HIP events recorded around each launch on the
-                   simulator's stream during the timed steps, against 8 TB/s;
+  roofline      -- the dominant kernel (the circuit pass, which applies the gates whose
+                   targets lie in its tiles in one sweep of the state), its algorithmic
+                   bytes per launch (2 * 16 B * amplitudes) over its average duration
+                   from HIP events recorded around each launch on the simulator's stream
+                   during the timed steps, against 8 TB/s;
   cpu_baseline  -- the oracle (the reference's plain method restated in C++/OpenMP) on the
                    host cores, on a bounded sample of the same workload;
   fused_c64     -- the precision form on the 32-qubit brick circuit of depth 32 (complex64
                    state, gates fused into k=5 blocks on FP32 MFMA; fused_c64_bf16x3 the
                    same on BF16x3 split-precision MFMA) against the plain FP64
-                   per-gate path on the same GPU: time of each, speedup, and fidelity /
+                   method on the same GPU: time of each, speedup, and fidelity /
                    max |d amp| of the fused state against the FP64 state (both resident in
                    HBM, compared on the GPU in FP64);
   batch         -- 512 variational circuits of 12-22 qubits in one autotuned hipGraph
@@ -52,8 +53,8 @@ def log(msg):
 
 
 def traffic_from_profiles():
-    """HBM bytes per pair-kernel launch measured with rocprofv3 PMC counters, if committed."""
-    f = REPO / "profiles" / "pair_kernel_brick30_traffic.json"
+    """HBM bytes per pass measured with rocprofv3 PMC counters, if committed."""
+    f = REPO / "profiles" / "pass_kernel_brick30_traffic.json"
     if not f.exists():
         return None
     try:
@@ -92,8 +93,8 @@ def cpu_baseline(n, circ, budget_s=20.0):
 def small_leg(n=20, layers=20, shots=1024):
     """The reference's CPU-runnable case on one GPU against the oracle on the host cores:
     20 qubits complex128, H then a CNOT chain (GHZ), 20 layers of U3 on every qubit and CZ
-    on a random perfect matching, 1024 samples.  Both run the same API calls (one per gate);
-    the timed region is the circuit from |0...0> plus the sampling, states allocated."""
+    on a random perfect matching, 1024 samples.  Both run the same API calls; the
+    timed region is the circuit from |0...0> plus the sampling, states allocated."""
     circ = circuits.ghz_u3_cz(n, layers, seed=CIRCUIT_SEED + 11)
     res = {}
     for name, lib in (("gpu", pyqcs.gpu_library()), ("cpu", pyqcs.oracle_library())):
@@ -118,7 +119,7 @@ def small_leg(n=20, layers=20, shots=1024):
         f"CPU oracle {tc * 1e3:.1f} ms on {cores} cores ({tc / tg:.1f}x); max|d amp| {diff:.1e}, "
         f"{same}/{shots} samples identical")
     return {"config": f"{n} qubits complex128: H + CNOT chain, {layers} layers U3 on all + CZ on a "
-                      f"random matching, {shots} samples (plain method, one kernel per gate)",
+                      f"random matching, {shots} samples (plain method)",
             "gates": len(circ), "shots": shots, "gpu_s": tg, "gpu_gates_per_s": len(circ) / tg,
             "cpu_oracle_s": tc, "cpu_cores": cores, "gpu_vs_cpu": tc / tg,
             "max_abs_diff_amp": diff, "samples_identical": same}
@@ -498,12 +499,11 @@ def planner_leg(n, depth, record_count, k=4, fixed_sweep=False):
     default stage plan, and the plan the model picks (taken only when its predicted gain
     over the default exceeds the model's error; one run each, so an override runs as the
     model picked it, before the planner's measured check has compared it with the default)
-    -- and each output compared with the plain per-gate complex128 path (one kernel per
-    gate, the reference's method) on a second state in HBM."""
+    -- and each output compared with the plain complex128 method on a second state in HBM."""
     lib = pyqcs.gpu_library()
     model, info = pyqcs.train_cost_model(lib, 2, k, (26, 28, 30, 32), record_count, (26, 28, 30), log=log)
     out = {"config": f"complex128 fused blocks (k<={k}), {n}-qubit QFT on a random brick layer and "
-                     f"{n}-qubit brick depth {depth}; outputs against the plain per-gate complex128 path",
+                     f"{n}-qubit brick depth {depth}; outputs against the plain complex128 method",
            "cost_model": info}
     prep_qft = circuits.brick(n, 1, seed=CIRCUIT_SEED + 9)
     work = {"qft": (prep_qft, circuits.qft(n)), "brick": ((), circuits.brick(n, depth, seed=CIRCUIT_SEED + 5))}
@@ -747,10 +747,8 @@ def main():
         log(f"calibration norm {sim.norm():.3f}")  # reads 16 * 2^n bytes
     sim.close()
 
-    pair = prof.get("pair", {"launches": 1, "seconds": 1, "bytes": 0})
-    avg_s = pair["seconds"] / pair["launches"]
-    bytes_per_launch = pair["bytes"] / pair["launches"]
-    achieved = bytes_per_launch / avg_s / 1e9
+    passes = prof.get("fused", {"launches": 1, "seconds": 1, "bytes": 0})
+    achieved = passes["bytes"] / passes["seconds"] / 1e9
     traffic = traffic_from_profiles()
 
     result = {
@@ -772,19 +770,21 @@ def main():
                         f"reduction + {args.shots} samples",
             "qubits": n, "depth": args.depth, "gates": ngates, "shots": args.shots,
             "circuit_seed": CIRCUIT_SEED, "sample_seed": SAMPLE_SEED,
-            "method": "plain: one kernel per gate",
+            "method": "plain: whole circuit per call, one kernel per sweep of the state",
+            "sweeps_per_step": passes["launches"] / args.steps,
         },
         "roofline": {
             "bound": "hbm",
-            "kernel": "k_pair<1, true> + k_pair_low<2, true> (U3 / MCX launches, HIP events over the timed steps)",
+            "kernel": "k_pass (HIP events over the timed steps)",
             "achieved": achieved,
             "peak": HBM_PEAK / 1e9,
             "unit": "GB/s",
             "frac": achieved / (HBM_PEAK / 1e9),
             "traffic": traffic,
         },
+        # what one sweep per gate would move, over the time taken; and what was moved
         "sweeps_per_s": alg_bytes / (2 * 16 * (1 << n)) * args.steps / wall,
-        "hbm_frac_whole_step": alg_bytes * args.steps / wall / HBM_PEAK,
+        "hbm_frac_whole_step": sum(v["bytes"] for v in prof.values()) / wall / HBM_PEAK,
     }
     if not args.no_subsystems:
         result["subsystems"] = subsystem_leg(n)

@@ -104,6 +104,19 @@ int qcs_ext_set_renormalize(qcs_simulator *sim, int enable);
  * (src/qcs.cu:2206-2332).  Default: all qubits local. */
 int qcs_ext_set_local_qubits(qcs_simulator *sim, bit_num_t num_local_qubits);
 
+/* A whole circuit in one call: gate i is qcs_simulator_gate_<names[name_of[i]]>, taking the
+ * next num_params[name_of[i]] entries of params and the next num_targets[i], num_negctrls[i]
+ * and num_ctrls[i] entries of targets, negctrls and ctrls (params must not be NULL).
+ * The state afterwards is what the same calls one by one leave, up to FP64 rounding (gates on
+ * different qubits may be applied in another order), and all work is queued on the stream on
+ * return.  Without measured qubits, complex128 states (precision 0) take runs of gates in
+ * passes of several gates per sweep.  *num_applied: gates applied; on failure the gates
+ * before the refused one have been. */
+int qcs_ext_run_circuit(qcs_simulator *sim, int32_t count, const char *const *names, const int32_t *num_params,
+                        const uint8_t *name_of, const uint8_t *num_targets, const uint8_t *num_negctrls,
+                        const uint8_t *num_ctrls, const bit_num_t *targets, const bit_num_t *negctrls,
+                        const bit_num_t *ctrls, const double *params, int32_t *num_applied);
+
 /* Current physical -> logical mapping. */
 int qcs_ext_get_mapping(qcs_simulator *sim, bit_num_t *perm_p2l, bit_num_t count);
 

@@ -1320,6 +1320,25 @@ extern "C"
             put(total, c.probability_total());
         });
     }
+    int qcs_ext_run_circuit(qcs_simulator *s, int32_t count, const char *const *names, const int32_t *num_params, const uint8_t *name_of, const uint8_t *nt, const uint8_t *nng, const uint8_t *nps, const bit_num_t *targets, const bit_num_t *negctrls, const bit_num_t *ctrls, const double *params, int32_t *applied)
+    {
+        return guard([&] {
+            if (applied == nullptr)
+                throw std::runtime_error("result pointer must not be NULL");
+            *applied = 0;
+            if (count < 0 || (count > 0 && (!names || !num_params || !name_of || !nt || !nng || !nps || !params)))
+                throw std::runtime_error("run_circuit: bad arrays");
+            for (int32_t i = 0; i < count; ++i)
+            {
+                run_gate(s, names[name_of[i]], params, targets, nt[i], negctrls, nng[i], ctrls, nps[i]);
+                targets += nt[i];
+                negctrls += nng[i];
+                ctrls += nps[i];
+                params += num_params[name_of[i]];
+                ++*applied;
+            }
+        });
+    }
     int qcs_ext_norm(qcs_simulator *s, double *norm)
     {
         return guard([&] {

@@ -415,6 +415,55 @@ extern "C"
     int qcs_ext_sample(qcs_simulator *s, uint64_t sd, uint64_t shots, uint64_t *out) { return guard([&] { core(s).sample(sd, shots, out); }); }
     int qcs_ext_sample_noalloc(qcs_simulator *s, uint64_t sd, uint64_t shots, uint64_t *out) { return guard([&] { core(s).sample_noalloc(sd, shots, out); }); }
     int qcs_ext_probability_total(qcs_simulator *s, double *total) { return guard([&] { put(total, core(s).probability_total()); }); }
+    int qcs_ext_run_circuit(qcs_simulator *s, int32_t count, const char *const *names, const int32_t *num_params, const uint8_t *name_of, const uint8_t *nt, const uint8_t *nng, const uint8_t *nps, const bit_num_t *targets, const bit_num_t *negctrls, const bit_num_t *ctrls, const double *params, int32_t *applied)
+    {
+        return guard([&] {
+            if (applied == nullptr)
+                throw std::runtime_error("result pointer must not be NULL");
+            *applied = 0;
+            auto &c = core(s);
+            if (count < 0 || (count > 0 && (!names || !num_params || !name_of || !nt || !nng || !nps || !params)))
+                throw std::runtime_error("run_circuit: bad arrays");
+            std::vector<qcore::CircuitGate> gates;
+            gates.reserve(size_t(count));
+            std::string refused;
+            bool stop = false;
+            for (int32_t i = 0; i < count && !stop; ++i)
+            {
+                try
+                {
+                    qcore::CircuitGate g;
+                    g.spec = qcore::make_gate(names[name_of[i]], params);
+                    g.targets = vec(targets, nt[i]);
+                    g.neg = vec(negctrls, nng[i]);
+                    g.pos = vec(ctrls, nps[i]);
+                    targets += nt[i];
+                    negctrls += nng[i];
+                    ctrls += nps[i];
+                    params += num_params[name_of[i]];
+                    gates.push_back(std::move(g));
+                }
+                catch (const std::exception &e)
+                {
+                    refused = e.what();
+                    stop = true;
+                }
+            }
+            size_t done = 0;
+            try
+            {
+                c.run_circuit(gates, &done);
+            }
+            catch (...)
+            {
+                *applied = int32_t(done);
+                throw;
+            }
+            *applied = int32_t(done);
+            if (stop)
+                throw std::runtime_error(refused);
+        });
+    }
     int qcs_ext_norm(qcs_simulator *s, double *norm) { return guard([&] { put(norm, core(s).norm()); }); }
     int qcs_ext_expect_z(qcs_simulator *s, double *out, int count) { return guard([&] { core(s).expect_z(out, count); }); }
     int qcs_ext_set_renormalize(qcs_simulator *s, int en) { return guard([&] { core(s).set_renormalize(en != 0); }); }

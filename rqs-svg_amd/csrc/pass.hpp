@@ -1,0 +1,81 @@
+// Circuit passes, host side: gates lowered to controlled 2x2 and phase operations, grouped
+// into sweeps of the state (pass_kernels.hpp) and into the rounds of each sweep.
+#pragma once
+#include "pass_kernels.hpp"
+#include "simulator.hpp"
+
+#include <vector>
+
+namespace qcore
+{
+    // What the lowering multiplies together is rounded to double once, when it is written.
+    using cl = std::complex<long double>;
+
+    // An operation on qubit t, or (t < 0) a phase, on the amplitudes whose index matches
+    // (cmask, cval); physical qubits.  kind: kPassRot, kPassFlip, kPassCross or kPassHad.
+    // pre: a phase of qubit t's |1> that comes first, on every amplitude.
+    struct PassGate
+    {
+        int t;
+        uint32_t kind;
+        uint64_t cmask, cval;
+        double m[4]; // as the kind's PassOp, or the phase in m[0..1]
+        cd pre = 1.0;
+    };
+
+    // Lowers a gate list to PassGates.  Uncontrolled 1-qubit gates are multiplied together per
+    // qubit (80-bit) and written as phase * rotation * phase only when another gate needs the
+    // qubit; the trailing phase waits on, since it commutes with controls and phases.  A
+    // 2-target gate becomes 2x2s between CNOTs (its matrix mixes amplitudes in pairs).
+    class PassLowering
+    {
+    public:
+        explicit PassLowering(int n) : one_(n) {}
+        // false, with nothing changed, for a gate that has no such form
+        bool add(const ResolvedGate &g);
+        // the operations of every gate added
+        std::vector<PassGate> finish();
+
+    private:
+        struct One
+        {
+            bool any = false;
+            cl m[4];
+        };
+        std::vector<One> one_; // pending 1-qubit gates, per qubit
+        cl global_ = 1.0;
+        std::vector<PassGate> out_;
+
+        void mul(int q, cl a, cl b, cl c, cl d);
+        void touch_z(int q);
+        cd touch_x(int q);
+        void phase(uint64_t cmask, uint64_t cval, cl p);
+        void two_by_two(int t, uint64_t cmask, uint64_t cval, cd a, cd b, cd c, cd d);
+        void flip(int t, uint64_t cmask, uint64_t cval) { two_by_two(t, cmask, cval, 0.0, 1.0, 1.0, 0.0); }
+    };
+
+    struct PassPlan
+    {
+        struct Pass
+        {
+            uint8_t tq[16];
+            uint32_t first_round, nrounds;
+        };
+        int m = 0;
+        std::vector<Pass> passes;
+        std::vector<qsv::PassRound> rounds;
+        std::vector<qsv::PassOp> ops; // the rounds' operations, then kPassOpPad unused ones
+        // rough cost in FP64 instructions per amplitude and lane (for choosing a path)
+        double work = 0;
+    };
+
+    // Tile bits of a pass over a state of n qubits.
+    int pass_tile_bits(int n);
+
+    // Sweeps that apply `gates` in an order equivalent to theirs: a gate may pass a deferred
+    // one only if on every shared qubit both act as a control or a phase.  A 2x2's target has
+    // to be a tile qubit; controls and phases need not be.  amp_bytes: 16 or 8 (complex64),
+    // which decides the low qubits that the first and last round of a sweep keep in the
+    // thread index, so that loads and stores cover whole lines.
+    PassPlan plan_passes(const std::vector<PassGate> &gates, int n, int m, int amp_bytes);
+} // namespace qcore

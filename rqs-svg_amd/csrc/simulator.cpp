@@ -17,6 +17,7 @@
 #include "simulator.hpp"
 
 #include "fused.hpp"
+#include "pass.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -71,7 +72,7 @@ namespace qcore
     {
         qsv::check(hipGetDevice(&device_), "hipGetDevice");
         qsv::check(hipStreamCreate(&stream_), "hipStreamCreate");
-        qsv::check(hipHostMalloc((void **)&pinned_, 64 * sizeof(double), hipHostMallocDefault), "hipHostMalloc");
+        qsv::check(hipHostMalloc((void **)&pinned_, kPinnedResults * sizeof(double) + kSmallProgram, hipHostMallocDefault), "hipHostMalloc");
         std::random_device rd; // src/qcs.cu:1845-1852
         seed_ = rd();
         engine_.seed(seed_);
@@ -97,6 +98,8 @@ namespace qcore
             (void)hipEventDestroy(e);
         if (open_a_)
             (void)hipEventDestroy(open_a_);
+        if (prog_copied_)
+            (void)hipEventDestroy(prog_copied_);
         if (pinned_)
             (void)hipHostFree(pinned_);
         if (stream_)
@@ -206,7 +209,9 @@ namespace qcore
             fused_->set_check(planner_check_ != 0);
         }
         work_len_ = std::max(qsv::reduce_workspace(count), qsv::expz_workspace(count)) + 16;
-        qsv::check(hipMalloc((void **)&work_, work_len_ * sizeof(double)), "hipMalloc workspace");
+        // the reductions' workspace, and behind it the device copy of a small pass program
+        work_len_ = (work_len_ + 31) & ~uint64_t(31);
+        qsv::check(hipMalloc((void **)&work_, work_len_ * sizeof(double) + kSmallProgram), "hipMalloc workspace");
         allocated_ = true;
         set_zero_state();
     }
@@ -229,6 +234,12 @@ namespace qcore
             (void)hipFree(work_);
             work_ = nullptr;
         }
+        if (prog_dev_)
+            (void)hipFree(prog_dev_);
+        if (prog_host_)
+            (void)hipHostFree(prog_host_);
+        prog_dev_ = prog_host_ = nullptr;
+        prog_cap_ = 0;
         for (auto p : levels_)
             (void)hipFree(p);
         levels_.clear();
@@ -472,6 +483,149 @@ namespace qcore
             apply_resolved(r);
         m0_ = keep[0];
         m1_ = keep[1];
+    }
+
+    ResolvedGate Simulator::resolve(const GateSpec &g, const std::vector<int> &targets, const std::vector<int> &neg, const std::vector<int> &pos) const
+    {
+        if ((int)targets.size() != g.ntargets)
+            throw std::runtime_error(fmt("gate needs %d target qubit(s), %d given", g.ntargets, (int)targets.size()));
+        check_operands(targets, neg, pos);
+        ResolvedGate r;
+        r.spec = g;
+        for (int q : targets)
+            r.tphys.push_back(l2p_[q]);
+        for (int q : pos)
+            r.pphys.push_back(l2p_[q]);
+        for (int q : neg)
+            r.nphys.push_back(l2p_[q]);
+        return r;
+    }
+
+    void Simulator::run_circuit(const std::vector<CircuitGate> &gates, size_t *applied)
+    {
+        need_alloc();
+        *applied = 0;
+        // Measured qubits (implicit controls, zeroed branches), a window of local qubits and
+        // the fused modes (their own queue) go gate by gate.
+        if (precision_ != 0 || !m0_.empty() || !m1_.empty() || n_local_ != n_)
+        {
+            for (const auto &g : gates)
+            {
+                operate(g.spec, g.targets, g.neg, g.pos);
+                ++*applied;
+            }
+            return;
+        }
+        constexpr size_t kRun = 4096; // gates planned together: bounds the program's size
+        std::vector<ResolvedGate> run;
+        for (size_t i = 0; i < gates.size();)
+        {
+            run.clear();
+            std::string refused;
+            bool stop = false;
+            for (; i < gates.size() && run.size() < kRun; ++i)
+            {
+                try
+                {
+                    run.push_back(resolve(gates[i].spec, gates[i].targets, gates[i].neg, gates[i].pos));
+                }
+                catch (const std::exception &e)
+                {
+                    refused = e.what();
+                    stop = true;
+                    break;
+                }
+            }
+            apply_run(run);
+            *applied += run.size();
+            if (stop)
+                throw std::runtime_error(refused);
+        }
+    }
+
+    void Simulator::reserve_program(size_t bytes)
+    {
+        if (prog_pending_)
+        { // the last program's upload still reads the staging area
+            qsv::check(hipEventSynchronize(prog_copied_), "hipEventSynchronize");
+            prog_pending_ = false;
+        }
+        if (!prog_copied_)
+            qsv::check(hipEventCreateWithFlags(&prog_copied_, hipEventDisableTiming), "hipEventCreate");
+        if (bytes <= kSmallProgram || bytes <= prog_cap_)
+            return;
+        // queued passes may still read the device copy
+        qsv::check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
+        if (prog_dev_)
+            (void)hipFree(prog_dev_);
+        if (prog_host_)
+            (void)hipHostFree(prog_host_);
+        prog_dev_ = prog_host_ = nullptr;
+        prog_cap_ = 0;
+        size_t cap = kSmallProgram;
+        while (cap < bytes)
+            cap *= 2;
+        qsv::check(hipMalloc(&prog_dev_, cap), "hipMalloc pass program");
+        qsv::check(hipHostMalloc(&prog_host_, cap, hipHostMallocDefault), "hipHostMalloc pass program");
+        prog_cap_ = cap;
+    }
+
+    void Simulator::apply_run(const std::vector<ResolvedGate> &gates)
+    {
+        if (gates.empty())
+            return;
+        state_changed();
+        const int m = pass_tile_bits(n_);
+        PassLowering lowering(n_);
+        double bytes = 0; // what one kernel per gate would move, in sweeps of the state
+        bool lowered = gates.size() > 1;
+        for (size_t i = 0; lowered && i < gates.size(); ++i)
+        {
+            const ResolvedGate &g = gates[i];
+            const int nc = int(g.pphys.size() + g.nphys.size());
+            // a controlled 2x2 needs 4 register bits clear of its controls
+            lowered = lowering.add(g) && nc + int(g.tphys.size()) <= m - 4;
+            const Kind kd = g.spec.kind;
+            if (kd != Kind::Identity)
+                bytes += std::ldexp(kd == Kind::PhaseOne || kd == Kind::PairSub ? 0.5 : 1.0, -nc);
+        }
+        if (!lowered)
+        {
+            for (const auto &g : gates)
+                apply_resolved(g);
+            return;
+        }
+        const std::vector<PassGate> low = lowering.finish();
+        if (low.empty())
+            return;
+        const PassPlan P = plan_passes(low, n_, m, 16);
+        // A pass moves the whole state once, so few gates with many controls are cheaper one by
+        // one; on states of up to 2^22 amplitudes the launches count, not the bytes.
+        if (n_ > 22 && bytes < double(P.passes.size()))
+        {
+            for (const auto &g : gates)
+                apply_resolved(g);
+            return;
+        }
+        const size_t rb = P.rounds.size() * sizeof(qsv::PassRound), ob = P.ops.size() * sizeof(qsv::PassOp);
+        static_assert(sizeof(qsv::PassRound) % 16 == 0 && sizeof(qsv::PassOp) % 16 == 0, "pass program alignment");
+        reserve_program(rb + ob);
+        const bool small = rb + ob <= kSmallProgram;
+        char *host = small ? reinterpret_cast<char *>(pinned_ + kPinnedResults) : static_cast<char *>(prog_host_);
+        char *dev = small ? reinterpret_cast<char *>(work_ + work_len_) : static_cast<char *>(prog_dev_);
+        std::memcpy(host, P.rounds.data(), rb);
+        std::memcpy(host + rb, P.ops.data(), ob);
+        qsv::check(hipMemcpyAsync(dev, host, rb + ob, hipMemcpyHostToDevice, stream_), "pass program upload");
+        qsv::check(hipEventRecord(prog_copied_, stream_), "hipEventRecord");
+        prog_pending_ = true;
+        const auto *rounds = reinterpret_cast<const qsv::PassRound *>(dev);
+        const auto *ops = reinterpret_cast<const qsv::PassOp *>(dev + rb);
+        for (const auto &ps : P.passes)
+        {
+            prof_begin(QCS_EXT_K_FUSED, 32.0 * (1ull << n_));
+            qsv::launch_pass(stream_, state_, n_, P.m, ps.tq, rounds + ps.first_round, int(ps.nrounds), ops);
+            prof_end();
+        }
     }
 
     void Simulator::apply_resolved(const ResolvedGate &r)

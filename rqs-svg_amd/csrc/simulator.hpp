@@ -22,6 +22,13 @@ namespace qcore
         unsigned mmask = 0, mval = 0;         // measured targets (bit j = target j) and values
     };
 
+    // One gate of a circuit given as a whole (run_circuit), logical qubits.
+    struct CircuitGate
+    {
+        GateSpec spec;
+        std::vector<int> targets, neg, pos;
+    };
+
     class Simulator
     {
     public:
@@ -50,6 +57,11 @@ namespace qcore
         void clear_measurement_state();
 
         void operate(const GateSpec &g, std::vector<int> targets, std::vector<int> neg, std::vector<int> pos);
+        // The gates in order, as operate() on each would leave the state.  A complex128 per-gate
+        // state with no measured qubits takes runs of gates as passes (pass.hpp) where that
+        // moves fewer bytes; every launch is queued before this returns.  Throws at the first
+        // gate that operate() would refuse, with the ones before it applied; *applied: how many.
+        void run_circuit(const std::vector<CircuitGate> &gates, size_t *applied);
         int measure(int q);
 
         void save_statevector(const char *path);
@@ -103,6 +115,10 @@ namespace qcore
         void move_physical(const std::vector<int> &dst);
         void remap_physical(const std::vector<int> &dst);
         void apply_resolved(const ResolvedGate &r);
+        // operands and mapping of a gate on a state without measured qubits
+        ResolvedGate resolve(const GateSpec &g, const std::vector<int> &targets, const std::vector<int> &neg, const std::vector<int> &pos) const;
+        void apply_run(const std::vector<ResolvedGate> &gates);
+        void reserve_program(size_t bytes);
         void ensure_levels();
         uint64_t logical_chunk() const;
         void ensure_stage();
@@ -144,7 +160,13 @@ namespace qcore
         bool levels_valid_ = false;
         double levels_total_ = 0.0;
         void state_changed() { levels_valid_ = false; }
-        double *pinned_ = nullptr; // 64 doubles of pinned host memory
+        double *pinned_ = nullptr; // pinned host memory: 64 doubles of results, then the staging area of small pass programs
+        static constexpr size_t kPinnedResults = 64, kSmallProgram = 64 << 10;
+        // pass programs (rounds and operations): small ones use the end of pinned_ and of work_
+        void *prog_host_ = nullptr, *prog_dev_ = nullptr;
+        size_t prog_cap_ = 0; // bytes of the two above
+        hipEvent_t prog_copied_ = nullptr;
+        bool prog_pending_ = false;
         qsv::c128 *stage_dev_ = nullptr;
         void *stage_host_ = nullptr;
         uint64_t stage_len_ = 0;

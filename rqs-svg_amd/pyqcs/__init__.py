@@ -14,7 +14,9 @@ callback.
 """
 from __future__ import annotations
 
+import array
 import ctypes
+import itertools
 import time
 import os
 import pathlib
@@ -120,6 +122,7 @@ class Library:
         lib.qcs_ext_sample_noalloc.argtypes = [vp, u64, u64, vp]
         lib.qcs_ext_probability_total.argtypes = [vp, P(ctypes.c_double)]
         lib.qcs_ext_norm.argtypes = [vp, P(ctypes.c_double)]
+        lib.qcs_ext_run_circuit.argtypes = [vp, ctypes.c_int32, P(ctypes.c_char_p), P(ctypes.c_int32)] + [vp] * 8 + [P(ctypes.c_int32)]
         lib.qcs_ext_expect_z.argtypes = [vp, vp, ctypes.c_int]
         lib.qcs_ext_set_renormalize.argtypes = [vp, ctypes.c_int]
         lib.qcs_ext_set_local_qubits.argtypes = [vp, bit_num_t]
@@ -182,6 +185,33 @@ def _arr(values):
     if not values:
         return None, 0
     return (bit_num_t * len(values))(*values), len(values)
+
+
+def _pack_circuit(circuit):
+    """The arrays of qcs_ext_run_circuit for a list of full (name, targets, params, ctrls,
+    negctrls) tuples; None for anything that the gate calls have to see one by one (short
+    tuples, unknown names, wrong parameter counts, values that are not plain integers)."""
+    try:
+        if set(map(len, circuit)) != {5}:
+            return None
+        names, targets, params, ctrls, negctrls = zip(*circuit)
+        index = {nm: i for i, nm in enumerate(dict.fromkeys(names))}
+        need = {nm: 1 if nm == "global_phase" else GATE_PARAMS[nm] for nm in index}
+        if list(map(len, params)) != list(map(need.__getitem__, names)):
+            return None
+        if "global_phase" in index and any(t for nm, t in zip(names, targets) if nm == "global_phase"):
+            return None
+        values = array.array("d", list(itertools.chain.from_iterable(params)))
+        values.append(0.0)  # never empty
+        counts = [bytes(map(len, qs)) for qs in (targets, negctrls, ctrls)]
+        lists = [array.array("h", list(itertools.chain.from_iterable(qs))) for qs in (targets, negctrls, ctrls)]
+        name_of = bytes(map(index.__getitem__, names))
+    except (TypeError, ValueError, KeyError, OverflowError, AttributeError):
+        return None
+    cnames = (ctypes.c_char_p * len(index))(*[nm.encode() for nm in index])
+    cneed = (ctypes.c_int32 * len(index))(*need.values())
+    addr = [a.buffer_info()[0] for a in (*lists, values)]
+    return (lists, values), (cnames, cneed, name_of, *counts, *addr)
 
 
 class Simulator:
@@ -247,8 +277,16 @@ class Simulator:
 
     def run(self, circuit):
         """Apply a list of (name, targets, params, ctrls, negctrls) tuples."""
-        for op in circuit:
-            self.gate(*op)
+        packed = _pack_circuit(circuit) if type(circuit) in (list, tuple) and len(circuit) > 1 else None
+        if packed is None:
+            for op in circuit:
+                self.gate(*op)
+            return
+        keep, arrays = packed  # keep: the buffers that arrays points into
+        applied = ctypes.c_int32()
+        rc = self.lib.qcs_ext_run_circuit(self.h, len(circuit), *arrays, ctypes.byref(applied))
+        if rc != 1:
+            self._call(rc, "gate_" + circuit[min(applied.value, len(circuit) - 1)][0])
 
     # --- measurement / state ----------------------------------------------------------
     def measure(self, q):

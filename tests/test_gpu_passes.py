@@ -1,0 +1,83 @@
+"""Circuit passes on the GPU: Simulator.run on a complex128 state against the same gates called
+one by one (the per-gate kernels) and, at small sizes, against the oracle.  Both sides round
+in FP64 at every gate: amplitudes of modulus <= 1 after g gates differ by at most a few
+roundings each, so the bound is 16 g 2^-53 times the largest amplitude."""
+import numpy as np
+import pytest
+
+import pyqcs
+from pyqcs import circuits
+from conftest import random_state
+
+pytestmark = pytest.mark.gpu
+
+
+def both(gpu, n, circ, mapping=None):
+    psi = random_state(n, n)
+    out = []
+    for whole in (True, False):
+        with pyqcs.Simulator(gpu, n, mapping=mapping, seed=3) as sim:
+            sim.set_statevector(psi)
+            if whole:
+                sim.run(circ)
+            else:
+                for op in circ:
+                    sim.gate(*op)
+            out.append(sim.statevector())
+    return out
+
+
+def bound(circ, psi):
+    return 16 * len(circ) * 2.0 ** -53 * np.max(np.abs(psi))
+
+
+# one-tile states around the smallest tile, the single-workgroup sizes, and the sizes where the
+# tile grows; 24 and 25 qubits lie on both sides of the cached / non-temporal access switch
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 9, 10, 11, 12, 13, 14, 16, 17, 18, 19, 21])
+def test_passes_match_gates(gpu, n):
+    for seed in range(3 if n < 18 else 1):
+        circ = circuits.random_all_gates(n, 120, seed=100 * n + seed, max_ctrls=min(4, n - 1)) if n > 1 else \
+            [("h", (0,), (), (), ()), ("rz", (0,), (0.3,), (), ()), ("u3", (0,), (0.2, 0.7, 1.1), (), ()), ("y", (0,), (), (), ())]
+        mapping = [int(q) for q in np.random.default_rng(seed).permutation(n)] if seed == 1 else None
+        print("n", n, "seed", seed, flush=True)
+        a, b = both(gpu, n, circ, mapping)
+        assert np.max(np.abs(a - b)) <= bound(circ, b)
+
+
+@pytest.mark.parametrize("n,family", [(24, "brick"), (25, "brick"), (20, "qft"), (20, "variational"), (19, "qaoa")])
+def test_passes_match_gates_families(gpu, n, family):
+    circ = {"brick": lambda: circuits.brick(n, 3, seed=5, mcx=3), "qft": lambda: circuits.qft(n),
+            "variational": lambda: circuits.variational(n, 3, seed=6), "qaoa": lambda: circuits.qaoa_ring(n, 2, seed=7)}[family]()
+    a, b = both(gpu, n, circ)
+    assert np.max(np.abs(a - b)) <= bound(circ, b)
+
+
+def test_run_refuses_like_the_gates(gpu, oracle):
+    # a refused gate in the middle: the ones before it are applied, the message is the gate's
+    n = 7
+    good = circuits.random_all_gates(n, 20, seed=8)
+    for bad, text in ((("x", (9,), (), (), ()), "gate_x"), (("swap", (1, 1), (), (), ()), "more than once"), (("h", (1, 2), (), (), ()), "target")):
+        states = []
+        for lib in (gpu, oracle):
+            with pyqcs.Simulator(lib, n, seed=1) as sim:
+                with pytest.raises(pyqcs.QcsError, match=text):
+                    sim.run(good + [bad] + good)
+                states.append(sim.statevector())
+        assert np.max(np.abs(states[0] - states[1])) <= 1e-13
+
+
+def test_run_with_measured_qubits_and_profile(gpu, oracle):
+    # measured qubits are implicit controls: such circuits go gate by gate
+    n = 8
+    c1, c2 = circuits.random_all_gates(n, 40, seed=11), circuits.random_all_gates(n, 40, seed=12)
+    res = []
+    for lib in (gpu, oracle):
+        with pyqcs.Simulator(lib, n, seed=4) as sim:
+            sim.run(c1)
+            bits = [sim.measure(2), sim.measure(5)]
+            sim.run(c2)
+            sim.call("reset_measurement_state")
+            sim.run(c1)
+            res.append((bits, sim.statevector()))
+    assert res[0][0] == res[1][0]
+    assert np.max(np.abs(res[0][1] - res[1][1])) <= 1e-13
