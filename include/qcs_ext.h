@@ -130,7 +130,10 @@ int qcs_ext_permute(qcs_simulator *sim, const bit_num_t *new_perm_p2l, bit_num_t
  * renormalisation.  mode 2: complex128 state, gates fused into blocks of at most 4 qubits
  * applied in FP64.  mode 3: as mode 1 with the block products on BF16x3 split-precision
  * MFMA (matrix and state each split into two bfloat16 parts, three bf16 products summed in
- * FP32).  Must be called before allocate_memory. */
+ * FP32).  Until qcs_ext_set_stage_bits, qcs_ext_set_plan or qcs_ext_set_planner asks for
+ * blocks or stages, modes 1 and 2 run their gates as circuit passes instead (as
+ * qcs_ext_run_circuit does; FP64 arithmetic on either state, rounded to the state's type once
+ * per sweep).  Must be called before allocate_memory. */
 int qcs_ext_set_precision(qcs_simulator *sim, int mode, int max_block_qubits);
 
 /* Fused precision modes: blocks of a flush are grouped into stages, each applied to

@@ -192,6 +192,12 @@ namespace qcore
         // LDS tile bits of the stage kernel (11, 12 or 13), or 0 for one launch per block.
         void set_stage_bits(int m);
         void set_stage_stream(bool on);
+        // Whether flushes without a model or a fixed plan run as circuit passes (modes 1 and 2).
+        void set_passes(bool on)
+        {
+            flush();
+            passes_ = on && !x3_;
+        }
         int stage_bits() const { return stage_bits_; }
         // tile bits of the default stage plan for this state (complex128: 2^12), 0 if
         // per-block launches are used; stages need at least 16 tiles
@@ -277,6 +283,7 @@ namespace qcore
         int kq_; // kernel block size (4 or 5)
         int stage_bits_ = 13;
         bool stage_stream_ = true;
+        bool passes_ = false;
         bool f64_ = false;
         bool x3_ = false;
         qsv::c64 *state_ = nullptr;

@@ -135,8 +135,12 @@ namespace qcore
         if (m != 0 && (m < 11 || m > 14))
             throw std::runtime_error("stage tile bits must be 0 (one sweep per block), 11, 12, 13 or 14");
         stage_bits_ = m;
+        stages_asked_ = true;
         if (fused_)
+        {
             fused_->set_stage_bits(m);
+            fused_->set_passes(false);
+        }
     }
 
     void Simulator::set_stage_stream(int on)
@@ -205,6 +209,7 @@ namespace qcore
         {
             fused_ = new FusedEngine(*this, block_qubits_, precision_);
             fused_->set_stage_bits(stage_bits_);
+            fused_->set_passes(!stages_asked_);
             fused_->set_stage_stream(stage_stream_ != 0);
             fused_->set_check(planner_check_ != 0);
         }
@@ -570,43 +575,30 @@ namespace qcore
         prog_cap_ = cap;
     }
 
-    void Simulator::apply_run(const std::vector<ResolvedGate> &gates)
+    int Simulator::run_passes(const std::vector<ResolvedGate> &gates)
     {
-        if (gates.empty())
-            return;
-        state_changed();
         const int m = pass_tile_bits(n_);
+        const int amp_bytes = fused_ && !fused_->f64() ? 8 : 16;
         PassLowering lowering(n_);
         double bytes = 0; // what one kernel per gate would move, in sweeps of the state
-        bool lowered = gates.size() > 1;
-        for (size_t i = 0; lowered && i < gates.size(); ++i)
+        for (const ResolvedGate &g : gates)
         {
-            const ResolvedGate &g = gates[i];
             const int nc = int(g.pphys.size() + g.nphys.size());
             // a controlled 2x2 needs 4 register bits clear of its controls
-            lowered = lowering.add(g) && nc + int(g.tphys.size()) <= m - 4;
+            if (nc + int(g.tphys.size()) > m - 4 || !lowering.add(g))
+                return -1;
             const Kind kd = g.spec.kind;
             if (kd != Kind::Identity)
                 bytes += std::ldexp(kd == Kind::PhaseOne || kd == Kind::PairSub ? 0.5 : 1.0, -nc);
         }
-        if (!lowered)
-        {
-            for (const auto &g : gates)
-                apply_resolved(g);
-            return;
-        }
         const std::vector<PassGate> low = lowering.finish();
         if (low.empty())
-            return;
-        const PassPlan P = plan_passes(low, n_, m, 16);
+            return 0;
+        const PassPlan P = plan_passes(low, n_, m, amp_bytes);
         // A pass moves the whole state once, so few gates with many controls are cheaper one by
         // one; on states of up to 2^22 amplitudes the launches count, not the bytes.
         if (n_ > 22 && bytes < double(P.passes.size()))
-        {
-            for (const auto &g : gates)
-                apply_resolved(g);
-            return;
-        }
+            return -1;
         const size_t rb = P.rounds.size() * sizeof(qsv::PassRound), ob = P.ops.size() * sizeof(qsv::PassOp);
         static_assert(sizeof(qsv::PassRound) % 16 == 0 && sizeof(qsv::PassOp) % 16 == 0, "pass program alignment");
         reserve_program(rb + ob);
@@ -622,10 +614,22 @@ namespace qcore
         const auto *ops = reinterpret_cast<const qsv::PassOp *>(dev + rb);
         for (const auto &ps : P.passes)
         {
-            prof_begin(QCS_EXT_K_FUSED, 32.0 * (1ull << n_));
-            qsv::launch_pass(stream_, state_, n_, P.m, ps.tq, rounds + ps.first_round, int(ps.nrounds), ops);
+            prof_begin(QCS_EXT_K_FUSED, 2.0 * amp_bytes * (1ull << n_));
+            with_state([&](auto *st) { qsv::launch_pass(stream_, st, n_, P.m, ps.tq, rounds + ps.first_round, int(ps.nrounds), ops); });
             prof_end();
         }
+        return int(P.passes.size());
+    }
+
+    void Simulator::apply_run(const std::vector<ResolvedGate> &gates)
+    {
+        if (gates.empty())
+            return;
+        state_changed();
+        if (gates.size() > 1 && run_passes(gates) >= 0)
+            return;
+        for (const auto &g : gates)
+            apply_resolved(g);
     }
 
     void Simulator::apply_resolved(const ResolvedGate &r)

@@ -118,6 +118,9 @@ namespace qcore
         // operands and mapping of a gate on a state without measured qubits
         ResolvedGate resolve(const GateSpec &g, const std::vector<int> &targets, const std::vector<int> &neg, const std::vector<int> &pos) const;
         void apply_run(const std::vector<ResolvedGate> &gates);
+        // Applies gates as circuit passes and returns how many, or returns -1 with nothing
+        // done where they have no such form or would not pay for their sweeps.
+        int run_passes(const std::vector<ResolvedGate> &gates);
         void reserve_program(size_t bytes);
         void ensure_levels();
         uint64_t logical_chunk() const;
@@ -142,6 +145,7 @@ namespace qcore
         int n_local_ = 0;
         int precision_ = 0;
         int stage_bits_ = 13;
+        bool stages_asked_ = false; // set_stage_bits was called
         int stage_stream_ = 1;
         int planner_check_ = 1;
         bool c64_state() const { return precision_ == 1 || precision_ == 3; }

@@ -81,3 +81,47 @@ def test_run_with_measured_qubits_and_profile(gpu, oracle):
             res.append((bits, sim.statevector()))
     assert res[0][0] == res[1][0]
     assert np.max(np.abs(res[0][1] - res[1][1])) <= 1e-13
+
+
+# The fused modes' default flushes: FP64 arithmetic, and for complex64 one rounding to FP32 of
+# every amplitude per sweep (2^-24 of its modulus) and two more when the state is rescaled, which
+# a unitary carries along unchanged: ||d|| <= (sweeps + 3) 2^-24 on a state of norm 1.
+@pytest.mark.parametrize("precision", [1, 2])
+@pytest.mark.parametrize("n", [4, 5, 9, 10, 12, 13, 18, 19, 22, 24])
+def test_fused_modes_run_as_passes(gpu, n, precision):
+    circ = circuits.random_all_gates(n, 150, seed=n, max_ctrls=3 if n > 5 else 1) if n < 22 else circuits.brick(n, 3, seed=n, mcx=3)
+    psi = random_state(n, n)
+    with pyqcs.Simulator(gpu, n) as plain, pyqcs.Simulator(gpu, n, precision=precision) as fused:
+        for sim in (plain, fused):
+            sim.set_statevector(psi)
+        for op in circ:
+            plain.gate(*op)
+        fused.run(circ)
+        gates, sweeps = fused.fusion_stats()  # flushes
+        d = np.linalg.norm(plain.statevector() - fused.statevector())
+    print("n", n, "precision", precision, "sweeps", sweeps, "||d||", d, flush=True)
+    assert gates == len(circ) and sweeps < len(circ)
+    assert d <= (sweeps + 3) * 2.0 ** -24 if precision == 1 else d <= 16 * len(circ) * 2.0 ** -53
+
+
+@pytest.mark.parametrize("precision,m", [(1, 13), (2, 12)])
+def test_fused_modes_asked_for_stages(gpu, precision, m):
+    # a stage size or a fixed plan turns passes off, also after a flush that ran as passes: the
+    # stages' sweep count is that of a simulator that never ran a pass
+    n = 17
+    circ = circuits.brick(n, 6, seed=4, mcx=2)
+    counts, states = [], []
+    for before, plan in ((False, False), (True, False), (True, True)):
+        with pyqcs.Simulator(gpu, n, precision=precision, stage_bits=None if before else 13) as sim:
+            if before:
+                sim.run(circ)
+                sim.call("set_zero_state")
+                sim.fusion_stats()
+                sim.set_plan(m, 3 if precision == 2 else 5, tiles=2) if plan else sim.set_stage_bits(13)
+            g0, s0 = sim.fusion_stats()
+            sim.run(circ)
+            g1, s1 = sim.fusion_stats()
+            counts.append((g1 - g0, s1 - s0))
+            states.append(sim.statevector())
+    assert counts[0] == counts[1] == counts[2] and counts[0][0] == len(circ)
+    assert np.array_equal(states[0], states[1]) and np.array_equal(states[0], states[2])
