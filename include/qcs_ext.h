@@ -175,9 +175,10 @@ int qcs_ext_overlap(qcs_simulator *a, qcs_simulator *b, double *out);
 
 /* Batching form: many independent circuits of 1-target gates (each with at most one
  * positive control), every circuit starting from |0...0>, outputs <Z_q> for all qubits of
- * every circuit (FP64 reductions).  libqcs.so runs the whole batch as one hipGraph launch:
- * circuits of up to lds_max_qubits qubits in a persistent LDS-resident kernel, larger ones
- * as fused blocks on complex64 states in HBM.  The oracle runs the plain method per circuit. */
+ * every circuit (FP64 reductions).  libqcs.so runs the whole batch as one hipGraph launch, by
+ * default as circuit passes (FP64 arithmetic; states of more than 12 qubits are kept as
+ * complex64); with a tuning set, circuits of up to lds_max_qubits qubits in a persistent
+ * LDS-resident kernel and larger ones as fused blocks on complex64 states in HBM.  The oracle runs the plain method per circuit. */
 typedef struct qcs_ext_batch qcs_ext_batch;
 int qcs_ext_batch_create(qcs_ext_batch **out);
 int qcs_ext_batch_destroy(qcs_ext_batch *batch);
@@ -192,9 +193,12 @@ int qcs_ext_batch_add_circuit(qcs_ext_batch *batch, bit_num_t num_qubits, int32_
 int qcs_ext_batch_set_tuning(qcs_ext_batch *batch, int lds_max_qubits, int block_size, int block_qubits, int streams, int stage_bits);
 /* Block products of the circuits in HBM: mode 1 = FP32 MFMA (the default), 3 = BF16x3
  * split-precision MFMA (the modes of qcs_ext_set_precision; states complex64 and <Z> FP64
- * either way).  The oracle computes in FP64 and only checks the mode. */
+ * either way).  With no tuning set mode 1 runs no products (see above) and mode 3 runs them
+ * for circuits of more than 14 qubits.  The oracle computes in FP64 and only checks the mode. */
 int qcs_ext_batch_set_precision(qcs_ext_batch *batch, int mode);
-/* Searches the tuning parameters on this batch; writes the chosen 5 values to tuning. */
+/* Searches the tuning parameters on this batch; writes the chosen 5 values to tuning.  Where no
+ * tuning was set and none beats the circuit passes, the batch stays as it was (and the values
+ * written are the ones it had: setting them would select the kernels above). */
 int qcs_ext_batch_autotune(qcs_ext_batch *batch, int *tuning);
 /* expz receives sum(num_qubits) doubles, circuit by circuit; seconds = device time. */
 int qcs_ext_batch_run(qcs_ext_batch *batch, double *expz, uint64_t count, double *seconds);
@@ -202,7 +206,8 @@ int qcs_ext_batch_info(qcs_ext_batch *batch, int *num_circuits, int *total_qubit
 /* Algorithmic HBM bytes of one run and its kernel launches (libqcs.so; prepares the batch):
  * every fused-block or stage sweep of a complex64 state in HBM reads and writes it (16 B
  * per amplitude) except a circuit's first stage round, which writes it from |0...0>
- * without reading (8 B), every basis-state fill writes it (8 B), every <Z> reduction reads
+ * without reading (8 B), every circuit pass but the first reads and every one but the last
+ * writes it (8 B each), every basis-state fill writes it (8 B), every <Z> reduction reads
  * it (8 B); circuits in the LDS-resident kernel move nothing through HBM.  The oracle writes 0
  * for both. */
 int qcs_ext_batch_traffic(qcs_ext_batch *batch, double *hbm_bytes, uint64_t *kernel_launches);

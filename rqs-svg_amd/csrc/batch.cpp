@@ -1,24 +1,34 @@
 // Batching form host side: partition, plan, capture into one hipGraph, autotune.
 //
-// Circuits of up to `lds_max_qubits` qubits go to the persistent LDS-resident kernel (one
-// workgroup per circuit, work-counter driven); larger ones keep a complex64 state in HBM.
-// Those of at least stage_bits + 4 qubits run as stages on LDS tiles, batched across
-// circuits: one launch per stage round covers the r-th stage of every such circuit.  The
-// rest run as fused k-qubit blocks, one launch each, spread over several streams.
+// By default circuits run as circuit passes (pass_kernels.hpp): one of up to 12 qubits as one
+// tile in the registers of one workgroup, from |0...0> to its sums for <Z>; a larger one as
+// passes over a complex64 state, batched across circuits: one launch per pass round covers the
+// r-th pass of every such circuit.  BF16x3 products are asked for by set_precision(3): circuits
+// of more than lds_max_qubits qubits then run as stages (below).
+// With a tuning set, circuits of up to `lds_max_qubits` qubits go to the persistent
+// LDS-resident kernel (one workgroup per circuit, work-counter driven); larger ones keep a
+// complex64 state in HBM.  Those of at least stage_bits + 4 qubits run as stages on LDS tiles,
+// batched across circuits in the same way.  The rest run as fused k-qubit blocks, one launch
+// each, spread over several streams.
 // Everything -- counter reset, the persistent kernel, the stage rounds, the fills and
 // block sequences of the smaller HBM circuits, the <Z> reductions -- is captured once into
 // a hipGraph and replayed with a single launch.
 #include "batch.hpp"
+#include "pass.hpp"
 #include "simulator.hpp"
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstring>
 #include <functional>
 #include <map>
 #include <memory>
+#include <mutex>
 #include <stdexcept>
+#include <system_error>
+#include <thread>
 
 namespace qcore
 {
@@ -34,6 +44,42 @@ namespace qcore
             auto u = dense_matrix(s);
             for (int i = 0; i < 4; ++i)
                 m[i] = u[i];
+        }
+
+        // f(0) .. f(count - 1), each once, on up to 16 threads of at least 8 calls each
+        template <class F>
+        void for_each_circuit(size_t count, F f)
+        {
+            std::exception_ptr err;
+            std::mutex err_mu;
+            std::atomic<size_t> next{0};
+            auto work = [&] {
+                try
+                {
+                    for (size_t i = next++; i < count; i = next++)
+                        f(i);
+                }
+                catch (...)
+                {
+                    std::lock_guard<std::mutex> lock(err_mu);
+                    err = std::current_exception();
+                }
+            };
+            const size_t threads = std::min<size_t>({size_t(16), std::max(1u, std::thread::hardware_concurrency()), count / 8});
+            std::vector<std::thread> pool;
+            try
+            {
+                for (size_t t = 1; t < threads; ++t)
+                    pool.emplace_back(work);
+            }
+            catch (const std::system_error &)
+            { // fewer threads, then
+            }
+            work();
+            for (auto &th : pool)
+                th.join();
+            if (err)
+                std::rethrow_exception(err);
         }
 
         qsv::BatchOp to_op(int target, int control, const cd m[4])
@@ -81,7 +127,7 @@ namespace qcore
         exec_ = nullptr;
         graph_ = nullptr;
         work_ = nullptr;
-        for (void *p : {(void *)d_circs_, (void *)d_ops_, (void *)d_out_, (void *)d_counter_, (void *)d_states_, (void *)d_partials_, (void *)d_mats_})
+        for (void *p : {(void *)d_circs_, (void *)d_ops_, (void *)d_out_, (void *)d_counter_, (void *)d_states_, (void *)d_partials_, (void *)d_mats_, (void *)d_sums_, d_prog_})
             if (p)
                 (void)hipFree(p);
         d_circs_ = nullptr;
@@ -91,6 +137,8 @@ namespace qcore
         d_states_ = nullptr;
         d_partials_ = nullptr;
         d_mats_ = nullptr;
+        d_sums_ = nullptr;
+        d_prog_ = nullptr;
         for (auto e : fork_join_)
             (void)hipEventDestroy(e);
         fork_join_.clear();
@@ -131,6 +179,7 @@ namespace qcore
             throw std::runtime_error("batch: stage bits must be 0, 11, 12 or 13");
         release();
         tuning_ = t;
+        passes_ = false;
     }
 
     void Batch::set_precision(int mode)
@@ -153,9 +202,42 @@ namespace qcore
         std::vector<qsv::BatchOp> ops;
         int small_max_n = 1;
         std::vector<int> large;
+        struct Passed
+        {
+            int ci;
+            PassPlan plan;
+        };
+        std::vector<Passed> passed;
+        // The circuits' pass plans, on up to 16 host threads: 50 us a circuit, 256 circuits would
+        // wait 13 ms for their first run (no passes: a circuit without such a plan).
+        std::vector<PassPlan> plans(circuits_.size());
+        if (passes_)
+            for_each_circuit(circuits_.size(), [&](size_t ci) {
+                const Circuit &C = circuits_[ci];
+                if (x3_ && C.n > T.lds_max_qubits)
+                    return;
+                PassLowering lowering(C.n);
+                ResolvedGate r;
+                for (const auto &g : C.gates)
+                {
+                    r.spec = make_gate(g.name, g.params);
+                    r.tphys.assign(1, g.target);
+                    r.pphys.assign(g.control >= 0 ? 1 : 0, g.control);
+                    if (!lowering.add(r))
+                        return;
+                }
+                const auto low = lowering.finish();
+                if (!low.empty())
+                    plans[ci] = plan_passes(low, C.n, std::clamp(C.n, qsv::kPassMinBits, qsv::kPassMaxBits), 8);
+            });
         for (int ci = 0; ci < (int)circuits_.size(); ++ci)
         {
             const Circuit &C = circuits_[ci];
+            if (!plans[ci].passes.empty())
+            {
+                passed.push_back(Passed{ci, std::move(plans[ci])});
+                continue;
+            }
             if (C.n > T.lds_max_qubits)
             {
                 large.push_back(ci);
@@ -237,7 +319,10 @@ namespace qcore
             const int kq = (C.n >= 5 && T.block_qubits == 5) ? 5 : 4;
             if (C.n < kq)
                 throw std::runtime_error("batch: circuit too small for the HBM path");
-            if (T.stage_bits > 0 && C.n >= T.stage_bits + 4 && !rg.empty())
+            // A tuned batch launches the blocks of states of less than 16 tiles one by one; in
+            // rounds with others they fill the chip as well (256 circuits of 6-16 qubits, the
+            // 15-qubit ones in BF16x3: 5033 launches before, 26 now).
+            if (T.stage_bits > 0 && C.n >= T.stage_bits + (passes_ ? 1 : 4) && !rg.empty())
             {
                 const auto plan = plan_stages(rg, C.n, T.stage_bits, kq);
                 // batched gates span at most 2 qubits, so every stage has a tile
@@ -272,6 +357,36 @@ namespace qcore
             place(sc.ci);
         for (const auto &bc : blocked)
             place(bc.ci);
+        // ---- circuit passes: one program for all circuits, tasks per launch ----
+        // Biggest circuits first: they have most passes, and most tiles to spread.
+        std::stable_sort(passed.begin(), passed.end(), [&](const Passed &a, const Passed &b) {
+            const int na = circuits_[a.ci].n, nb = circuits_[b.ci].n;
+            return na != nb ? na > nb : a.plan.work > b.plan.work;
+        });
+        std::vector<qsv::PassRound> prounds;
+        std::vector<qsv::PassOp> pops;
+        std::vector<qsv::PassZ> pz;
+        struct PassLaunch
+        {
+            int m;
+            uint32_t tiles = 0;
+            std::vector<qsv::PassTask> tasks;
+            size_t offset = 0; // of the tasks in the program
+        };
+        // launches 0 .. 2: whole circuits on tiles of 2^10 .. 2^12; from 3 on: the rounds
+        std::vector<PassLaunch> plaunch{{10}, {11}, {12}};
+        uint64_t sums_total = 0;
+        std::vector<uint64_t> pass_state; // per passed circuit
+        std::vector<size_t> pass_sums;
+        for (const auto &pc : passed)
+        {
+            pass_state.push_back(state_total);
+            pass_sums.push_back(sums_total);
+            const int n = circuits_[pc.ci].n, m = pc.plan.m;
+            if (n > m)
+                state_total += uint64_t(1) << n;
+            sums_total += (n > m ? uint64_t(1) << (n - m) : 1) * qsv::kPassSums;
+        }
         // ---- device buffers (addresses go into the task arrays below) ----
         auto upload = [](void **dst, const void *src, size_t bytes) {
             if (bytes == 0)
@@ -287,6 +402,88 @@ namespace qcore
             qsv::check(hipMalloc((void **)&d_states_, state_total * sizeof(qsv::c64)), "hipMalloc batch states");
         if (partial_total)
             qsv::check(hipMalloc((void **)&d_partials_, partial_total * sizeof(double)), "hipMalloc batch");
+        if (sums_total)
+            qsv::check(hipMalloc((void **)&d_sums_, sums_total * sizeof(double)), "hipMalloc batch");
+        size_t nrounds_total = 0, nops_total = 0;
+        for (const auto &pc : passed)
+        {
+            nrounds_total += pc.plan.rounds.size();
+            nops_total += pc.plan.ops.size();
+        }
+        prounds.reserve(nrounds_total);
+        pops.reserve(nops_total);
+        for (size_t i = 0; i < passed.size(); ++i)
+        {
+            const Circuit &C = circuits_[passed[i].ci];
+            const PassPlan &P = passed[i].plan;
+            const int n = C.n, m = P.m;
+            const uint32_t tiles = n > m ? uint32_t(1) << (n - m) : 1;
+            const uint32_t first_op = uint32_t(pops.size()), first_round = uint32_t(prounds.size());
+            pops.insert(pops.end(), P.ops.begin(), P.ops.end());
+            for (auto r : P.rounds)
+            {
+                r.first += first_op;
+                prounds.push_back(r);
+            }
+            for (size_t p = 0; p < P.passes.size(); ++p)
+            {
+                const auto &ps = P.passes[p];
+                const size_t li = n > m ? 3 + p : size_t(m - qsv::kPassMinBits);
+                if (li == plaunch.size())
+                    plaunch.push_back(PassLaunch{qsv::kPassMaxBits});
+                PassLaunch &L = plaunch[li];
+                qsv::PassTask t{};
+                t.state = n > m ? d_states_ + pass_state[i] : nullptr;
+                t.sums = d_sums_ + pass_sums[i];
+                t.tile_begin = L.tiles;
+                t.first_round = first_round + ps.first_round;
+                t.nrounds = ps.nrounds;
+                for (int b = 0; b < m; ++b)
+                    t.tq[b / 4] |= uint32_t(ps.tq[b]) << (8 * (b % 4));
+                auto bit_of = [&](uint32_t q) { return uint8_t(std::find(ps.tq, ps.tq + m, q) - ps.tq); };
+                const qsv::PassRound &R = P.rounds[ps.first_round + ps.nrounds - 1];
+                for (int j = 0; j < m; ++j)
+                    t.zb[j] = bit_of(j < 4 ? R.rq[j] : R.tq[j - 4]);
+                if (p == 0)
+                    t.flags |= qsv::kPassZeroState;
+                if (p + 1 == P.passes.size())
+                {
+                    t.flags |= qsv::kPassExpectZ;
+                    uint32_t outside = 0; // qubits below q that are not tile qubits
+                    for (int q = 0; q < n; ++q)
+                    {
+                        const int b = bit_of(q);
+                        qsv::PassZ z{};
+                        z.sums = t.sums;
+                        z.out = d_out_ + C.out_offset + q;
+                        z.ntiles = tiles;
+                        z.slot = b < m ? 1 + b : 0;
+                        z.sign = b < m ? 0 : uint32_t(1) << outside++;
+                        pz.push_back(z);
+                    }
+                }
+                L.tiles += tiles;
+                L.tasks.push_back(t);
+            }
+        }
+        // rounds, operations, tasks of each launch, <Z> entries (all multiples of 16 bytes)
+        std::vector<char> prog;
+        auto put = [&](const void *src, size_t bytes) {
+            const size_t off = prog.size();
+            prog.insert(prog.end(), static_cast<const char *>(src), static_cast<const char *>(src) + bytes);
+            return off;
+        };
+        static_assert(sizeof(qsv::PassRound) % 16 == 0 && sizeof(qsv::PassOp) % 16 == 0 && sizeof(qsv::PassTask) % 16 == 0 && sizeof(qsv::PassZ) % 16 == 0, "pass program alignment");
+        prog.reserve(prounds.size() * sizeof(qsv::PassRound) + pops.size() * sizeof(qsv::PassOp) + pz.size() * sizeof(qsv::PassZ) + (2 * passed.size() + plaunch.size()) * sizeof(qsv::PassTask));
+        put(prounds.data(), prounds.size() * sizeof(qsv::PassRound));
+        const size_t pops_off = put(pops.data(), pops.size() * sizeof(qsv::PassOp));
+        for (auto &L : plaunch)
+            L.offset = put(L.tasks.data(), L.tasks.size() * sizeof(qsv::PassTask));
+        const size_t pz_off = put(pz.data(), pz.size() * sizeof(qsv::PassZ));
+        const uint32_t pz_count = uint32_t(pz.size());
+        upload(&d_prog_, prog.data(), prog.size());
+        // states within the 256 MB memory-side cache keep cached accesses
+        const bool pass_nt = state_total * sizeof(qsv::c64) > (uint64_t(256) << 20);
         // ---- staged circuits: task arrays of the rounds, the fill and the reduction ----
         struct Round
         {
@@ -368,6 +565,16 @@ namespace qcore
             hbm_bytes_ += 16.0 * amps * double(bc.blocks.size()) + 8.0 * amps + 8.0 * amps;
             launches_ += 1 + bc.blocks.size() + 2;
         }
+        for (const auto &pc : passed)
+        {
+            // the first pass does not read, the last does not write
+            const double amps = double(uint64_t(1) << circuits_[pc.ci].n);
+            if (circuits_[pc.ci].n > pc.plan.m)
+                hbm_bytes_ += 16.0 * amps * double(pc.plan.passes.size() - 1);
+        }
+        for (const auto &L : plaunch)
+            launches_ += L.tasks.empty() ? 0 : 1;
+        launches_ += passed.empty() ? 0 : 1;
         int grid = 0;
         if (!small.empty())
         {
@@ -375,7 +582,11 @@ namespace qcore
             grid = std::min<int>(qsv::batch_lds_grid(T.block_size, small_max_n), (int)small.size());
         }
         // ---- streams and graph capture ----
-        const int ns = std::max(1, T.streams);
+        // no more streams than chains of launches: each takes 30 us to create
+        int chains = int(!small.empty()) + int(!staged.empty()) + (blocked.empty() ? 0 : T.streams) + int(plaunch.size() > 3);
+        for (int i = 0; i < 3; ++i)
+            chains += int(!plaunch[i].tasks.empty());
+        const int ns = std::clamp(chains, 1, T.streams);
         for (int i = 0; i < ns; ++i)
         {
             hipStream_t s;
@@ -397,7 +608,7 @@ namespace qcore
         // or issued directly by run_direct
         work_ = [this, blocked = std::move(blocked), blocked_state, blocked_partial, rounds, nstaged, kq_staged,
                  stage_bits = T.stage_bits, zsum_offset, zsum_blocks_total, zsum_qubits_total, grid, nsmall,
-                 small_max_n, ns, block_size = T.block_size, x3 = x3_]() mutable {
+                 small_max_n, ns, block_size = T.block_size, x3 = x3_, plaunch, pops_off, pz_off, pz_count, pass_nt]() mutable {
             hipStream_t s0 = streams_[0];
             qsv::check(hipEventRecord(fork_join_[0], s0), "hipEventRecord");
             for (int i = 1; i < ns; ++i)
@@ -408,6 +619,17 @@ namespace qcore
             // circuits (biggest first) the ones after it
             int next = 0;
             auto stream = [&]() { return streams_[ns == 1 ? 0 : 1 + (next++) % (ns - 1)]; };
+            // the pass rounds are the longest chain; then each kind of whole circuits
+            const auto *prog = static_cast<const char *>(d_prog_);
+            auto launch_tasks = [&](hipStream_t s, const PassLaunch &L) {
+                qsv::launch_pass_tasks(s, L.m, pass_nt, reinterpret_cast<const qsv::PassTask *>(prog + L.offset), int(L.tasks.size()), L.tiles,
+                                       reinterpret_cast<const qsv::PassRound *>(prog), reinterpret_cast<const qsv::PassOp *>(prog + pops_off));
+            };
+            for (size_t i = 3; i < plaunch.size(); ++i)
+                launch_tasks(s0, plaunch[i]);
+            for (size_t i = 3; i-- > 0;)
+                if (!plaunch[i].tasks.empty())
+                    launch_tasks(stream(), plaunch[i]);
             if (nstaged > 0)
             {
                 hipStream_t s = stream();
@@ -430,6 +652,8 @@ namespace qcore
                 qsv::check(hipEventRecord(fork_join_[ns + i], streams_[i]), "hipEventRecord");
                 qsv::check(hipStreamWaitEvent(s0, fork_join_[ns + i], 0), "hipStreamWaitEvent");
             }
+            if (pz_count > 0)
+                qsv::launch_pass_z(s0, reinterpret_cast<const qsv::PassZ *>(prog + pz_off), pz_count);
         };
         qsv::check(hipStreamBeginCapture(s0, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
         try
@@ -514,14 +738,19 @@ namespace qcore
 
     BatchTuning Batch::autotune()
     {
-        auto measure = [&](const BatchTuning &t) {
-            set_tuning(t);
+        auto time = [&] {
             run(nullptr); // warm-up (first replay)
             double best = 1e30;
             for (int r = 0; r < 2; ++r)
                 best = std::min(best, run(nullptr));
             return best;
         };
+        auto measure = [&](const BatchTuning &t) {
+            set_tuning(t);
+            return time();
+        };
+        const BatchTuning untuned = tuning_;
+        const double passes_s = passes_ ? time() : 1e30;
         BatchTuning best = tuning_;
         double best_s = measure(best);
         auto try_set = [&](auto setter, std::initializer_list<int> values) {
@@ -544,6 +773,12 @@ namespace qcore
         try_set([](BatchTuning &t, int v) { t.block_qubits = v / 16; t.stage_bits = v % 16; },
                 {4 * 16 + 0, 4 * 16 + 11, 4 * 16 + 12, 4 * 16 + 13, 5 * 16 + 0, 5 * 16 + 11, 5 * 16 + 12, 5 * 16 + 13});
         try_set([](BatchTuning &t, int v) { t.streams = v; }, {1, 2, 4});
+        if (passes_s <= best_s)
+        { // as before the search
+            set_tuning(untuned);
+            passes_ = true;
+            return untuned;
+        }
         set_tuning(best);
         return best;
     }

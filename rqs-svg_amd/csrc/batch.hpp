@@ -45,7 +45,9 @@ namespace qcore
         const BatchTuning &tuning() const { return tuning_; }
         // Block products of the circuits in HBM: 1 = FP32 MFMA (default), 3 = BF16x3
         // split-precision MFMA (three bf16 products, FP32 accumulation).  States stay
-        // complex64 and <Z> FP64 either way; the LDS-resident circuits are unaffected.
+        // complex64 and <Z> FP64 either way; the LDS-resident circuits are unaffected.  With no
+        // tuning set, circuit passes (FP64 arithmetic) take the place of the FP32 products and
+        // of the LDS-resident kernel.
         void set_precision(int mode);
         int precision() const { return x3_ ? 3 : 1; }
         // Runs every circuit from |0...0>, writes <Z_q> of circuit c at offset
@@ -57,7 +59,8 @@ namespace qcore
         // The plain method per circuit (complex128 simulators, one kernel per gate); returns
         // host wall seconds of the loop.
         double run_plain(double *expz);
-        // Coordinate search over the tuning parameters on this batch; keeps the best.
+        // Coordinate search over the tuning parameters on this batch, and of circuit passes where
+        // no tuning was set; keeps the best.
         BatchTuning autotune();
         uint64_t graph_nodes() const { return graph_nodes_; }
         // algorithmic HBM bytes and kernel launches of one run (prepares the batch)
@@ -87,6 +90,7 @@ namespace qcore
         int total_qubits_ = 0;
         BatchTuning tuning_;
         bool x3_ = false;
+        bool passes_ = true; // no tuning set: circuit passes
         bool prepared_ = false;
         int device_ = 0;
         std::vector<hipStream_t> streams_;
@@ -105,5 +109,7 @@ namespace qcore
         qsv::c64 *d_states_ = nullptr;
         double *d_partials_ = nullptr;
         float *d_mats_ = nullptr;
+        double *d_sums_ = nullptr; // tiles' sums of the circuits that run as passes
+        void *d_prog_ = nullptr;   // their rounds, operations, tasks and <Z> entries
     };
 } // namespace qcore

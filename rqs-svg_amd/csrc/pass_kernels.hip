@@ -298,51 +298,61 @@ namespace qsv
             }
         }
 
-        // GUARD: the state is smaller than the tile; indices past it read as zero and are not
-        // written.  One tile per workgroup.
-        template <class A, int M, bool NT, bool GUARD>
-        __global__ __launch_bounds__(1 << (M - 4), QSV_PASS_WAVES) void k_pass(A *__restrict__ s, PassTile tile, const PassRound *__restrict__ rounds_, const PassOp *__restrict__ ops_)
+        // The amplitude index of tile amplitude 0 of tile `t`: the bits of t at the qubits that
+        // are not tile qubits.
+        template <int M, class Qubit>
+        __device__ __forceinline__ uint64_t tile_base(uint64_t t, Qubit tq)
         {
-            constexpr int TB = M - 4; // thread-index bits
-            __shared__ double x[1 << M];
-            const RoundPtr rounds = (RoundPtr)rounds_;
-            const OpPtr ops = (OpPtr)ops_;
-            const uint32_t tid = threadIdx.x;
-            const uint64_t count = uint64_t(1) << tile.n;
-            uint64_t base = blockIdx.x;
             for (int b = 0; b < M; ++b)
             {
-                const uint64_t lo = base & ((uint64_t(1) << tile.tq[b]) - 1);
-                base = lo | ((base ^ lo) << 1);
+                const uint64_t lo = t & ((uint64_t(1) << tq(b)) - 1);
+                t = lo | ((t ^ lo) << 1);
             }
-            uint64_t idx = 0;    // this thread's amplitude index with the register bits 0
-            uint32_t slot = 0;   // the LDS address of its slot, register bits 0
-            uint64_t ro[4];      // the register bits' index and slot offsets
-            uint32_t rl[4];
-            auto layout = [&](RoundPtr R) {
-                idx = base;
-                slot = 0;
-#pragma unroll
-                for (int i = 0; i < TB; ++i)
-                {
-                    const uint32_t bit = (tid >> i) & 1;
-                    idx |= uint64_t(bit) << R->tq[i];
-                    slot ^= uint32_t(-int(bit)) & R->tl[i];
-                }
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                {
-                    ro[j] = uint64_t(1) << R->rq[j];
-                    rl[j] = R->rl[j];
-                }
-            };
-            auto roff = [&](int r) {
-                uint64_t o = 0;
+            return t;
+        }
+
+        // A thread's place in the current round's layout.
+        struct Place
+        {
+            uint64_t idx;   // its amplitude index with the register bits 0
+            uint64_t ro[4]; // the register bits' index offsets
+            __device__ __forceinline__ uint64_t at(int r) const
+            {
+                uint64_t o = idx;
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
                     if ((r >> j) & 1)
                         o |= ro[j];
                 return o;
+            }
+        };
+
+        // The rounds on one tile.  load(i): amplitude i of the state; x: 2^M doubles of LDS.
+        template <int M, class Load>
+        __device__ __forceinline__ void run_rounds(Amps &a, Place &at_, double *x, uint64_t base, const PassRound *__restrict__ rounds_, int nrounds, const PassOp *__restrict__ ops_, Load load)
+        {
+            constexpr int TB = M - 4; // thread-index bits
+            const RoundPtr rounds = (RoundPtr)rounds_;
+            const OpPtr ops = (OpPtr)ops_;
+            const uint32_t tid = threadIdx.x;
+            uint32_t slot = 0; // the LDS address of the thread's slot, register bits 0
+            uint32_t rl[4];    // the register bits' slot offsets
+            auto layout = [&](RoundPtr R) {
+                at_.idx = base;
+                slot = 0;
+#pragma unroll
+                for (int i = 0; i < TB; ++i)
+                {
+                    const uint32_t bit = (tid >> i) & 1;
+                    at_.idx |= uint64_t(bit) << R->tq[i];
+                    slot ^= uint32_t(-int(bit)) & R->tl[i];
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                {
+                    at_.ro[j] = uint64_t(1) << R->rq[j];
+                    rl[j] = R->rl[j];
+                }
             };
             auto rslot = [&](int r) {
                 uint32_t o = 0;
@@ -353,7 +363,6 @@ namespace qsv
                 return o;
             };
             auto at = [&](uint32_t address) -> double & { return *reinterpret_cast<double *>(reinterpret_cast<char *>(x) + address); };
-            Amps a;
             uint32_t adr[16]; // LDS addresses of the thread's amplitudes in the current layout
             layout(rounds);
 #pragma unroll
@@ -362,8 +371,7 @@ namespace qsv
 #pragma unroll
             for (int r = 0; r < 16; ++r)
             {
-                const uint64_t i = idx | roff(r);
-                const v2d v = !GUARD || i < count ? pload<NT>(s + i) : v2d{0.0, 0.0};
+                const v2d v = load(at_.at(r));
                 a.x[r] = v.x;
                 a.y[r] = v.y;
             }
@@ -371,7 +379,7 @@ namespace qsv
             // first touch by a scalar load would cost a memory round trip (13 qubits, one tile of
             // 388 operations: 235 -> 121 us).
             {
-                const uint32_t first = rounds[0].first, last = rounds[tile.nrounds - 1].first + rounds[tile.nrounds - 1].count;
+                const uint32_t first = rounds[0].first, last = rounds[nrounds - 1].first + rounds[nrounds - 1].count;
                 auto touch = [&](const void *p, uint32_t bytes) {
                     uint32_t v = 0;
                     for (uint32_t b = tid * 128; b < bytes; b += (128u << TB))
@@ -379,9 +387,9 @@ namespace qsv
                     asm volatile("" ::"v"(v));
                 };
                 touch(ops_ + first, (last - first + 1) * uint32_t(sizeof(PassOp)));
-                touch(rounds_, uint32_t(tile.nrounds) * uint32_t(sizeof(PassRound)));
+                touch(rounds_, uint32_t(nrounds) * uint32_t(sizeof(PassRound)));
             }
-            for (int rd = 0; rd < tile.nrounds; ++rd)
+            for (int rd = 0; rd < nrounds; ++rd)
             {
                 const RoundPtr R = rounds + rd;
                 if (rd > 0)
@@ -424,20 +432,141 @@ namespace qsv
                     // the next operation's load is issued before this one's arithmetic
                     OpRegs nxt;
                     nxt.load(first + (i + 1));
-                    const uint64_t mine = __builtin_amdgcn_ballot_w64((idx & cur.cmask) == cur.cval);
+                    const uint64_t mine = __builtin_amdgcn_ballot_w64((at_.idx & cur.cmask) == cur.cval);
                     __builtin_amdgcn_sched_barrier(0);
                     apply_op(a, cur.kind, cur.sel, mine, cur.m[0], cur.m[1], cur.m[2], cur.m[3]);
                     __builtin_amdgcn_sched_barrier(0);
                     cur = nxt;
                 }
             }
+        }
+
+        // GUARD: the state is smaller than the tile; indices past it read as zero and are not
+        // written.  One tile per workgroup.
+        template <class A, int M, bool NT, bool GUARD>
+        __global__ __launch_bounds__(1 << (M - 4), QSV_PASS_WAVES) void k_pass(A *__restrict__ s, PassTile tile, const PassRound *__restrict__ rounds, const PassOp *__restrict__ ops)
+        {
+            __shared__ double x[1 << M];
+            const uint64_t count = uint64_t(1) << tile.n;
+            Amps a;
+            Place at;
+            run_rounds<M>(a, at, x, tile_base<M>(blockIdx.x, [&](int b) { return tile.tq[b]; }), rounds, tile.nrounds, ops,
+                          [&](uint64_t i) { return !GUARD || i < count ? pload<NT>(s + i) : v2d{0.0, 0.0}; });
 #pragma unroll
             for (int r = 0; r < 16; ++r)
             {
-                const uint64_t i = idx | roff(r);
+                const uint64_t i = at.at(r);
                 if (!GUARD || i < count)
                     pstore<NT>(s + i, v2d{a.x[r], a.y[r]});
             }
+        }
+
+        // Sum of the tile's probabilities (out[0]) and, per tile bit b, the sum over the half with
+        // the bit 0 less the one with it 1 (out[1 + b]): 4 register bits, 6 lane bits (each
+        // step of the wave's butterfly yields its bit's difference), then the waves through LDS.
+        // zb: the tile bit of each register bit and thread bit.
+        template <int M>
+        __device__ __forceinline__ void tile_z(const Amps &a, double *x, const uint8_t *zb, double *out)
+        {
+            constexpr int W = 1 << (M - 10); // waves
+            double v[11];
+            double p[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                p[r] = __builtin_fma(a.x[r], a.x[r], a.y[r] * a.y[r]);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+            { // halve p, keeping the differences of the bit
+                double d = 0.0;
+#pragma unroll
+                for (int r = 0; r < (8 >> j); ++r)
+                {
+                    const double lo = p[2 * r], hi = p[2 * r + 1];
+                    d += lo - hi;
+                    p[r] = lo + hi;
+                }
+                v[1 + j] = d;
+            }
+            v[0] = p[0];
+#pragma unroll
+            for (int k = 0; k < 6; ++k)
+            {
+                const double t = v[0], o = __shfl_xor(t, 1 << k);
+                v[0] = t + o;
+#pragma unroll
+                for (int j = 1; j < 5 + k; ++j)
+                    v[j] += __shfl_xor(v[j], 1 << k);
+                v[5 + k] = (threadIdx.x >> k) & 1 ? o - t : t - o;
+            }
+            pass_sync<M>(); // the last exchange's reads are done
+            const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+            if (lane == 0)
+#pragma unroll
+                for (int j = 0; j < 11; ++j)
+                    x[11 * wave + j] = v[j];
+            pass_sync<M>();
+            if (threadIdx.x <= M)
+            { // thread 0: the sum; thread 1 + i: register bit i, or thread bit i - 4
+                const int j = threadIdx.x;
+                double sum = 0.0;
+                for (int w = 0; w < W; ++w)
+                {
+                    const double y = x[11 * w + (j < 11 ? j : 0)];
+                    sum += j >= 11 && ((w >> (j - 11)) & 1) ? -y : y;
+                }
+                out[j == 0 ? 0 : 1 + zb[j - 1]] = sum;
+            }
+        }
+
+        // One tile of one of several circuits per workgroup (PassTask).  Bound by FP64 arithmetic
+        // like k_pass: 96 circuits of 10-20 qubits run 8 rounds of up to 4172 tiles, 35 to 400 us
+        // each, and the whole circuits of up to 12 qubits beside the first; the batch takes 1.25
+        // ms where per-block launches, stage rounds and the LDS kernel took 2.7.
+        template <int M, bool NT>
+        __global__ __launch_bounds__(1 << (M - 4), QSV_PASS_WAVES) void k_pass_tasks(const PassTask *__restrict__ tasks_, int ntasks, const PassRound *__restrict__ rounds, const PassOp *__restrict__ ops)
+        {
+            __shared__ double x[1 << M];
+            const auto tasks = (const __attribute__((address_space(4))) PassTask *)tasks_;
+            int lo = 0, hi = ntasks - 1; // the last task that begins at or before this workgroup
+            while (lo < hi)
+            {
+                const int mid = (lo + hi + 1) >> 1;
+                if (tasks[mid].tile_begin <= blockIdx.x)
+                    lo = mid;
+                else
+                    hi = mid - 1;
+            }
+            const auto &T = tasks[lo];
+            const uint32_t t = blockIdx.x - T.tile_begin, flags = T.flags;
+            c64 *const s = T.state;
+            Amps a;
+            Place at;
+            run_rounds<M>(a, at, x, tile_base<M>(t, [&](int b) { return (T.tq[b >> 2] >> (8 * (b & 3))) & 255u; }), rounds + T.first_round, int(T.nrounds), ops,
+                          [&](uint64_t i) { return flags & kPassZeroState ? v2d{i == 0 ? 1.0 : 0.0, 0.0} : pload<NT>(s + i); });
+            if (flags & kPassExpectZ)
+                tile_z<M>(a, x, reinterpret_cast<const uint8_t *>(tasks_[lo].zb), T.sums + uint64_t(t) * kPassSums);
+            else
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    pstore<NT>(s + at.at(r), v2d{a.x[r], a.y[r]});
+        }
+
+        // <Z_q> of a circuit from its tiles' sums: one wave per qubit; lane l adds tiles l,
+        // l + 64, ... in order, then a fixed tree.
+        __global__ __launch_bounds__(64) void k_pass_z(const PassZ *__restrict__ qubits)
+        {
+            const PassZ Q = qubits[blockIdx.x];
+            double acc = 0.0;
+            for (uint32_t t = threadIdx.x; t < Q.ntiles; t += 64)
+            {
+                const double v = Q.sums[uint64_t(t) * kPassSums + Q.slot];
+                acc += (t & Q.sign) ? -v : v;
+            }
+#pragma unroll
+            for (int k = 32; k >= 1; k /= 2)
+                acc += __shfl_down(acc, k);
+            if (threadIdx.x == 0)
+                *Q.out = acc;
         }
     } // namespace
 
@@ -475,6 +604,30 @@ namespace qsv
         else
             nt ? go(k_pass<A, 12, true, false>) : go(k_pass<A, 12, false, false>);
         check(hipGetLastError(), "pass kernel");
+    }
+
+    void launch_pass_tasks(hipStream_t st, int m, bool nt, const PassTask *tasks, int ntasks, uint32_t tiles, const PassRound *rounds, const PassOp *ops)
+    {
+        if (tasks == nullptr || rounds == nullptr || ops == nullptr || ntasks < 1 || tiles < uint32_t(ntasks))
+            throw std::runtime_error("pass: no tasks");
+        auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(tiles), dim3(1 << (m - 4)), 0, st, tasks, ntasks, rounds, ops); };
+        if (m == 10)
+            nt ? go(k_pass_tasks<10, true>) : go(k_pass_tasks<10, false>);
+        else if (m == 11)
+            nt ? go(k_pass_tasks<11, true>) : go(k_pass_tasks<11, false>);
+        else if (m == 12)
+            nt ? go(k_pass_tasks<12, true>) : go(k_pass_tasks<12, false>);
+        else
+            throw std::runtime_error("pass: tile size out of range");
+        check(hipGetLastError(), "pass kernel");
+    }
+
+    void launch_pass_z(hipStream_t st, const PassZ *qubits, uint32_t count)
+    {
+        if (qubits == nullptr || count < 1)
+            throw std::runtime_error("pass: no qubits");
+        hipLaunchKernelGGL(k_pass_z, dim3(count), dim3(64), 0, st, qubits);
+        check(hipGetLastError(), "pass <Z> kernel");
     }
 
     template void launch_pass<c128>(hipStream_t, c128 *, int, int, const uint8_t *, const PassRound *, int, const PassOp *);

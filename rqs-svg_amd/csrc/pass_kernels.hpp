@@ -62,4 +62,31 @@ namespace qsv
     // operations past the last round's).
     template <class A>
     void launch_pass(hipStream_t s, A *state, int n, int m, const uint8_t *tq, const PassRound *rounds, int nrounds, const PassOp *ops);
+
+    // One pass of one circuit among several (the batching form), complex64 states: tiles
+    // tile_begin .. of the launch.  The first pass may start from |0...0> without reading, the
+    // last one write its tiles' sums (kPassSums doubles each: all probabilities, then per
+    // tile bit those with the bit 0 less those with it 1) in place of the amplitudes.  A circuit
+    // smaller than the tile does both (its amplitudes past 2^n stay zero).
+    constexpr uint32_t kPassZeroState = 1, kPassExpectZ = 2;
+    constexpr int kPassSums = 16;
+    struct alignas(16) PassTask
+    {
+        c64 *state;
+        double *sums;
+        uint32_t tile_begin, first_round, nrounds, flags;
+        uint32_t tq[4]; // tile qubits, ascending, a byte each (words: they become scalar loads)
+        uint8_t zb[16]; // tile bit of the last round's 4 register bits and its thread bits
+    };
+    // tasks in device memory, tile_begin ascending from 0; tiles: those of all tasks.
+    void launch_pass_tasks(hipStream_t s, int m, bool nt, const PassTask *tasks, int ntasks, uint32_t tiles, const PassRound *rounds, const PassOp *ops);
+
+    // <Z_q> of one qubit: the sum over tiles of sums[slot], negative where tile & sign.
+    struct alignas(16) PassZ
+    {
+        const double *sums;
+        double *out;
+        uint32_t ntiles, slot, sign, pad;
+    };
+    void launch_pass_z(hipStream_t s, const PassZ *qubits, uint32_t count);
 } // namespace qsv

@@ -125,3 +125,40 @@ def test_fused_modes_asked_for_stages(gpu, precision, m):
             states.append(sim.statevector())
     assert counts[0] == counts[1] == counts[2] and counts[0][0] == len(circ)
     assert np.array_equal(states[0], states[1]) and np.array_equal(states[0], states[2])
+
+
+# Batches with no tuning set run as passes: the circuits of up to 12 qubits never leave FP64; a
+# larger one is rounded to FP32 after every pass but the last (2^-24 of each modulus, carried
+# along unchanged), and |d<Z>| <= 2 ||d|| + ||d||^2.  Together, alone, replayed and launched
+# without the graph the circuits give the same bits.
+@pytest.mark.parametrize("mode", [1, 3])
+def test_batch_as_passes(gpu, oracle, mode):
+    work = []
+    for n in list(range(1, 15)) + ([15, 16, 17, 19] if mode == 1 else []):
+        for depth in (1, 5) if n < 17 else (3,):
+            work.append((n, circuits.variational_batch(1, seed=100 * n + depth, nmin=n, nmax=n, dmin=depth, dmax=depth)[0][1]))
+    work.append((9, [("h", 3, (), -1), ("z", 3, (), 8), ("t", 0, (), -1), ("sx", 8, (), 0), ("u3", 5, (0.4, 1.0, 2.0), 2)]))
+    work.append((13, [("y", 12, (), -1), ("p", 12, (0.3,), 0), ("x", 0, (), 12)]))  # one kind of gate a tile
+    ref, whole = pyqcs.Batch(oracle), pyqcs.Batch(gpu)
+    for n, g in work:
+        ref.add(n, g)
+        whole.add(n, g)
+    whole.set_precision(mode)
+    want, _ = ref.run()
+    got, _ = whole.run()
+    for again, _ in (whole.run(), whole.run_direct(), whole.run()):
+        assert all(np.array_equal(x, y) for x, y in zip(got, again))
+    for (n, g), z, w in zip(work, got, want):
+        with_alone = pyqcs.Batch(gpu)
+        with_alone.add(n, g)
+        with_alone.set_precision(mode)
+        alone, _ = with_alone.run()
+        rounded = with_alone.traffic()["hbm_bytes"] / (16.0 * 2 ** n)
+        d = rounded * 2.0 ** -24
+        print("n", n, "gates", len(g), "roundings", rounded, "max|d<Z>|", np.max(np.abs(z - w)), flush=True)
+        assert rounded == 0 if n <= 12 else rounded < len(g)
+        assert np.max(np.abs(z - w)) <= 2 * d + d * d + 1e-13
+        assert np.array_equal(alone[0], z)
+        with_alone.close()
+    whole.close()
+    ref.close()
