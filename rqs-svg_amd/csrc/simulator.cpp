@@ -312,6 +312,7 @@ namespace qcore
         state_changed();
         if (fused_)
             fused_->drop();
+        consistent_ = m0_.empty() && m1_.empty();
         with_state([&](auto *st) { qsv::launch_fill_random(stream_, st, uint64_t(1) << n_, seed_); });
     }
 
@@ -319,6 +320,7 @@ namespace qcore
     {
         m0_.clear();
         m1_.clear();
+        consistent_ = true;
     }
 
     void Simulator::check_operands(const std::vector<int> &t, const std::vector<int> &ng, const std::vector<int> &ps) const
@@ -483,7 +485,13 @@ namespace qcore
             }
         }
         if (fused_)
+        {
+            // matrix products over more qubits than the gate's own: zeros stay zero only while
+            // every amplitude is finite
+            if (!m0_.empty() || !m1_.empty())
+                consistent_ = false;
             fused_->enqueue(r);
+        }
         else
             apply_resolved(r);
         m0_ = keep[0];
@@ -818,8 +826,15 @@ namespace qcore
         (result ? m1_ : m0_).push_back(q);
         const double pk = result ? p1 : p0;
         const double scale = (renormalize_ && pk > 0) ? 1.0 / std::sqrt(pk) : 1.0;
-        prof_begin(QCS_EXT_K_COLLAPSE, S * (1ull << (n_ - 1)) * (scale != 1.0 ? 3.0 : 1.0));
-        with_state([&](auto *st) { qsv::launch_collapse(stream_, st, n_, tq, result, scale); });
+        // qubits measured before whose other halves are zero already
+        std::vector<int> fixed;
+        if (consistent_)
+            for (int x : ops)
+                if (x != tq)
+                    fixed.push_back(x);
+        std::sort(fixed.begin(), fixed.end());
+        prof_begin(QCS_EXT_K_COLLAPSE, S * std::ldexp(0.5, n_ - int(fixed.size())) * (scale != 1.0 ? 3.0 : 1.0));
+        with_state([&](auto *st) { qsv::launch_collapse(stream_, st, n_, tq, result, scale, fixed.data(), int(fixed.size()), setb); });
         prof_end();
         return result;
     }
@@ -986,9 +1001,10 @@ namespace qcore
             return levels_total_;
         ensure_levels();
         prof_begin(QCS_EXT_K_REDUCE, (c64_state() ? 8.0 : 16.0) * (1ull << n_));
-        with_state([&](auto *st) { qsv::build_fold_levels(stream_, st, uint64_t(1) << n_, levels_); });
+        std::vector<double *> levels = levels_;
+        levels.back() = pinned_; // the total; a search starts one level below
+        with_state([&](auto *st) { qsv::build_fold_levels(stream_, st, uint64_t(1) << n_, levels); });
         prof_end();
-        qsv::check(hipMemcpyAsync(pinned_, levels_.back(), sizeof(double), hipMemcpyDeviceToHost, stream_), "copy");
         qsv::check(hipStreamSynchronize(stream_), "sync");
         levels_total_ = pinned_[0];
         levels_valid_ = true;
@@ -1145,6 +1161,7 @@ namespace qcore
         if (!fused_)
             throw std::runtime_error("recording plan timings needs a fused precision mode (1, 2 or 3, allocated)");
         state_changed();
+        consistent_ = m0_.empty() && m1_.empty();
         return fused_->record_plans(capacity, features, log2_us);
     }
 
@@ -1167,6 +1184,7 @@ namespace qcore
         if (count < 0 || (count > 0 && (!features || !log2_us)))
             throw std::runtime_error("planner_record: bad output buffers");
         state_changed();
+        consistent_ = m0_.empty() && m1_.empty();
         fused_->record(count, seed, features, log2_us);
     }
 

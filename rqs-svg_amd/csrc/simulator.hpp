@@ -164,6 +164,8 @@ namespace qcore
         bool levels_valid_ = false;
         double levels_total_ = 0.0;
         void state_changed() { levels_valid_ = false; }
+        // every amplitude that contradicts a measured qubit's value is zero
+        bool consistent_ = true;
         double *pinned_ = nullptr; // pinned host memory: 64 doubles of results, then the staging area of small pass programs
         static constexpr size_t kPinnedResults = 64, kSmallProgram = 64 << 10;
         // pass programs (rounds and operations): small ones use the end of pinned_ and of work_

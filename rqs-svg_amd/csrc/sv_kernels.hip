@@ -766,15 +766,17 @@ namespace qsv
         }
 
         // ---------------- collapse ----------------
+        // The pairs of qubit tq in the subspace sub (tq among its operands).  Bound by memory:
+        // 27 qubits complex128, alone 196 us; each qubit fixed before halves it (measuring all
+        // from qubit 0 up: 24 of these 4.1 -> 0.5 ms).
         template <class A>
-        __global__ __launch_bounds__(kBlock) void k_collapse(A *__restrict__ s, uint64_t half, int tq, int result, double scale, int rescale)
+        __global__ __launch_bounds__(kBlock) void k_collapse(A *__restrict__ s, uint64_t pairs, Subspace sub, int tq, int result, double scale, int rescale)
         {
             uint64_t i = uint64_t(blockIdx.x) * kBlock + threadIdx.x;
             const uint64_t bit = uint64_t(1) << tq;
-            for (; i < half; i += uint64_t(gridDim.x) * kBlock)
+            for (; i < pairs; i += uint64_t(gridDim.x) * kBlock)
             {
-                uint64_t lo = i & (bit - 1);
-                uint64_t i0 = lo | ((i ^ lo) << 1);
+                const uint64_t i0 = expand(i, sub);
                 uint64_t kill = result ? i0 : (i0 | bit);
                 uint64_t keep = result ? (i0 | bit) : i0;
                 sta(s + kill, v2d{0.0, 0.0});
@@ -788,13 +790,14 @@ namespace qsv
 
         // Collapse on a qubit whose runs are shorter than a line (2^tq amplitudes of S bytes,
         // fewer than 128 B): every amplitude is read and written, zeroed or scaled by its bit,
-        // so that all accesses cover whole lines.
+        // so that all accesses cover whole lines.  sub: operands of line bits and above.
         template <class A>
-        __global__ __launch_bounds__(kBlock) void k_collapse_lines(A *__restrict__ s, uint64_t count, int tq, int result, double scale)
+        __global__ __launch_bounds__(kBlock) void k_collapse_lines(A *__restrict__ s, uint64_t count, Subspace sub, int tq, int result, double scale)
         {
-            uint64_t i = uint64_t(blockIdx.x) * kBlock + threadIdx.x;
-            for (; i < count; i += uint64_t(gridDim.x) * kBlock)
+            uint64_t t = uint64_t(blockIdx.x) * kBlock + threadIdx.x;
+            for (; t < count; t += uint64_t(gridDim.x) * kBlock)
             {
+                const uint64_t i = expand(t, sub);
                 const v2d a = lda(s + i);
                 const bool kept = int((i >> tq) & 1) == result;
                 sta(s + i, kept ? v2d{a.x * scale, a.y * scale} : v2d{0.0, 0.0});
@@ -1602,47 +1605,42 @@ namespace qsv
     } // namespace
 
     template <class A>
-    void reduce_pair_probs(hipStream_t s, const A *state, const Subspace &sub, uint64_t tbit, uint64_t nitems, double *work, double out[2])
+    void reduce_pair_probs(hipStream_t s, const A *state, const Subspace &sub, uint64_t tbit, uint64_t nitems, double *work, double *out)
     {
-        // work layout: [result(2)] [level arrays ...]
-        double *dev_out = work;
         uint64_t g = (nitems + kTile - 1) / kTile;
-        double *lvl = work + 2;
+        double *lvl = work; // level arrays
         if (g == 1)
         {
-            hipLaunchKernelGGL(k_reduce_pair<A>, dim3(1), dim3(kBlock), 0, s, state, nitems, sub, tbit, dev_out, uint64_t(1));
+            hipLaunchKernelGGL(k_reduce_pair<A>, dim3(1), dim3(kBlock), 0, s, state, nitems, sub, tbit, out, uint64_t(1));
             after_launch("reduce kernel");
         }
         else
         {
             hipLaunchKernelGGL(k_reduce_pair<A>, dim3(g), dim3(kBlock), 0, s, state, nitems, sub, tbit, lvl, g);
             after_launch("reduce kernel");
-            finish_tiles<2>(s, lvl, g, g, lvl + 2 * g, dev_out);
+            finish_tiles<2>(s, lvl, g, g, lvl + 2 * g, out);
         }
-        check(hipMemcpyAsync(out, dev_out, 2 * sizeof(double), hipMemcpyDeviceToHost, s), "reduce copy");
         check(hipStreamSynchronize(s), "reduce sync");
     }
 
     template <class A>
     void reduce_probs(hipStream_t s, const A *state, uint64_t count, double *work, double *out)
     {
-        double *dev_out = work;
         if (reduce_per_unit<A>() == 2 && (count & 1))
             throw std::runtime_error("reduce: complex64 states have an even amplitude count");
         uint64_t g = (count / reduce_per_unit<A>() + kTile - 1) / kTile;
-        double *lvl = work + 2;
+        double *lvl = work; // level arrays
         if (g == 1)
         {
-            hipLaunchKernelGGL(k_reduce_probs<A>, dim3(1), dim3(kBlock), 0, s, state, count, dev_out);
+            hipLaunchKernelGGL(k_reduce_probs<A>, dim3(1), dim3(kBlock), 0, s, state, count, out);
             after_launch("reduce kernel");
         }
         else
         {
             hipLaunchKernelGGL(k_reduce_probs<A>, dim3(g), dim3(kBlock), 0, s, state, count, lvl);
             after_launch("reduce kernel");
-            finish_tiles<1>(s, lvl, g, g, lvl + g, dev_out);
+            finish_tiles<1>(s, lvl, g, g, lvl + g, out);
         }
-        check(hipMemcpyAsync(out, dev_out, sizeof(double), hipMemcpyDeviceToHost, s), "reduce copy");
         check(hipStreamSynchronize(s), "reduce sync");
     }
 
@@ -1773,20 +1771,37 @@ namespace qsv
     }
 
     template <class A>
-    void launch_collapse(hipStream_t s, A *state, int n, int tq, int result, double scale)
+    void launch_collapse(hipStream_t s, A *state, int n, int tq, int result, double scale, const int *fixed, int nfixed, uint64_t fixed_ones)
     {
         if (tq < 0 || tq >= n || n < 1)
             throw std::runtime_error("collapse: qubit out of range");
-        if ((uint64_t(sizeof(A)) << tq) < 128 && n >= 8)
+        // Everything off the fixed qubits' values is zero and stays so.  Fixed qubits below a
+        // line's bits do not narrow the lines to touch: they are left out, and whole lines with
+        // their zeros are rewritten.
+        const int line_bits = sizeof(A) == 16 ? 3 : 4;
+        Subspace sub{};
+        bool have_tq = tq < line_bits && n >= 8; // handled inside the lines
+        const bool lines = have_tq;
+        for (int i = 0; i <= nfixed; ++i)
         {
-            // runs of 2^tq amplitudes shorter than a line: whole lines read and written
-            const uint64_t count = uint64_t(1) << n;
-            hipLaunchKernelGGL(k_collapse_lines<A>, dim3(grid_for(count, kBlock * 4)), dim3(kBlock), 0, s, state, count, tq, result, scale);
-            after_launch("collapse kernel (whole lines)");
-            return;
+            const int q = i < nfixed ? fixed[i] : n;
+            if (i < nfixed && (q < 0 || q >= n || q == tq || (i > 0 && q <= fixed[i - 1])))
+                throw std::runtime_error("collapse: fixed qubits must be ascending, inside the state and not the measured one");
+            if (!have_tq && q > tq)
+            {
+                sub.ops[sub.nops++] = tq;
+                have_tq = true;
+            }
+            if (q < line_bits || q == n)
+                continue;
+            sub.ops[sub.nops++] = q;
+            sub.set_bits |= fixed_ones & (uint64_t(1) << q);
         }
-        uint64_t half = uint64_t(1) << (n - 1);
-        hipLaunchKernelGGL(k_collapse<A>, dim3(grid_for(half, kBlock)), dim3(kBlock), 0, s, state, half, tq, result, scale, scale != 1.0 ? 1 : 0);
+        const uint64_t count = uint64_t(1) << (n - sub.nops);
+        if (lines)
+            hipLaunchKernelGGL(k_collapse_lines<A>, dim3(grid_for(count, kBlock * 4)), dim3(kBlock), 0, s, state, count, sub, tq, result, scale);
+        else
+            hipLaunchKernelGGL(k_collapse<A>, dim3(grid_for(count, kBlock)), dim3(kBlock), 0, s, state, count, sub, tq, result, scale, scale != 1.0 ? 1 : 0);
         after_launch("collapse kernel");
     }
 
@@ -1933,8 +1948,8 @@ namespace qsv
         if (off > kNoAllocLevelBytes)
             throw std::runtime_error("sample_noalloc: prefix levels exceed the scratch array");
         uint64_t *outcomes = reinterpret_cast<uint64_t *>(base + kNoAllocLevelBytes);
+        levels[ns - 2] = pinned; // the total; the search starts one level below
         fold_into(s, state, sz, ns, levels);
-        check(hipMemcpyAsync(pinned, levels[ns - 2], sizeof(double), hipMemcpyDeviceToHost, s), "copy");
         check(hipStreamSynchronize(s), "sync");
         const double total = pinned[0];
         if (nshots == 0)
@@ -2099,7 +2114,7 @@ namespace qsv
     template void reduce_pair_probs<A>(hipStream_t, const A *, const Subspace &, uint64_t, uint64_t, double *, double *);                               \
     template void reduce_probs<A>(hipStream_t, const A *, uint64_t, double *, double *);                                                                \
     template void expect_z<A>(hipStream_t, const A *, int, double *, double *, const int *, int, double *);                                            \
-    template void launch_collapse<A>(hipStream_t, A *, int, int, int, double);                                                                          \
+    template void launch_collapse<A>(hipStream_t, A *, int, int, int, double, const int *, int, uint64_t);                                               \
     template void renormalize_async<A>(hipStream_t, A *, uint64_t, double *);                                                                           \
     template void build_fold_levels<A>(hipStream_t, const A *, uint64_t, const std::vector<double *> &);                                                \
     template void launch_sample_search<A>(hipStream_t, const A *, uint64_t, const std::vector<double *> &, double, uint64_t, uint64_t, const int *, int, uint64_t *); \

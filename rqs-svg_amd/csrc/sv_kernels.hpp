@@ -99,9 +99,11 @@ namespace qsv
     // ---- reductions (FP64, canonical order of include/qcs_ext.h) ----
     // Workspace size in doubles for reduce_* on `nitems` items.
     uint64_t reduce_workspace(uint64_t nitems);
-    // {p0,p1} over the subspace `sub` (p1 at index | tbit); host out[2], stream synchronised.
+    // out: pinned host memory, which the last kernel writes (a copy of its own took 6 us); the
+    // stream is synchronised.
+    // {p0,p1} over the subspace `sub` (p1 at index | tbit)
     template <class A>
-    void reduce_pair_probs(hipStream_t s, const A *state, const Subspace &sub, uint64_t tbit, uint64_t nitems, double *work, double out[2]);
+    void reduce_pair_probs(hipStream_t s, const A *state, const Subspace &sub, uint64_t tbit, uint64_t nitems, double *work, double *out);
     // canonical sum of p(i) over all amplitudes
     template <class A>
     void reduce_probs(hipStream_t s, const A *state, uint64_t count, double *work, double *out);
@@ -123,7 +125,11 @@ namespace qsv
     void renormalize_async(hipStream_t s, A *state, uint64_t count, double *work);
 
     // ---- measurement collapse ----
-    template <class A> void launch_collapse(hipStream_t s, A *state, int n, int tq, int result, double scale);
+    // Zeroes qubit tq's half other than `result` and scales the rest.  fixed: qubits (ascending,
+    // values in fixed_ones) off whose values every amplitude is zero already; the rest of the
+    // state is then left alone.
+    template <class A>
+    void launch_collapse(hipStream_t s, A *state, int n, int tq, int result, double scale, const int *fixed = nullptr, int nfixed = 0, uint64_t fixed_ones = 0);
 
     // ---- sampling ----
     // Level sizes of the 64-ary fold for 2^n entries; level 0 is the state itself.
