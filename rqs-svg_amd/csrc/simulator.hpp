@@ -162,6 +162,9 @@ namespace qcore
         // the sampling prefix levels (and their total) describe the current state; cleared
         // by every call that may change the state
         bool levels_valid_ = false;
+        static constexpr uint64_t kShotChunk = 65536; // outcomes fetched at a time
+        uint64_t *shots_ = nullptr;                   // pinned, kept until free_memory
+        uint64_t shots_cap_ = 0;
         double levels_total_ = 0.0;
         void state_changed() { levels_valid_ = false; }
         // every amplitude that contradicts a measured qubit's value is zero

@@ -136,8 +136,9 @@ namespace qsv
     std::vector<uint64_t> fold_level_sizes(uint64_t count);
     template <class A>
     void build_fold_levels(hipStream_t s, const A *state, uint64_t count, const std::vector<double *> &levels);
+    // Outcomes of shots first .. first + nshots - 1 to out (device or pinned host memory).
     template <class A>
-    void launch_sample_search(hipStream_t s, const A *state, uint64_t count, const std::vector<double *> &levels, double total, uint64_t seed, uint64_t nshots, const int *p2l, int n, uint64_t *out_dev);
+    void launch_sample_search(hipStream_t s, const A *state, uint64_t count, const std::vector<double *> &levels, double total, uint64_t seed, uint64_t first, uint64_t nshots, const int *p2l, int n, uint64_t *out);
 
     // ---- sampling without allocation ----
     // The prefix levels and the outcomes live in a file-scope device array of

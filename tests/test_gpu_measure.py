@@ -51,3 +51,23 @@ def test_measurement_sequences(gpu, oracle, n, precision):
                 assert np.max(np.abs(a - b)) <= tol * max(1.0, np.max(np.abs(b)))
                 assert np.array_equal(a == 0, b == 0) or steps == ("gates",)  # gates: zeros by rounding
             assert unit or abs(g[4] - o[4]) <= tol * max(1.0, o[4])
+
+
+# Whole and partial blocks of 64 at the top level, one level and several; more shots than are
+# fetched at a time; a state whose zeros make long runs of equal prefixes.  Outcomes are integers
+# from FP64 sums in a fixed order: exactly the oracle's.
+@pytest.mark.parametrize("n,shots", [(1, 5), (2, 100), (5, 64), (6, 65), (7, 1000), (11, 70000), (12, 1), (13, 3000), (18, 65537)])
+def test_sampling_is_the_oracles(gpu, oracle, n, shots):
+    psi = random_state(n, n)
+    holes = np.where(np.arange(1 << n) % 7 < 5, 0.0, psi)
+    states = [psi] + ([holes / np.linalg.norm(holes)] if n > 3 else [])
+    for k, state in enumerate(states):
+        res = []
+        for lib in (gpu, oracle):
+            with pyqcs.Simulator(lib, n, seed=1) as sim:
+                sim.set_statevector(state)
+                res.append((sim.sample(shots, seed=9 + k), sim.probability_total()))
+                if lib is gpu:  # the buffer is kept: fewer shots, then as many again
+                    assert np.array_equal(sim.sample(max(1, shots // 3), seed=9 + k), res[-1][0][:max(1, shots // 3)])
+                    assert np.array_equal(sim.sample(shots, seed=9 + k), res[-1][0])
+        assert res[0][1] == res[1][1] and np.array_equal(res[0][0], res[1][0])
