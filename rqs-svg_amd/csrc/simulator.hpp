@@ -123,7 +123,7 @@ namespace qcore
         int run_passes(const std::vector<ResolvedGate> &gates);
         void reserve_program(size_t bytes);
         void ensure_levels();
-        uint64_t logical_chunk() const;
+        uint64_t stage_len() const;
         void ensure_stage();
 
         // profiling: events around each launch
@@ -176,9 +176,9 @@ namespace qcore
         size_t prog_cap_ = 0; // bytes of the two above
         hipEvent_t prog_copied_ = nullptr;
         bool prog_pending_ = false;
-        qsv::c128 *stage_dev_ = nullptr;
-        void *stage_host_ = nullptr;
-        uint64_t stage_len_ = 0;
+        static constexpr uint64_t kSlotLen = uint64_t(1) << 17, kSlots = 16; // 16 slots of 2 MiB
+        qsv::c128 *stage_ = nullptr, *stage_dev_ = nullptr; // pinned, and its device copy for loads
+        std::vector<hipEvent_t> stage_events_;
         std::vector<hipEvent_t> events_;
 
         bool profile_ = false;

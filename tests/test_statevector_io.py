@@ -124,3 +124,20 @@ def test_gpu_set_statevector_clears_measurement(gpu, oracle):
     o = _measure_then_set(oracle, n, psi)
     assert g[0] == o[0] and g[1] == o[1]
     assert np.max(np.abs(g[2] - o[2])) <= 1e-13
+
+
+# One part of a slot, one slot, few slots without copying threads, one ring, and several; with
+# and without a qubit mapping.  Amplitudes pass unchanged (complex64 states: rounded once).
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,precision", [(1, 0), (9, 0), (16, 0), (17, 0), (18, 0), (19, 2), (20, 0), (21, 1), (22, 0), (23, 0)])
+def test_state_through_the_slots(gpu, n, precision):
+    rng = np.random.default_rng(n)
+    mapping = [int(q) for q in rng.permutation(n)] if n % 2 else None
+    with pyqcs.Simulator(gpu, n, precision=precision, mapping=mapping) as sim:
+        for _ in range(2):  # the second pass finds the slots in use
+            psi = rng.standard_normal(1 << n) + 1j * rng.standard_normal(1 << n)
+            sim.set_statevector(psi)
+            want = psi.astype(np.complex64) if precision == 1 else psi
+            assert np.array_equal(sim.statevector(), want)
+        i = (1 << n) - 1
+        assert np.array_equal(sim.statevector()[[0, i // 2, i]], want[[0, i // 2, i]])
