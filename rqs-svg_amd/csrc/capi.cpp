@@ -430,9 +430,10 @@ extern "C"
             bool stop = false;
             for (int32_t i = 0; i < count && !stop; ++i)
             {
+                gates.emplace_back();
                 try
                 {
-                    qcore::CircuitGate g;
+                    qcore::CircuitGate &g = gates.back();
                     g.spec = qcore::make_gate(names[name_of[i]], params);
                     g.targets = vec(targets, nt[i]);
                     g.neg = vec(negctrls, nng[i]);
@@ -441,10 +442,10 @@ extern "C"
                     negctrls += nng[i];
                     ctrls += nps[i];
                     params += num_params[name_of[i]];
-                    gates.push_back(std::move(g));
                 }
                 catch (const std::exception &e)
                 {
+                    gates.pop_back();
                     refused = e.what();
                     stop = true;
                 }

@@ -740,7 +740,7 @@ namespace qcore
         }
     } // namespace
 
-    PassPlan plan_passes(const std::vector<PassGate> &gates, int n, int m, int amp_bytes)
+    PassPlan plan_passes(const std::vector<PassGate> &gates, int n, int m, int amp_bytes, const std::function<void(const PassPlan &, bool)> &planned)
     {
         if (n < 1 || n > qsv::kMaxQubits || m < qsv::kPassMinBits || m > qsv::kPassMaxBits || (n < m && m != qsv::kPassMinBits))
             throw std::runtime_error("passes: state or tile size out of range");
@@ -791,6 +791,8 @@ namespace qcore
             plan_rounds(P, gates, taken, ps.tq, n, m, line_bits);
             ps.nrounds = uint32_t(P.rounds.size()) - ps.first_round;
             P.passes.push_back(ps);
+            if (planned)
+                planned(P, rem.empty());
         }
         P.ops.resize(P.ops.size() + qsv::kPassOpPad, qsv::PassOp{});
         return P;

@@ -4,6 +4,7 @@
 #include "pass_kernels.hpp"
 #include "simulator.hpp"
 
+#include <functional>
 #include <vector>
 
 namespace qcore
@@ -76,6 +77,7 @@ namespace qcore
     // one only if on every shared qubit both act as a control or a phase.  A 2x2's target has
     // to be a tile qubit; controls and phases need not be.  amp_bytes: 16 or 8 (complex64),
     // which decides the low qubits that the first and last round of a sweep keep in the
-    // thread index, so that loads and stores cover whole lines.
-    PassPlan plan_passes(const std::vector<PassGate> &gates, int n, int m, int amp_bytes);
+    // thread index, so that loads and stores cover whole lines.  planned: called after each
+    // pass with the plan so far and whether that is all of it.
+    PassPlan plan_passes(const std::vector<PassGate> &gates, int n, int m, int amp_bytes, const std::function<void(const PassPlan &, bool)> &planned = {});
 } // namespace qcore

@@ -63,6 +63,9 @@ namespace qsv
     template <class A>
     void launch_pass(hipStream_t s, A *state, int n, int m, const uint8_t *tq, const PassRound *rounds, int nrounds, const PassOp *ops);
 
+    // Copies a program (16-byte units) from pinned host memory to device memory.
+    void launch_program_copy(hipStream_t s, void *dst, const void *src, size_t bytes);
+
     // One pass of one circuit among several (the batching form), complex64 states: tiles
     // tile_begin .. of the launch.  The first pass may start from |0...0> without reading, the
     // last one write its tiles' sums (kPassSums doubles each: all probabilities, then per

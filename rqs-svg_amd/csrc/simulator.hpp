@@ -116,7 +116,7 @@ namespace qcore
         void remap_physical(const std::vector<int> &dst);
         void apply_resolved(const ResolvedGate &r);
         // operands and mapping of a gate on a state without measured qubits
-        ResolvedGate resolve(const GateSpec &g, const std::vector<int> &targets, const std::vector<int> &neg, const std::vector<int> &pos) const;
+        void resolve(ResolvedGate &r, const GateSpec &g, const std::vector<int> &targets, const std::vector<int> &neg, const std::vector<int> &pos) const;
         void apply_run(const std::vector<ResolvedGate> &gates);
         // Applies gates as circuit passes and returns how many, or returns -1 with nothing
         // done where they have no such form or would not pay for their sweeps.

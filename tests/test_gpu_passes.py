@@ -52,6 +52,15 @@ def test_passes_match_gates_families(gpu, n, family):
     assert np.max(np.abs(a - b)) <= bound(circ, b)
 
 
+# programs longer than their staging area: several groups of passes, which start again at its
+# beginning; and more gates than are planned together
+@pytest.mark.parametrize("n,gates", [(13, 1500), (14, 5000), (20, 1200), (23, 400)])
+def test_long_programs_match_gates(gpu, n, gates):
+    circ = circuits.random_all_gates(n, gates, seed=gates, max_ctrls=2)
+    a, b = both(gpu, n, circ)
+    assert np.max(np.abs(a - b)) <= bound(circ, b)
+
+
 def test_run_refuses_like_the_gates(gpu, oracle):
     # a refused gate in the middle: the ones before it are applied, the message is the gate's
     n = 7
