@@ -302,6 +302,7 @@ namespace qcore
         std::vector<Staged> staged;
         std::vector<Blocked> blocked;
         std::vector<float> mats;
+        ComposeList compose;
         for (int ci : large)
         {
             const Circuit &C = circuits_[ci];
@@ -333,12 +334,12 @@ namespace qcore
                 {
                     Staged sc{ci, {}};
                     for (const auto &st : plan)
-                        sc.stages.push_back(prepare_stage(rg, st, kq, T.stage_bits, C.n, mats, x3_));
+                        sc.stages.push_back(prepare_stage(rg, st, kq, T.stage_bits, C.n, mats, x3_, false, &compose));
                     staged.push_back(std::move(sc));
                     continue;
                 }
             }
-            blocked.push_back(Blocked{ci, prepare_blocks(rg, plan_greedy(rg, kq), kq, C.n, mats, x3_)});
+            blocked.push_back(Blocked{ci, prepare_blocks(rg, plan_greedy(rg, kq), kq, C.n, mats, x3_, &compose)});
         }
         // largest first: round launches hand out the biggest states' tiles first, and with
         // sizes descending every state starts at a multiple of its own size
@@ -545,6 +546,7 @@ namespace qcore
             };
             zsum_offset = append(zt.data(), zt.size() * sizeof(qsv::ZsumTask));
         }
+        compose.append(mats);
         upload((void **)&d_mats_, mats.data(), mats.size() * sizeof(float));
         // algorithmic traffic and launches of one run (see qcs_ext_batch_traffic)
         hbm_bytes_ = 0;
@@ -600,6 +602,8 @@ namespace qcore
             fork_join_.push_back(e);
         }
         hipStream_t s0 = streams_[0];
+        compose.launch(s0, d_mats_);
+        qsv::check(hipStreamSynchronize(s0), "hipStreamSynchronize");
         const int nsmall = (int)small.size();
         const int nstaged = (int)staged.size();
         std::vector<uint64_t> blocked_state(state_off.begin() + nstaged, state_off.end());

@@ -149,7 +149,36 @@ namespace qcore
         return lay;
     }
 
+    namespace
+    {
+        // A gate's place in a block: target bits, and masks of the controls inside it.
+        struct InBlock
+        {
+            int tpos[4] = {0, 0, 0, 0};
+            unsigned need1 = 0, need0 = 0, tmask = 0;
+            InBlock(const ResolvedGate &g, const BlockLayout &lay)
+            {
+                for (int j = 0; j < g.spec.ntargets; ++j)
+                {
+                    tpos[j] = local_pos(lay.qubits, g.tphys[j]);
+                    tmask |= 1u << tpos[j];
+                }
+                for (int q : g.pphys)
+                    if (const int p = local_pos(lay.qubits, q); p >= 0)
+                        need1 |= 1u << p;
+                for (int q : g.nphys)
+                    if (const int p = local_pos(lay.qubits, q); p >= 0)
+                        need0 |= 1u << p;
+            }
+        };
+    } // namespace
+
     std::vector<cd> block_matrix(const std::vector<ResolvedGate> &gates, const PlannedBlock &b, const BlockLayout &lay)
+    {
+        return block_columns(gates, b, lay, 0, 1 << (int)lay.qubits.size());
+    }
+
+    std::vector<cd> block_columns(const std::vector<ResolvedGate> &gates, const PlannedBlock &b, const BlockLayout &lay, int first, int count)
     {
         const int kq = (int)lay.qubits.size();
         const int K = 1 << kq;
@@ -163,27 +192,11 @@ namespace qcore
             const int t = g.spec.ntargets;
             const int T = 1 << t;
             auto U = dense_matrix(g.spec);
-            int tpos[4] = {0, 0, 0, 0};
-            for (int j = 0; j < t; ++j)
-                tpos[j] = local_pos(lay.qubits, g.tphys[j]);
-            unsigned need1 = 0, need0 = 0; // control bits inside the block
-            for (int q : g.pphys)
-            {
-                int p = local_pos(lay.qubits, q);
-                if (p >= 0)
-                    need1 |= 1u << p;
-            }
-            for (int q : g.nphys)
-            {
-                int p = local_pos(lay.qubits, q);
-                if (p >= 0)
-                    need0 |= 1u << p;
-            }
-            unsigned tmask = 0;
-            for (int j = 0; j < t; ++j)
-                tmask |= 1u << tpos[j];
-            // M <- G M, applying the controlled gate to every column of M
-            for (int c = 0; c < K; ++c)
+            const InBlock at(g, lay);
+            const int *tpos = at.tpos;
+            const unsigned need1 = at.need1, need0 = at.need0, tmask = at.tmask;
+            // M <- G M, applying the controlled gate to the columns of M
+            for (int c = first; c < first + count; ++c)
             {
                 for (int r = 0; r < K; ++r)
                     col[r] = M[size_t(r) * K + c];
@@ -222,6 +235,99 @@ namespace qcore
             }
         }
         return M;
+    }
+
+    // ---- matrices composed on the device ----
+    void ComposeList::matrix(const std::vector<ResolvedGate> &all, const PlannedBlock &b, const BlockLayout &lay, size_t dst, bool x3)
+    {
+        const int kq = (int)lay.qubits.size();
+        qsv::ComposeJob j{};
+        j.kind = x3 ? qsv::kComposeX3 : kq == 5 ? qsv::kComposeThree : qsv::kComposeReal;
+        j.kq = uint32_t(kq);
+        j.first_gate = uint32_t(gates.size());
+        j.count = uint32_t(b.gates.size());
+        j.dst = uint32_t(dst);
+        if (kq > 5 || dst > 0xffffffffu)
+            throw std::runtime_error("compose: block or buffer too large");
+        for (int gi : b.gates)
+        {
+            const ResolvedGate &g = all[gi];
+            const InBlock at(g, lay);
+            qsv::ComposeGate c{};
+            c.coef = uint32_t(coefs.size());
+            c.t = uint8_t(g.spec.ntargets);
+            c.tmask = uint8_t(at.tmask);
+            c.need1 = uint8_t(at.need1);
+            c.need0 = uint8_t(at.need0);
+            for (int t = 0; t < g.spec.ntargets; ++t)
+            {
+                if (at.tpos[t] < 0)
+                    throw std::runtime_error("compose: a target outside its block");
+                c.tpos[t] = uint8_t(at.tpos[t]);
+            }
+            const auto U = dense_matrix(g.spec);
+            coefs.insert(coefs.end(), U.begin(), U.end());
+            gates.push_back(c);
+        }
+        jobs.push_back(j);
+    }
+
+    void ComposeList::table(const std::vector<std::vector<cd>> &diags, const std::vector<std::vector<int>> &bpos, int m, size_t dst)
+    {
+        const uint32_t first = uint32_t(diagonals.size());
+        int kq = 0;
+        for (size_t i = 0; i < diags.size(); ++i)
+        {
+            qsv::ComposeDiagonal d{};
+            d.coef = uint32_t(coefs.size());
+            kq = (int)bpos[i].size();
+            if (kq > 8 || diags[i].size() != size_t(1) << kq)
+                throw std::runtime_error("compose: bad diagonal");
+            for (int j = 0; j < kq; ++j)
+                d.bpos[j] = uint8_t(bpos[i][j]);
+            coefs.insert(coefs.end(), diags[i].begin(), diags[i].end());
+            diagonals.push_back(d);
+        }
+        if (dst > 0xffffffffu || m < qsv::kComposeTableBits)
+            throw std::runtime_error("compose: bad table");
+        for (uint32_t at = 0; at < (1u << m); at += 1u << qsv::kComposeTableBits)
+        {
+            qsv::ComposeJob j{};
+            j.kind = qsv::kComposeTable;
+            j.kq = uint32_t(kq);
+            j.first_gate = first;
+            j.count = uint32_t(diags.size());
+            j.dst = uint32_t(dst);
+            j.first = at;
+            jobs.push_back(j);
+        }
+    }
+
+    void ComposeList::append(std::vector<float> &mats)
+    {
+        if (jobs.empty())
+            return;
+        auto put = [&](const void *src, size_t bytes) {
+            while (mats.size() % 4)
+                mats.push_back(0.f);
+            const size_t off = mats.size();
+            mats.resize(off + (bytes + sizeof(float) - 1) / sizeof(float));
+            if (bytes)
+                std::memcpy(mats.data() + off, src, bytes);
+            return off;
+        };
+        jobs_at_ = put(jobs.data(), jobs.size() * sizeof(qsv::ComposeJob));
+        gates_at_ = put(gates.data(), gates.size() * sizeof(qsv::ComposeGate));
+        diagonals_at_ = put(diagonals.data(), diagonals.size() * sizeof(qsv::ComposeDiagonal));
+        coefs_at_ = put(coefs.data(), coefs.size() * sizeof(cd));
+    }
+
+    void ComposeList::launch(hipStream_t s, float *mats_dev) const
+    {
+        if (jobs.empty())
+            return;
+        qsv::launch_compose(s, mats_dev, reinterpret_cast<const qsv::ComposeJob *>(mats_dev + jobs_at_), uint32_t(jobs.size()), reinterpret_cast<const qsv::ComposeGate *>(mats_dev + gates_at_),
+                            reinterpret_cast<const qsv::ComposeDiagonal *>(mats_dev + diagonals_at_), reinterpret_cast<const double *>(mats_dev + coefs_at_));
     }
 
     FusedEngine::FusedEngine(Simulator &sim, int k, int mode) : sim_(sim), k_(k), f64_(mode == 2), x3_(mode == 3)
@@ -958,7 +1064,74 @@ namespace qcore
         }
     }
 
-    std::vector<PreparedBlock> prepare_blocks(const std::vector<ResolvedGate> &gates, const std::vector<PlannedBlock> &plan, int kq, int n, std::vector<float> &mats, bool x3)
+    // A block matrix in the form that its kernels read; dst holds (2K)^2 floats.
+    static void write_matrix(const std::vector<cd> &M, int kq, bool x3, float *dst)
+    {
+        const int K = 1 << kq, D = 2 * K;
+        const size_t per = size_t(D) * D;
+        std::vector<double> R(per);
+        for (int r = 0; r < K; ++r)
+            for (int c = 0; c < K; ++c)
+            {
+                const cd z = M[size_t(r) * K + c];
+                R[(2 * r) * D + 2 * c] = z.real();
+                R[(2 * r) * D + 2 * c + 1] = -z.imag();
+                R[(2 * r + 1) * D + 2 * c] = z.imag();
+                R[(2 * r + 1) * D + 2 * c + 1] = z.real();
+            }
+        if (!x3)
+        {
+            write_fp32_matrix(M, R, kq, dst);
+            return;
+        }
+        // bfloat16 high parts then low parts, 2 * per halves = per floats of storage
+        std::vector<uint16_t> parts(2 * per);
+        split_bf16(R.data(), per, parts.data(), parts.data() + per);
+        std::memcpy(dst, parts.data(), 2 * per * sizeof(uint16_t));
+    }
+
+    static bool is_diagonal(Kind k) { return k == Kind::GlobalPhase || k == Kind::PhaseOne || k == Kind::Diag1 || k == Kind::Diag2 || k == Kind::Identity; }
+
+    // The block's diagonal if every entry off it is exactly zero (a product of diagonal gates,
+    // or gates that cancel), else nothing.
+    static std::vector<cd> block_diagonal(const std::vector<ResolvedGate> &gates, const PlannedBlock &b, const BlockLayout &lay)
+    {
+        const int K = 1 << (int)lay.qubits.size();
+        std::vector<cd> d(K, 1.0);
+        if (std::all_of(b.gates.begin(), b.gates.end(), [&](int gi) { return is_diagonal(gates[gi].spec.kind); }))
+        {
+            for (int gi : b.gates)
+            {
+                const ResolvedGate &g = gates[gi];
+                const InBlock at(g, lay);
+                const auto U = dense_matrix(g.spec);
+                const int T = 1 << g.spec.ntargets;
+                for (unsigned x = 0; x < unsigned(K); ++x)
+                {
+                    if ((x & at.need1) != at.need1 || (x & at.need0))
+                        continue;
+                    int r = 0;
+                    for (int j = 0; j < g.spec.ntargets; ++j)
+                        r |= int((x >> at.tpos[j]) & 1) << j;
+                    d[x] = U[size_t(r) * T + r] * d[x];
+                }
+            }
+            return d;
+        }
+        // the first and the last column tell most blocks apart: no control holds, all do
+        for (int i = 0; i < K; ++i)
+        {
+            const int c = i == 0 ? 0 : i == 1 ? K - 1 : i - 1;
+            const auto M = block_columns(gates, b, lay, c, 1);
+            for (int r = 0; r < K; ++r)
+                if (r != c && M[size_t(r) * K + c] != cd(0.0, 0.0))
+                    return {};
+            d[c] = M[size_t(c) * K + c];
+        }
+        return d;
+    }
+
+    std::vector<PreparedBlock> prepare_blocks(const std::vector<ResolvedGate> &gates, const std::vector<PlannedBlock> &plan, int kq, int n, std::vector<float> &mats, bool x3, ComposeList *compose)
     {
         const int D = 2 << kq;
         const size_t per = size_t(D) * D;
@@ -968,32 +1141,15 @@ namespace qcore
         for (const auto &pb : plan)
         {
             const BlockLayout lay = layout_block(gates, pb, kq, n);
-            const auto M = block_matrix(gates, pb, lay);
             PreparedBlock b;
             b.kq = kq;
             b.gates = (int)pb.gates.size();
             b.matrix_offset = mats.size();
             mats.resize(mats.size() + per);
-            std::vector<double> R(per);
-            for (int r = 0; r < K; ++r)
-                for (int c = 0; c < K; ++c)
-                {
-                    const cd z = M[size_t(r) * K + c];
-                    R[(2 * r) * D + 2 * c] = z.real();
-                    R[(2 * r) * D + 2 * c + 1] = -z.imag();
-                    R[(2 * r + 1) * D + 2 * c] = z.imag();
-                    R[(2 * r + 1) * D + 2 * c + 1] = z.real();
-                }
-            if (x3)
-            { // bfloat16 high parts then low parts, 2 * per halves = per floats of storage
-                std::vector<uint16_t> parts(2 * per);
-                split_bf16(R.data(), per, parts.data(), parts.data() + per);
-                std::memcpy(mats.data() + b.matrix_offset, parts.data(), 2 * per * sizeof(uint16_t));
-            }
+            if (compose)
+                compose->matrix(gates, pb, lay, b.matrix_offset, x3);
             else
-            {
-                write_fp32_matrix(M, R, kq, mats.data() + b.matrix_offset);
-            }
+                write_matrix(block_matrix(gates, pb, lay), kq, x3, mats.data() + b.matrix_offset);
             std::vector<int> outside = lay.pos_out;
             outside.insert(outside.end(), lay.neg_out.begin(), lay.neg_out.end());
             uint64_t setb = 0;
@@ -1323,7 +1479,7 @@ namespace qcore
         return window.size() < grow.size() ? window : grow;
     }
 
-    PreparedStage prepare_stage(const std::vector<ResolvedGate> &gates, const PlannedStage &st, int kq, int m, int n, std::vector<float> &mats, bool x3, bool table)
+    PreparedStage prepare_stage(const std::vector<ResolvedGate> &gates, const PlannedStage &st, int kq, int m, int n, std::vector<float> &mats, bool x3, bool table, ComposeList *compose)
     {
         if ((int)st.tile.size() != m)
             throw std::runtime_error("stage: tile size mismatch");
@@ -1334,9 +1490,8 @@ namespace qcore
         const auto plan = plan_greedy(sub, kq);
         const int D = 2 << kq;
         const size_t per = size_t(D) * D;
-        const int K = 1 << kq;
         std::vector<qsv::StageBlock> desc;
-        std::vector<std::vector<cd>> diagonals; // per block: its diagonal, empty if not diagonal
+        std::vector<BlockLayout> lays;
         for (const auto &pb : plan)
         {
             if (pb.wide)
@@ -1347,41 +1502,7 @@ namespace qcore
             for (int i = m - 1; i >= 0 && (int)lay.qubits.size() < kq; --i)
                 if (local_pos(lay.qubits, st.tile[i]) < 0)
                     lay.qubits.push_back(st.tile[i]);
-            const auto M = block_matrix(sub, pb, lay);
-            {
-                // products of diagonal gates have exactly zero off-diagonal entries
-                bool diagonal = table;
-                for (int r = 0; r < K && diagonal; ++r)
-                    for (int c = 0; c < K && diagonal; ++c)
-                        diagonal = r == c || M[size_t(r) * K + c] == cd(0.0, 0.0);
-                std::vector<cd> d;
-                for (int e = 0; diagonal && e < K; ++e)
-                    d.push_back(M[size_t(e) * K + e]);
-                diagonals.push_back(std::move(d));
-            }
-            std::vector<double> R(per);
-            for (int r = 0; r < K; ++r)
-                for (int c = 0; c < K; ++c)
-                {
-                    const cd z = M[size_t(r) * K + c];
-                    R[(2 * r) * D + 2 * c] = z.real();
-                    R[(2 * r) * D + 2 * c + 1] = -z.imag();
-                    R[(2 * r + 1) * D + 2 * c] = z.imag();
-                    R[(2 * r + 1) * D + 2 * c + 1] = z.real();
-                }
             qsv::StageBlock sb{};
-            sb.matrix = uint32_t(mats.size());
-            mats.resize(mats.size() + per);
-            if (x3)
-            {
-                std::vector<uint16_t> parts(2 * per);
-                split_bf16(R.data(), per, parts.data(), parts.data() + per);
-                std::memcpy(mats.data() + sb.matrix, parts.data(), 2 * per * sizeof(uint16_t));
-            }
-            else
-            {
-                write_fp32_matrix(M, R, kq, mats.data() + sb.matrix);
-            }
             std::vector<char> is_block(m, 0);
             for (int j = 0; j < kq; ++j)
             {
@@ -1398,6 +1519,32 @@ namespace qcore
             for (int b = 0; b < m; ++b)
                 sb.lds[b] = qsv::stage_lds_offset(uint32_t(sb.w[b]));
             desc.push_back(sb);
+            lays.push_back(std::move(lay));
+        }
+        // With table: the diagonal blocks after the last other block become one table over
+        // the tile indices (tile index bit b = tile qubit b = the blocks' weight 1 << b),
+        // their diagonals multiplied in block order (FP64, rounded to FP32).  A stage of
+        // diagonal blocks only runs as that table alone; otherwise the stage kernel applies
+        // it as the tile is stored, and the blocks before it run as usual.
+        size_t first_trail = desc.size();
+        std::vector<std::vector<cd>> diagonals(desc.size());
+        while (table && first_trail > 0)
+        {
+            diagonals[first_trail - 1] = block_diagonal(sub, plan[first_trail - 1], lays[first_trail - 1]);
+            if (diagonals[first_trail - 1].empty())
+                break;
+            --first_trail;
+        }
+        for (size_t i = 0; i < (first_trail > 0 ? first_trail : desc.size()); ++i)
+        {
+            if (first_trail == 0 && compose)
+                break; // the table alone is read
+            desc[i].matrix = uint32_t(mats.size());
+            mats.resize(mats.size() + per);
+            if (compose)
+                compose->matrix(sub, plan[i], lays[i], desc[i].matrix, x3);
+            else
+                write_matrix(block_matrix(sub, plan[i], lays[i]), kq, x3, mats.data() + desc[i].matrix);
         }
         static_assert(sizeof(qsv::StageBlock) % 16 == 0, "StageBlock keeps 16-B alignment");
         PreparedStage p;
@@ -1411,20 +1558,25 @@ namespace qcore
         p.tsub.nops = m;
         for (int b = 0; b < m; ++b)
             p.tsub.ops[b] = st.tile[b];
-        // With table: the diagonal blocks after the last other block become one table over
-        // the tile indices (tile index bit b = tile qubit b = the blocks' weight 1 << b),
-        // their diagonals multiplied in block order (FP64, rounded to FP32).  A stage of
-        // diagonal blocks only runs as that table alone; otherwise the stage kernel applies
-        // it as the tile is stored, and the blocks before it run as usual.
-        size_t first_trail = desc.size();
-        while (first_trail > 0 && !diagonals[first_trail - 1].empty())
-            --first_trail;
         if (table && first_trail < desc.size())
         {
             while (mats.size() % 4)
                 mats.push_back(0.f);
-            (first_trail == 0 ? p.table_offset : p.trail_offset) = mats.size();
-            for (int idx = 0; idx < (1 << m); ++idx)
+            const size_t at = mats.size();
+            (first_trail == 0 ? p.table_offset : p.trail_offset) = at;
+            mats.resize(at + (size_t(2) << m));
+            if (compose)
+            {
+                std::vector<std::vector<int>> bpos;
+                for (size_t bi = first_trail; bi < desc.size(); ++bi)
+                {
+                    bpos.emplace_back();
+                    for (int jj = 0; jj < kq; ++jj)
+                        bpos.back().push_back(__builtin_ctz(unsigned(desc[bi].w[jj])));
+                }
+                compose->table({diagonals.begin() + long(first_trail), diagonals.end()}, bpos, m, at);
+            }
+            for (int idx = 0; !compose && idx < (1 << m); ++idx)
             {
                 cd v(1.0, 0.0);
                 for (size_t bi = first_trail; bi < desc.size(); ++bi)
@@ -1435,8 +1587,8 @@ namespace qcore
                             e |= 1 << jj;
                     v *= diagonals[bi][e];
                 }
-                mats.push_back(float(v.real()));
-                mats.push_back(float(v.imag()));
+                mats[at + 2 * size_t(idx)] = float(v.real());
+                mats[at + 2 * size_t(idx) + 1] = float(v.imag());
             }
             if (first_trail > 0)
                 desc.resize(first_trail);
@@ -1683,6 +1835,7 @@ namespace qcore
         // one matrix buffer for the whole flush: FP32 (complex64 modes) or FP64 entries
         std::vector<float> mats;
         std::vector<double> mats64;
+        ComposeList compose;
         struct Item
         {
             bool stage;
@@ -1702,7 +1855,7 @@ namespace qcore
                     it.st128 = prepare_stage128(gates, s, n, mats64, k);
                 else
                 {
-                    it.st = prepare_stage(gates, s, k, m, n, mats, x3_, true);
+                    it.st = prepare_stage(gates, s, k, m, n, mats, x3_, true, &compose);
                     attach_stage(it.st, state_, mats);
                 }
             }
@@ -1717,16 +1870,18 @@ namespace qcore
                         b.gates = 1;
                 }
                 else
-                    it.blocks = prepare_blocks(one, plan, kq_, n, mats, x3_);
+                    it.blocks = prepare_blocks(one, plan, kq_, n, mats, x3_, &compose);
             }
             items.push_back(std::move(it));
         }
+        compose.append(mats);
         const size_t bytes = f64_ ? mats64.size() * sizeof(double) : mats.size() * sizeof(float);
         reserve_matrices(bytes);
         std::memcpy(rhost_, f64_ ? (const void *)mats64.data() : (const void *)mats.data(), bytes);
         qsv::check(hipMemcpyAsync(rdev_, rhost_, bytes, hipMemcpyHostToDevice, sim_.stream_), "matrix upload");
         qsv::check(hipEventRecord(copy_done_, sim_.stream_), "hipEventRecord");
         copy_pending_ = true;
+        compose.launch(sim_.stream_, static_cast<float *>(rdev_));
         for (auto &it : items)
         {
             if (it.stage)
@@ -1794,13 +1949,16 @@ namespace qcore
             return;
         }
         std::vector<float> mats;
-        auto blocks = prepare_blocks(gates, plan, kq_, n, mats, x3_);
+        ComposeList compose;
+        auto blocks = prepare_blocks(gates, plan, kq_, n, mats, x3_, &compose);
+        compose.append(mats);
         const size_t bytes = mats.size() * sizeof(float);
         reserve_matrices(bytes);
         std::memcpy(rhost_, mats.data(), bytes);
         qsv::check(hipMemcpyAsync(rdev_, rhost_, bytes, hipMemcpyHostToDevice, sim_.stream_), "matrix upload");
         qsv::check(hipEventRecord(copy_done_, sim_.stream_), "hipEventRecord");
         copy_pending_ = true;
+        compose.launch(sim_.stream_, static_cast<float *>(rdev_));
         for (auto &b : blocks)
         {
             sim_.prof_begin(QCS_EXT_K_FUSED, b.bytes);

@@ -1,5 +1,6 @@
 // Precision form: complex64 state with queued gates fused into k-qubit dense blocks.
 #pragma once
+#include "compose_kernels.hpp"
 #include "fused_kernels.hpp"
 #include "simulator.hpp"
 
@@ -38,6 +39,28 @@ namespace qcore
     // 2^kq x 2^kq matrix (row-major) of the block's gates composed in FP64, in the local
     // basis of `lay.qubits`; gates' controls that are in lay.qubits act inside the matrix.
     std::vector<cd> block_matrix(const std::vector<ResolvedGate> &gates, const PlannedBlock &b, const BlockLayout &lay);
+    // Its columns first .. first + count - 1 only (the others are the identity's).
+    std::vector<cd> block_columns(const std::vector<ResolvedGate> &gates, const PlannedBlock &b, const BlockLayout &lay, int first, int count);
+
+    // Matrices and tables of a flush that the device composes: filled by prepare_blocks and
+    // prepare_stage, which then only leave room for them in `mats`.
+    struct ComposeList
+    {
+        std::vector<qsv::ComposeJob> jobs;
+        std::vector<qsv::ComposeGate> gates;
+        std::vector<qsv::ComposeDiagonal> diagonals;
+        std::vector<cd> coefs;
+        // the block's matrix, to be written dst floats into the buffer (x3: as bfloat16 parts)
+        void matrix(const std::vector<ResolvedGate> &gates, const PlannedBlock &b, const BlockLayout &lay, size_t dst, bool x3);
+        // the product table of diagonals over 2^m indices; bpos[i]: tile bits of diagonal i's bits
+        void table(const std::vector<std::vector<cd>> &diags, const std::vector<std::vector<int>> &bpos, int m, size_t dst);
+        // Appends the list to `mats`, and launches it on the uploaded copy.
+        void append(std::vector<float> &mats);
+        void launch(hipStream_t s, float *mats_dev) const;
+
+    private:
+        size_t jobs_at_ = 0, gates_at_ = 0, diagonals_at_ = 0, coefs_at_ = 0; // floats
+    };
 
     // A composed block ready to launch: matrix at matrix_offset (floats) of a matrix buffer.
     struct PreparedBlock
@@ -54,7 +77,8 @@ namespace qcore
     // Lays out and composes every planned block; appends the real (2^(kq+1))^2 matrices to
     // `mats` (host) in launch order.
     // x3: store each matrix as bfloat16 high parts followed by low parts (BF16x3 kernels).
-    std::vector<PreparedBlock> prepare_blocks(const std::vector<ResolvedGate> &gates, const std::vector<PlannedBlock> &plan, int kq, int n, std::vector<float> &mats, bool x3 = false);
+    // compose: the matrices go on that list instead of being composed here.
+    std::vector<PreparedBlock> prepare_blocks(const std::vector<ResolvedGate> &gates, const std::vector<PlannedBlock> &plan, int kq, int n, std::vector<float> &mats, bool x3 = false, ComposeList *compose = nullptr);
     // hi[i] + lo[i] ~ R[i] with both parts bfloat16 bits rounded to nearest even.
     void split_bf16(const double *R, size_t count, uint16_t *hi, uint16_t *lo);
     // Launches one prepared block whose matrices were uploaded to mats_dev.
@@ -120,7 +144,8 @@ namespace qcore
     // table, the diagonal blocks after the last other block become the product of their
     // diagonals over the tile indices (FP64 products rounded to FP32): a stage of diagonal
     // blocks only then runs as that table alone, another applies it as its tiles are stored.
-    PreparedStage prepare_stage(const std::vector<ResolvedGate> &gates, const PlannedStage &st, int kq, int m, int n, std::vector<float> &mats, bool x3, bool table = false);
+    // compose: as for prepare_blocks, the table too.
+    PreparedStage prepare_stage(const std::vector<ResolvedGate> &gates, const PlannedStage &st, int kq, int m, int n, std::vector<float> &mats, bool x3, bool table = false, ComposeList *compose = nullptr);
     // Blocks a complex64 stage with tables runs through LDS (as stage128_lds_blocks).
     int stage64_lds_blocks(const std::vector<ResolvedGate> &gates, int kq);
     // The stage's task on `state` as the launch's tiles from tile_begin on (checked).
