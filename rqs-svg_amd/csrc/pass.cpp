@@ -740,9 +740,9 @@ namespace qcore
         }
     } // namespace
 
-    PassPlan plan_passes(const std::vector<PassGate> &gates, int n, int m, int amp_bytes, const std::function<void(const PassPlan &, bool)> &planned)
+    PassPlan plan_passes(const std::vector<PassGate> &gates, int n, int m, int amp_bytes, int low_bits, const std::function<void(const PassPlan &, bool)> &planned)
     {
-        if (n < 1 || n > qsv::kMaxQubits || m < qsv::kPassMinBits || m > qsv::kPassMaxBits || (n < m && m != qsv::kPassMinBits))
+        if (n < 1 || n > qsv::kMaxQubits || m < qsv::kPassMinBits || m > qsv::kPassMaxBits || (n < m && m != qsv::kPassMinBits) || low_bits < (amp_bytes == 16 ? 3 : 4) || low_bits > 4)
             throw std::runtime_error("passes: state or tile size out of range");
         PassPlan P;
         P.m = m;
@@ -763,14 +763,14 @@ namespace qcore
             }
             else
             {
-                // qubits 0..3 (contiguous runs of 16 amplitudes) and m - 4 others: those of the
-                // 2x2s in order, or the run of qubits that takes most
-                const uint64_t low = 15, all = (bit(n) - 1);
-                uint64_t avoid, best = grow(gates, rem.data(), rem.size(), all, low, m - 4, false, avoid);
+                // the low qubits (contiguous runs of amplitudes) and m - low_bits others: those of
+                // the 2x2s in order, or the run of qubits that takes most
+                const uint64_t low = bit(low_bits) - 1, all = (bit(n) - 1);
+                uint64_t avoid, best = grow(gates, rem.data(), rem.size(), all, low, m - low_bits, false, avoid);
                 int best_w = count_take(gates, rem.data(), rem.size(), best, 0);
-                for (int a = 4; a + (m - 4) <= n; ++a)
+                for (int a = low_bits; a + (m - low_bits) <= n; ++a)
                 {
-                    const uint64_t w = low | ((bit(m - 4) - 1) << a);
+                    const uint64_t w = low | ((bit(m - low_bits) - 1) << a);
                     const int c = count_take(gates, rem.data(), rem.size(), w, 0);
                     if (c > best_w)
                         best_w = c, best = w;

@@ -77,7 +77,8 @@ namespace qcore
     // one only if on every shared qubit both act as a control or a phase.  A 2x2's target has
     // to be a tile qubit; controls and phases need not be.  amp_bytes: 16 or 8 (complex64),
     // which decides the low qubits that the first and last round of a sweep keep in the
-    // thread index, so that loads and stores cover whole lines.  planned: called after each
+    // thread index, so that loads and stores cover whole lines.  low_bits: qubits 0 .. low_bits - 1
+    // are in every tile (4, or 3 for complex128: one line of 128 bytes).  planned: called after each
     // pass with the plan so far and whether that is all of it.
-    PassPlan plan_passes(const std::vector<PassGate> &gates, int n, int m, int amp_bytes, const std::function<void(const PassPlan &, bool)> &planned = {});
+    PassPlan plan_passes(const std::vector<PassGate> &gates, int n, int m, int amp_bytes, int low_bits = 4, const std::function<void(const PassPlan &, bool)> &planned = {});
 } // namespace qcore

@@ -657,10 +657,17 @@ namespace qcore
             }
             off += rb + ob;
         };
+        // With 3 low qubits in each tile instead of 4 a tile has room for one more other qubit, but
+        // a pass over a large complex128 state is 3 % slower.  Above 23 qubits the plan with fewer
+        // passes is taken (30 qubits, brick depth 3: 5 passes 33.2 ms, 4 passes 27.5 ms; QFT: 7
+        // either way, 56.2 and 58.0 ms), up to there the one with 3 (20 qubits, 20 layers: 405 and
+        // 372 us; 23 qubits, QAOA: 280 and 246).  Complex64 lines are 16 amplitudes, and its passes
+        // are bound by arithmetic: 25 qubits, 6 layers in 6 or 7 passes, both 1.9 ms.
+        const int low_bits = amp_bytes == 8 ? 4 : 3;
         PassPlan P;
         try
         {
-            P = plan_passes(low, n_, m, amp_bytes, [&](const PassPlan &so_far, bool last) {
+            P = plan_passes(low, n_, m, amp_bytes, low_bits, [&](const PassPlan &so_far, bool last) {
                 if (early && !last && so_far.passes.size() >= 2 * (done + 1))
                     launch(so_far, false);
             });
@@ -669,6 +676,12 @@ namespace qcore
         {
             (void)hipStreamSynchronize(stream_); // copies may be on their way
             throw;
+        }
+        if (n_ > 23 && low_bits == 3)
+        {
+            PassPlan four = plan_passes(low, n_, m, amp_bytes, 4);
+            if (four.passes.size() <= P.passes.size())
+                P = std::move(four);
         }
         // A pass moves the whole state once, so few gates with many controls are cheaper one by
         // one; on states of up to 2^22 amplitudes the launches count, not the bytes.

@@ -251,7 +251,7 @@ int main(int argc, char **argv)
             gates.push_back(g);
         }
         const std::vector<PassGate> low = lowering.finish();
-        const PassPlan P = plan_passes(low, n, m, amp_bytes);
+        const PassPlan P = plan_passes(low, n, m, amp_bytes, amp_bytes == 16 && (mix(seed) & 1) ? 3 : 4);
         std::vector<cd> a(1ull << n);
         for (auto &z : a)
             z = cd(unif(seed) - 0.5, unif(seed) - 0.5);
