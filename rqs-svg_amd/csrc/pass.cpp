@@ -740,7 +740,81 @@ namespace qcore
         }
     } // namespace
 
-    PassPlan plan_passes(const std::vector<PassGate> &gates, int n, int m, int amp_bytes, int low_bits, const std::function<void(const PassPlan &, bool)> &planned)
+    namespace
+    {
+        // a target set filled up to a tile of m qubits with the lowest others
+        uint64_t fill_tile(uint64_t set, int n, int m)
+        {
+            for (int q = 0; q < n && __builtin_popcountll(set) < m; ++q)
+                set |= bit(q);
+            return set;
+        }
+    } // namespace
+
+    std::vector<uint64_t> search_tiles(const std::vector<PassGate> &gates, int n, int m, int low_least, int low_most, int width, int count)
+    {
+        struct Kept
+        {
+            std::vector<int> rem;
+            std::vector<uint64_t> tiles;
+            long left = 0; // weight of rem
+        };
+        std::vector<Kept> kept(1), next;
+        if (n <= m || width < 1 || count < 1 || low_least < 3 || low_most > 4)
+            return {};
+        for (size_t i = 0; i < gates.size(); ++i)
+            kept[0].rem.push_back(int(i));
+        std::vector<int> taken;
+        std::vector<std::pair<int, uint64_t>> tries;
+        while (!gates.empty())
+        {
+            next.clear();
+            for (const Kept &k : kept)
+            {
+                tries.clear();
+                auto add = [&](uint64_t set) {
+                    set = fill_tile(set, n, m);
+                    if (std::none_of(tries.begin(), tries.end(), [&](auto &t) { return t.second == set; }))
+                        tries.push_back({count_take(gates, k.rem.data(), k.rem.size(), set, 0), set});
+                };
+                for (int low_bits = low_least; low_bits <= low_most; ++low_bits)
+                {
+                    const uint64_t low = bit(low_bits) - 1;
+                    uint64_t avoid;
+                    add(grow(gates, k.rem.data(), k.rem.size(), bit(n) - 1, low, m - low_bits, false, avoid));
+                    for (int a = low_bits; a + (m - low_bits) <= n; ++a)
+                        add(low | ((bit(m - low_bits) - 1) << a));
+                }
+                std::stable_sort(tries.begin(), tries.end(), [](auto &a, auto &b) { return a.first > b.first; });
+                for (size_t t = 0; t < tries.size() && t < size_t(count); ++t)
+                {
+                    Kept x{k.rem, k.tiles, 0};
+                    taken.clear();
+                    take(gates, x.rem, tries[t].second, 0, taken);
+                    if (taken.empty())
+                        continue;
+                    put_back_phases(gates, taken, x.rem);
+                    x.tiles.push_back(tries[t].second);
+                    if (x.rem.empty())
+                        return x.tiles;
+                    for (int gi : x.rem)
+                        x.left += weight(gates[gi]);
+                    // one of those that leave as much: mostly the same tiles in another order
+                    if (std::none_of(next.begin(), next.end(), [&](auto &o) { return o.left == x.left && o.rem.size() == x.rem.size(); }))
+                        next.push_back(std::move(x));
+                }
+            }
+            if (next.empty())
+                return {};
+            std::stable_sort(next.begin(), next.end(), [](auto &a, auto &b) { return a.left < b.left; });
+            if (next.size() > size_t(width))
+                next.resize(size_t(width));
+            kept.swap(next);
+        }
+        return {};
+    }
+
+    PassPlan plan_passes(const std::vector<PassGate> &gates, int n, int m, int amp_bytes, int low_bits, const std::function<void(const PassPlan &, bool)> &planned, const std::vector<uint64_t> &tiles)
     {
         if (n < 1 || n > qsv::kMaxQubits || m < qsv::kPassMinBits || m > qsv::kPassMaxBits || (n < m && m != qsv::kPassMinBits) || low_bits < (amp_bytes == 16 ? 3 : 4) || low_bits > 4)
             throw std::runtime_error("passes: state or tile size out of range");
@@ -766,17 +840,19 @@ namespace qcore
                 // the low qubits (contiguous runs of amplitudes) and m - low_bits others: those of
                 // the 2x2s in order, or the run of qubits that takes most
                 const uint64_t low = bit(low_bits) - 1, all = (bit(n) - 1);
-                uint64_t avoid, best = grow(gates, rem.data(), rem.size(), all, low, m - low_bits, false, avoid);
-                int best_w = count_take(gates, rem.data(), rem.size(), best, 0);
-                for (int a = low_bits; a + (m - low_bits) <= n; ++a)
+                uint64_t avoid, best = P.passes.size() < tiles.size() ? tiles[P.passes.size()] : grow(gates, rem.data(), rem.size(), all, low, m - low_bits, false, avoid);
+                if (tiles.empty())
                 {
-                    const uint64_t w = low | ((bit(m - low_bits) - 1) << a);
-                    const int c = count_take(gates, rem.data(), rem.size(), w, 0);
-                    if (c > best_w)
-                        best_w = c, best = w;
+                    int best_w = count_take(gates, rem.data(), rem.size(), best, 0);
+                    for (int a = low_bits; a + (m - low_bits) <= n; ++a)
+                    {
+                        const uint64_t w = low | ((bit(m - low_bits) - 1) << a);
+                        const int c = count_take(gates, rem.data(), rem.size(), w, 0);
+                        if (c > best_w)
+                            best_w = c, best = w;
+                    }
+                    best = fill_tile(best, n, m);
                 }
-                for (int q = 0; q < n && __builtin_popcountll(best) < m; ++q)
-                    best |= bit(q);
                 int b = 0;
                 for (int q = 0; q < n; ++q)
                     if ((best >> q) & 1)

@@ -80,5 +80,9 @@ namespace qcore
     // thread index, so that loads and stores cover whole lines.  low_bits: qubits 0 .. low_bits - 1
     // are in every tile (4, or 3 for complex128: one line of 128 bytes).  planned: called after each
     // pass with the plan so far and whether that is all of it.
-    PassPlan plan_passes(const std::vector<PassGate> &gates, int n, int m, int amp_bytes, int low_bits = 4, const std::function<void(const PassPlan &, bool)> &planned = {});
+    PassPlan plan_passes(const std::vector<PassGate> &gates, int n, int m, int amp_bytes, int low_bits = 4, const std::function<void(const PassPlan &, bool)> &planned = {}, const std::vector<uint64_t> &tiles = {});
+    // Tiles (masks of m qubits) of a plan of few passes, for plan_passes: after each of the
+    // `width` sequences kept, the `count` tiles that take most are tried (with the low_least to
+    // low_most low qubits), and the sequences kept that leave least.  Empty if none is found.
+    std::vector<uint64_t> search_tiles(const std::vector<PassGate> &gates, int n, int m, int low_least, int low_most, int width, int count);
 } // namespace qcore

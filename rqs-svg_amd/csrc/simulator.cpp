@@ -607,12 +607,36 @@ namespace qcore
         if (low.empty())
             return 0;
         static_assert(sizeof(qsv::PassRound) % 16 == 0 && sizeof(qsv::PassOp) % 16 == 0, "pass program alignment");
+        // With 3 low qubits in each tile instead of 4 a tile has room for one more other qubit, but
+        // a pass over a large complex128 state is 3 % slower.  Up to 23 qubits the tiles have 3 (20
+        // qubits, 20 layers: 405 and 372 us; 23 qubits, QAOA: 280 and 246); above, the plan with 4
+        // is taken unless one with 3 has fewer passes (30 qubits, brick depth 3: 5 passes 33.2 ms,
+        // 4 passes 27.5 ms; QFT: 7 either way, 56.2 and 58.0 ms), and from 28 qubits on, where a
+        // pass takes longer than the search (0.2 to 1 ms), more sequences of tiles are tried (30
+        // qubits, 4 RY/RZ/CNOT layers: 6 passes 54.2 ms, 4 passes 42.3 ms; brick depth 24: 15 and
+        // 13, 179 and 162 ms; 28 qubits, two-qubit gates: 6 and 5, 10.2 and 8.8 ms).
+        // Complex64 lines are 16 amplitudes, and its passes are bound by arithmetic: 25 qubits, 6
+        // layers in 6 or 7 passes, both 1.9 ms.
+        const int low_bits = amp_bytes == 8 ? 4 : 3;
+        std::vector<uint64_t> tiles; // above 22 qubits
+        if (n_ > 22)
+        {
+            tiles = n_ >= 28 && low_bits == 3 ? search_tiles(low, n_, m, 3, 4, n_ >= 30 ? 8 : 4, 6) : search_tiles(low, n_, m, low_bits, low_bits, 1, 1);
+            if (n_ > 23 && low_bits == 3)
+            {
+                std::vector<uint64_t> four = search_tiles(low, n_, m, 4, 4, 1, 1);
+                if (!four.empty() && (tiles.empty() || four.size() <= tiles.size()))
+                    tiles = std::move(four);
+            }
+            // A pass moves the whole state once, so few gates with many controls are cheaper one
+            // by one; on smaller states the launches count, not the bytes.
+            if (bytes < double(tiles.size()))
+                return -1;
+        }
         // Passes are copied and launched in groups as they are planned, the first of 2 and each of
         // two more than all before it, so that they run while others are planned and there are
-        // few copies (20 qubits, 20 layers in 13 passes: 905 -> 761 us a
-        // call; 13 qubits, 6 layers: 222 -> 200).  Above 22 qubits planning is short beside the passes, and
-        // their number has to be known (below).
-        const bool early = n_ <= 22;
+        // few copies (20 qubits, 20 layers in 13 passes: 905 -> 761 us a call; 13 qubits, 6 layers:
+        // 222 -> 200).
         char *host = nullptr, *dev = nullptr;
         size_t cap = 0, off = 0;
         auto area = [&](size_t want) {
@@ -633,7 +657,7 @@ namespace qcore
             {
                 if (off > 0) // the groups before are still in it
                     qsv::check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
-                area(early ? std::max(rb + ob + pad, 2 * low.size() * sizeof(qsv::PassOp)) : rb + ob + pad);
+                area(std::max(rb + ob + pad, 2 * low.size() * sizeof(qsv::PassOp)));
             }
             auto *rounds = reinterpret_cast<qsv::PassRound *>(host + off);
             std::memcpy(rounds, &P.rounds[first_round], rb);
@@ -657,36 +681,22 @@ namespace qcore
             }
             off += rb + ob;
         };
-        // With 3 low qubits in each tile instead of 4 a tile has room for one more other qubit, but
-        // a pass over a large complex128 state is 3 % slower.  Above 23 qubits the plan with fewer
-        // passes is taken (30 qubits, brick depth 3: 5 passes 33.2 ms, 4 passes 27.5 ms; QFT: 7
-        // either way, 56.2 and 58.0 ms), up to there the one with 3 (20 qubits, 20 layers: 405 and
-        // 372 us; 23 qubits, QAOA: 280 and 246).  Complex64 lines are 16 amplitudes, and its passes
-        // are bound by arithmetic: 25 qubits, 6 layers in 6 or 7 passes, both 1.9 ms.
-        const int low_bits = amp_bytes == 8 ? 4 : 3;
         PassPlan P;
         try
         {
-            P = plan_passes(low, n_, m, amp_bytes, low_bits, [&](const PassPlan &so_far, bool last) {
-                if (early && !last && so_far.passes.size() >= 2 * (done + 1))
-                    launch(so_far, false);
-            });
+            P = plan_passes(
+                low, n_, m, amp_bytes, low_bits,
+                [&](const PassPlan &so_far, bool last) {
+                    if (!last && so_far.passes.size() >= 2 * (done + 1))
+                        launch(so_far, false);
+                },
+                tiles);
         }
         catch (...)
         {
             (void)hipStreamSynchronize(stream_); // copies may be on their way
             throw;
         }
-        if (n_ > 23 && low_bits == 3)
-        {
-            PassPlan four = plan_passes(low, n_, m, amp_bytes, 4);
-            if (four.passes.size() <= P.passes.size())
-                P = std::move(four);
-        }
-        // A pass moves the whole state once, so few gates with many controls are cheaper one by
-        // one; on states of up to 2^22 amplitudes the launches count, not the bytes.
-        if (!early && bytes < double(P.passes.size()))
-            return -1;
         launch(P, true);
         return int(P.passes.size());
     }

@@ -251,7 +251,11 @@ int main(int argc, char **argv)
             gates.push_back(g);
         }
         const std::vector<PassGate> low = lowering.finish();
-        const PassPlan P = plan_passes(low, n, m, amp_bytes, amp_bytes == 16 && (mix(seed) & 1) ? 3 : 4);
+        const int low_bits = amp_bytes == 16 && (mix(seed) & 1) ? 3 : 4;
+        const std::vector<uint64_t> tiles = mix(seed) & 1 ? search_tiles(low, n, m, low_bits, 4, 1 + int(mix(seed) % 4), 1 + int(mix(seed) % 6)) : std::vector<uint64_t>();
+        const PassPlan P = plan_passes(low, n, m, amp_bytes, low_bits, {}, tiles);
+        if (!tiles.empty() && P.passes.size() != tiles.size())
+            fail("the plan does not follow its tiles", c);
         std::vector<cd> a(1ull << n);
         for (auto &z : a)
             z = cd(unif(seed) - 0.5, unif(seed) - 0.5);
