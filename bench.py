@@ -495,8 +495,9 @@ def planner_leg(n, depth, record_count, k=4, fixed_sweep=False):
     blocks and stages at 26-32 qubits, and every candidate stage plan's launches on
     training circuits at 26-30 qubits, none of them the evaluated circuits), then an n-qubit
     QFT on the state of one random brick layer and an n-qubit brick circuit of the given
-    depth, each run three ways -- the greedy fusion fallback (one sweep per block), the
-    default stage plan, and the plan the model picks (taken only when its predicted gain
+    depth, each run four ways -- the greedy fusion fallback (one sweep per block), the
+    stage plan that a model is compared with, circuit passes (the default without a model), and
+    the plan the model picks (taken only when its predicted gain
     over the default exceeds the model's error; one run each, so an override runs as the
     model picked it, before the planner's measured check has compared it with the default)
     -- and each output compared with the plain complex128 method on a second state in HBM."""
@@ -529,10 +530,12 @@ def planner_leg(n, depth, record_count, k=4, fixed_sweep=False):
             plain.run(circ)
             plain.norm()
             res["plain_per_gate_s"] = time.perf_counter() - t0
-            for mode in ("greedy", "stages", "learned"):
+            for mode in ("greedy", "stages", "passes", "learned"):
                 pyqcs.set_planner(fused, model if mode == "learned" else None)
                 if mode == "greedy":
                     fused.set_plan(0, k, window=64, rule=0)
+                elif mode == "stages":
+                    fused.set_plan(12, min(k, 3), tiles=2)
                 else:
                     fused.set_plan(None)
                 _, b0 = fused.fusion_stats()
@@ -550,7 +553,7 @@ def planner_leg(n, depth, record_count, k=4, fixed_sweep=False):
                     res["learned_choices"] = st1["learned_choices"] - st0["learned_choices"]
                     res["flushes"] = st1["flushes"] - st0["flushes"]
                     res["learned_plan"] = list(pyqcs.planner_last_choice(fused))
-                log(f"planner leg: {name} {mode}: {dt:.3f}s, {b1 - b0} sweeps, fidelity vs per-gate "
+                log(f"planner leg: {name} {mode}: {dt:.3f}s, {b1 - b0} sweeps, fidelity vs plain "
                     f"{fid:.15f}, max|d| {maxdiff:.2e}")
             pyqcs.set_planner(fused, None)
             if fixed_sweep:
@@ -569,7 +572,7 @@ def planner_leg(n, depth, record_count, k=4, fixed_sweep=False):
             res["learned_vs_greedy"] = res["greedy_s"] / res["learned_s"]
             res["stages_vs_greedy"] = res["greedy_s"] / res["stages_s"]
             log(f"planner leg: {name}: learned vs default stages {res['learned_vs_stages']:.3f}x, "
-                f"vs greedy {res['learned_vs_greedy']:.2f}x; plain per-gate {res['plain_per_gate_s']:.2f}s")
+                f"vs greedy {res['learned_vs_greedy']:.2f}x; plain {res['plain_per_gate_s']:.2f}s")
             out[name] = res
     finally:
         pyqcs.set_planner(fused, None)
