@@ -27,7 +27,6 @@
 #include <memory>
 #include <mutex>
 #include <stdexcept>
-#include <system_error>
 #include <thread>
 
 namespace qcore
@@ -67,12 +66,13 @@ namespace qcore
             };
             const size_t threads = std::min<size_t>({size_t(16), std::max(1u, std::thread::hardware_concurrency()), count / 8});
             std::vector<std::thread> pool;
+            pool.reserve(threads);
             try
             {
                 for (size_t t = 1; t < threads; ++t)
                     pool.emplace_back(work);
             }
-            catch (const std::system_error &)
+            catch (const std::exception &)
             { // fewer threads, then
             }
             work();
@@ -486,6 +486,8 @@ namespace qcore
             L.offset = put(L.tasks.data(), L.tasks.size() * sizeof(qsv::PassTask));
         const size_t pz_off = put(pz.data(), pz.size() * sizeof(qsv::PassZ));
         const uint32_t pz_count = uint32_t(pz.size());
+        if (!pops.empty()) // one small circuit's task and entries are less than the padding
+            prog.resize(std::max(prog.size(), pops_off + (pops.size() + qsv::kPassOpPad) * sizeof(qsv::PassOp)));
         upload(&d_prog_, prog.data(), prog.size());
         // states within the 256 MB memory-side cache keep cached accesses
         const bool pass_nt = state_total * sizeof(qsv::c64) > (uint64_t(256) << 20);
