@@ -26,8 +26,8 @@
 #include <cstring>
 #include <functional>
 #include <mutex>
+#include <new>
 #include <stdexcept>
-#include <system_error>
 #include <thread>
 
 #include <qcs_ext.h>
@@ -582,8 +582,11 @@ namespace qcore
         size_t cap = kSmallProgram;
         while (cap < bytes)
             cap *= 2;
-        qsv::check(hipMalloc(&prog_dev_, cap), "hipMalloc pass program");
-        qsv::check(hipHostMalloc(&prog_host_, cap, hipHostMallocDefault), "hipHostMalloc pass program");
+        if (hipMalloc(&prog_dev_, cap) != hipSuccess || hipHostMalloc(&prog_host_, cap, hipHostMallocDefault) != hipSuccess)
+        {
+            (void)hipGetLastError();
+            throw std::bad_alloc();
+        }
         prog_cap_ = cap;
     }
 
@@ -691,13 +694,20 @@ namespace qcore
                         launch(so_far, false);
                 },
                 tiles);
+            launch(P, true);
+        }
+        catch (const std::bad_alloc &)
+        {
+            (void)hipStreamSynchronize(stream_); // copies may be on their way
+            if (done > 0)
+                throw;
+            return -1; // nothing is launched, and gate by gate no memory is needed
         }
         catch (...)
         {
-            (void)hipStreamSynchronize(stream_); // copies may be on their way
+            (void)hipStreamSynchronize(stream_);
             throw;
         }
-        launch(P, true);
         return int(P.passes.size());
     }
 
@@ -949,12 +959,13 @@ namespace qcore
             CopyCrew(size_t count, std::function<void(size_t)> copy) : count_(count), done_(count, 0), copy_(std::move(copy))
             {
                 const size_t threads = count < 4 ? 0 : std::min<size_t>({size_t(8), std::max(1u, std::thread::hardware_concurrency()), count / 2});
+                pool_.reserve(threads);
                 try
                 {
                     for (size_t t = 0; t < threads; ++t)
                         pool_.emplace_back([this] { work(); });
                 }
-                catch (const std::system_error &)
+                catch (const std::exception &)
                 { // fewer threads, then: done() copies too
                 }
             }
