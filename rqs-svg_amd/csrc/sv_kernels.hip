@@ -788,9 +788,10 @@ namespace qsv
             }
         }
 
-        // Collapse on a qubit whose runs are shorter than a line (2^tq amplitudes of S bytes,
-        // fewer than 128 B): every amplitude is read and written, zeroed or scaled by its bit,
-        // so that all accesses cover whole lines.  sub: operands of line bits and above.
+        // Collapse on a qubit whose runs (2^tq amplitudes of S bytes) are shorter than a line, or
+        // than half of one without a rescale: every amplitude is read and written, zeroed or
+        // scaled by its bit, so that all accesses cover whole lines.  sub: operands of line bits
+        // and above.
         template <class A>
         __global__ __launch_bounds__(kBlock) void k_collapse_lines(A *__restrict__ s, uint64_t count, Subspace sub, int tq, int result, double scale)
         {
@@ -1812,13 +1813,19 @@ namespace qsv
     {
         if (tq < 0 || tq >= n || n < 1)
             throw std::runtime_error("collapse: qubit out of range");
-        // Everything off the fixed qubits' values is zero and stays so.  Fixed qubits below a
-        // line's bits do not narrow the lines to touch: they are left out, and whole lines with
-        // their zeros are rewritten.
+        // Everything off the fixed qubits' values is zero and stays so.  Fixed qubits inside the
+        // unit of memory to touch do not narrow it: they are left out, and its zeros are
+        // rewritten.  Where amplitudes are read as well that unit is a line of 128 B, where they
+        // are only zeroed half of one.  27 qubits, complex128 (complex64): the qubit that tells a
+        // line's halves apart, 2 (3), zeroed by halves 252 us (97), by whole lines 770 (333); 32-B
+        // runs take 835 (402) against 770 (334), and halves with a rescale 980 (403) against 755
+        // (328).  Qubits 3 and 4 after those below: 204 and 104 us by lines, 156 and 78 by halves.
         const int line_bits = sizeof(A) == 16 ? 3 : 4;
+        const bool rescale = scale != 1.0;
+        const bool lines = tq < (rescale ? line_bits : line_bits - 1) && n >= 8; // handled inside the lines
+        const int unit_bits = lines || rescale ? line_bits : line_bits - 1;
         Subspace sub{};
-        bool have_tq = tq < line_bits && n >= 8; // handled inside the lines
-        const bool lines = have_tq;
+        bool have_tq = lines;
         for (int i = 0; i <= nfixed; ++i)
         {
             const int q = i < nfixed ? fixed[i] : n;
@@ -1829,7 +1836,7 @@ namespace qsv
                 sub.ops[sub.nops++] = tq;
                 have_tq = true;
             }
-            if (q < line_bits || q == n)
+            if (q < unit_bits || q == n)
                 continue;
             sub.ops[sub.nops++] = q;
             sub.set_bits |= fixed_ones & (uint64_t(1) << q);
@@ -1838,7 +1845,7 @@ namespace qsv
         if (lines)
             hipLaunchKernelGGL(k_collapse_lines<A>, dim3(grid_for(count, kBlock * 4)), dim3(kBlock), 0, s, state, count, sub, tq, result, scale);
         else
-            hipLaunchKernelGGL(k_collapse<A>, dim3(grid_for(count, kBlock)), dim3(kBlock), 0, s, state, count, sub, tq, result, scale, scale != 1.0 ? 1 : 0);
+            hipLaunchKernelGGL(k_collapse<A>, dim3(grid_for(count, kBlock)), dim3(kBlock), 0, s, state, count, sub, tq, result, scale, rescale ? 1 : 0);
         after_launch("collapse kernel");
     }
 

@@ -53,6 +53,26 @@ def test_measurement_sequences(gpu, oracle, n, precision):
             assert unit or abs(g[4] - o[4]) <= tol * max(1.0, o[4])
 
 
+# The qubits inside a line of 128 B and around half of it, before, between and after others that
+# narrow the collapse, with and without the rescale.
+@pytest.mark.parametrize("n", [7, 8, 10])
+@pytest.mark.parametrize("renormalize", [False, True])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_collapse_within_lines(gpu, oracle, n, renormalize, precision):
+    tol = 1e-13 if precision == 0 else 1e-6  # as above
+    for order in ((0, 1, 2, 3, 4, 5), (4, 3, 2, 1, 0), (2, 5, 3, 0, 4), (3, 1, 2, 6)):
+        res = []
+        for lib, prec in ((gpu, precision), (oracle, 0)):
+            with pyqcs.Simulator(lib, n, seed=11, precision=prec, num_clbits=n) as sim:
+                sim.set_renormalize(renormalize)
+                sim.set_statevector(random_state(n, n + 1))
+                for q in order:
+                    res.append((sim.measure_to_clbit(q, q), sim.statevector()))
+        for (r, a), (s, b) in zip(res[:len(order)], res[len(order):]):
+            assert r == s and np.array_equal(a == 0, b == 0)
+            assert np.max(np.abs(a - b)) <= tol * max(1.0, np.max(np.abs(b)))
+
+
 # Whole and partial blocks of 64 at the top level, one level and several; more shots than are
 # fetched at a time; a state whose zeros make long runs of equal prefixes.  Outcomes are integers
 # from FP64 sums in a fixed order: exactly the oracle's.
