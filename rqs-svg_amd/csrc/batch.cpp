@@ -380,6 +380,10 @@ namespace qcore
         std::vector<PassLaunch> plaunch{{10}, {11}, {12}};
         size_t large_passed = 0;
         uint64_t sums_total = 0;
+        // Circuits of one tile write their <Z> themselves where the batch has no others; with larger
+        // ones there is a launch that adds up tiles' sums, and it does theirs too.  (12 circuits of
+        // 7-9 qubits: 64.5 -> 62.4 us; 24 of 4-10: 28.4 -> 26.8.)
+        const bool one_launch = passed.size() == circuits_.size() && std::all_of(passed.begin(), passed.end(), [&](const Passed &p) { return circuits_[p.ci].n <= p.plan.m; });
         std::vector<uint64_t> pass_state; // per passed circuit
         std::vector<size_t> pass_sums;
         for (const auto &pc : passed)
@@ -438,7 +442,7 @@ namespace qcore
                 PassLaunch &L = plaunch[li];
                 qsv::PassTask t{};
                 t.state = n > m ? d_states_ + pass_state[i] : nullptr;
-                t.sums = d_sums_ + pass_sums[i];
+                t.sums = one_launch ? d_out_ + C.out_offset : d_sums_ + pass_sums[i];
                 t.tile_begin = L.tiles;
                 t.first_round = first_round + ps.first_round;
                 t.nrounds = ps.nrounds;
@@ -452,9 +456,9 @@ namespace qcore
                     t.flags |= qsv::kPassZeroState;
                 if (p + 1 == P.passes.size())
                 {
-                    t.flags |= qsv::kPassExpectZ;
+                    t.flags |= qsv::kPassExpectZ | (one_launch ? uint32_t(n) << qsv::kPassQubits : 0);
                     uint32_t outside = 0; // qubits below q that are not tile qubits
-                    for (int q = 0; q < n; ++q)
+                    for (int q = 0; q < n && !one_launch; ++q)
                     {
                         const int b = bit_of(q);
                         qsv::PassZ z{};
@@ -582,7 +586,7 @@ namespace qcore
         }
         for (const auto &L : plaunch)
             launches_ += L.tasks.empty() ? 0 : 1;
-        launches_ += passed.empty() ? 0 : 1;
+        launches_ += pz.empty() ? 0 : 1;
         int grid = 0;
         if (!small.empty())
         {

@@ -464,9 +464,10 @@ namespace qsv
         // Sum of the tile's probabilities (out[0]) and, per tile bit b, the sum over the half with
         // the bit 0 less the one with it 1 (out[1 + b]): 4 register bits, 6 lane bits (each
         // step of the wave's butterfly yields its bit's difference), then the waves through LDS.
-        // zb: the tile bit of each register bit and thread bit.
+        // zb: the tile bit of each register bit and thread bit.  qubits > 0: only the differences of
+        // that many tile bits, from out[0] on.
         template <int M>
-        __device__ __forceinline__ void tile_z(const Amps &a, double *x, const uint8_t *zb, double *out)
+        __device__ __forceinline__ void tile_z(const Amps &a, double *x, const uint8_t *zb, double *out, uint32_t qubits)
         {
             constexpr int W = 1 << (M - 10); // waves
             double v[11];
@@ -514,7 +515,11 @@ namespace qsv
                     const double y = x[11 * w + (j < 11 ? j : 0)];
                     sum += j >= 11 && ((w >> (j - 11)) & 1) ? -y : y;
                 }
-                out[j == 0 ? 0 : 1 + zb[j - 1]] = sum;
+                const uint32_t b = j == 0 ? 0 : zb[j - 1];
+                if (qubits == 0)
+                    out[j == 0 ? 0 : 1 + b] = sum;
+                else if (j > 0 && b < qubits)
+                    out[b] = sum;
             }
         }
 
@@ -544,7 +549,7 @@ namespace qsv
             run_rounds<M>(a, at, x, tile_base<M>(t, [&](int b) { return (T.tq[b >> 2] >> (8 * (b & 3))) & 255u; }), rounds + T.first_round, int(T.nrounds), ops,
                           [&](uint64_t i) { return flags & kPassZeroState ? v2d{i == 0 ? 1.0 : 0.0, 0.0} : pload<NT>(s + i); });
             if (flags & kPassExpectZ)
-                tile_z<M>(a, x, reinterpret_cast<const uint8_t *>(tasks_[lo].zb), T.sums + uint64_t(t) * kPassSums);
+                tile_z<M>(a, x, reinterpret_cast<const uint8_t *>(tasks_[lo].zb), T.sums + uint64_t(t) * kPassSums, flags >> kPassQubits);
             else
 #pragma unroll
                 for (int r = 0; r < 16; ++r)

@@ -70,8 +70,9 @@ namespace qsv
     // tile_begin .. of the launch.  The first pass may start from |0...0> without reading, the
     // last one write its tiles' sums (kPassSums doubles each: all probabilities, then per
     // tile bit those with the bit 0 less those with it 1) in place of the amplitudes.  A circuit
-    // smaller than the tile does both (its amplitudes past 2^n stay zero).
-    constexpr uint32_t kPassZeroState = 1, kPassExpectZ = 2;
+    // of one tile does both (its amplitudes past 2^n stay zero), and its differences are its <Z>:
+    // with its qubit count in flags from kPassQubits on, sums is where they go, qubit 0 first.
+    constexpr uint32_t kPassZeroState = 1, kPassExpectZ = 2, kPassQubits = 8;
     constexpr int kPassSums = 16;
     struct alignas(16) PassTask
     {
