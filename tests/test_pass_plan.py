@@ -15,7 +15,7 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 
 @pytest.fixture(scope="module")
-def checker(tmp_path_factory):
+def pass_check(tmp_path_factory):
     if not LIB.exists():
         pytest.skip("libqcs.so not built")
     if not shutil.which(HIPCC) and not os.path.exists(HIPCC):
@@ -28,7 +28,7 @@ def checker(tmp_path_factory):
 
 
 @pytest.mark.parametrize("seed", [1, 2, 3])
-def test_pass_programs_match_the_gates(checker, seed):
-    p = subprocess.run([str(checker), "48", str(seed)], capture_output=True, text=True, timeout=300)
+def test_pass_programs_match_the_gates(pass_check, seed):
+    p = subprocess.run([str(pass_check), "48", str(seed)], capture_output=True, text=True, timeout=300)
     assert p.returncode == 0, p.stdout[-2000:] + p.stderr[-2000:]
     assert p.stdout.strip().endswith("ok")
