@@ -172,6 +172,9 @@ namespace qcore
     void Simulator::reinitialize_mapping()
     { // src/qcs.cu:1860-1885
         state_changed();
+        // the data stays where it is, so the measured qubits' zeros are not at their new places
+        if (!m0_.empty() || !m1_.empty())
+            consistent_ = false;
         p2l_.assign(n_, 0);
         l2p_.assign(n_, 0);
         if (initial_p2l.empty())
