@@ -1100,6 +1100,7 @@ namespace qcore
         if (fused_)
             fused_->drop();
         ensure_stage();
+        consistent_ = m0_.empty() && m1_.empty(); // a failure on the way leaves part of the new state
         const uint64_t len = std::min(count, kSlotLen), slots = count / len;
         auto slot = [&](uint64_t i) { return stage_ + (i % kSlots) * kSlotLen; };
         qsv::check(hipStreamSynchronize(stream_), "sync"); // no earlier work reads the slots
@@ -1161,6 +1162,7 @@ namespace qcore
             if (fused_)
                 fused_->drop();
             ensure_stage();
+            consistent_ = m0_.empty() && m1_.empty(); // as in set_statevector
             const uint64_t chunk = stage_len();
             for (uint64_t first = 0; first < count; first += chunk)
             {
