@@ -475,7 +475,7 @@ namespace qcore
             }
             large_passed += n > m;
         }
-        // rounds, operations, tasks of each launch, <Z> entries (all multiples of 16 bytes)
+        // rounds, padding, operations, tasks of each launch, <Z> entries (all multiples of 16 bytes)
         std::vector<char> prog;
         auto put = [&](const void *src, size_t bytes) {
             const size_t off = prog.size();
@@ -483,8 +483,9 @@ namespace qcore
             return off;
         };
         static_assert(sizeof(qsv::PassRound) % 16 == 0 && sizeof(qsv::PassOp) % 16 == 0 && sizeof(qsv::PassTask) % 16 == 0 && sizeof(qsv::PassZ) % 16 == 0, "pass program alignment");
-        prog.reserve(prounds.size() * sizeof(qsv::PassRound) + pops.size() * sizeof(qsv::PassOp) + pz.size() * sizeof(qsv::PassZ) + (2 * passed.size() + plaunch.size()) * sizeof(qsv::PassTask));
+        prog.reserve(qsv::pass_rounds_bytes(prounds.size()) + pops.size() * sizeof(qsv::PassOp) + pz.size() * sizeof(qsv::PassZ) + (2 * passed.size() + plaunch.size()) * sizeof(qsv::PassTask));
         put(prounds.data(), prounds.size() * sizeof(qsv::PassRound));
+        prog.resize(qsv::pass_rounds_bytes(prounds.size()));
         const size_t pops_off = put(pops.data(), pops.size() * sizeof(qsv::PassOp));
         for (auto &L : plaunch)
             L.offset = put(L.tasks.data(), L.tasks.size() * sizeof(qsv::PassTask));

@@ -382,8 +382,9 @@ namespace qsv
                 const uint32_t first = rounds[0].first, last = rounds[nrounds - 1].first + rounds[nrounds - 1].count;
                 auto touch = [&](const void *p, uint32_t bytes) {
                     uint32_t v = 0;
-                    for (uint32_t b = tid * 128; b < bytes; b += (128u << TB))
-                        v |= *reinterpret_cast<const uint32_t *>(static_cast<const char *>(p) + b);
+                    // one step past the end falls on the last word: p need not begin a line
+                    for (uint32_t b = tid * 128; b < bytes + 124; b += (128u << TB))
+                        v |= *reinterpret_cast<const uint32_t *>(static_cast<const char *>(p) + (b < bytes ? b : bytes - 4));
                     asm volatile("" ::"v"(v));
                 };
                 touch(ops_ + first, (last - first + 1) * uint32_t(sizeof(PassOp)));
@@ -584,6 +585,15 @@ namespace qsv
         }
     } // namespace
 
+    namespace
+    {
+        void check_program(const PassRound *rounds, const PassOp *ops)
+        {
+            if (reinterpret_cast<uintptr_t>(rounds) % alignof(PassRound) || reinterpret_cast<uintptr_t>(ops) % alignof(PassOp))
+                throw std::runtime_error("pass: rounds or operations are not aligned");
+        }
+    } // namespace
+
     template <class A>
     void launch_pass(hipStream_t st, A *state, int n, int m, const uint8_t *tq, const PassRound *rounds, int nrounds, const PassOp *ops)
     {
@@ -591,6 +601,7 @@ namespace qsv
             throw std::runtime_error("pass: state or tile size out of range");
         if (state == nullptr || rounds == nullptr || ops == nullptr || nrounds < 1)
             throw std::runtime_error("pass: no state or no rounds");
+        check_program(rounds, ops);
         PassTile tile{};
         for (int b = 0; b < m; ++b)
         {
@@ -633,6 +644,7 @@ namespace qsv
     {
         if (tasks == nullptr || rounds == nullptr || ops == nullptr || ntasks < 1 || tiles < uint32_t(ntasks))
             throw std::runtime_error("pass: no tasks");
+        check_program(rounds, ops);
         auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(tiles), dim3(1 << (m - 4)), 0, st, tasks, ntasks, rounds, ops); };
         if (m == 10)
             nt ? go(k_pass_tasks<10, true>) : go(k_pass_tasks<10, false>);

@@ -27,7 +27,8 @@ namespace qsv
         kPassKinds = 42,
     };
 
-    // One cache line, read by one scalar load.
+    // Half a line, read by scalar loads of its own 64 bytes: programs place the operations, after
+    // the rounds, on a multiple of that.
     struct alignas(64) PassOp
     {
         uint32_t kind;
@@ -40,13 +41,16 @@ namespace qsv
     // A round: which tile bits are register bits (4) and which the thread-index bits, each
     // with its physical qubit and its LDS byte offset (8 pass_slot); the operations
     // ops[first .. first+count).
-    struct PassRound
+    struct alignas(16) PassRound
     {
         uint32_t rq[4], rl[4];
         uint32_t tq[12], tl[12];
         uint32_t first, count;
         uint32_t pad[2];
     };
+
+    // bytes of `count` rounds with the padding to the operations behind them
+    constexpr size_t pass_rounds_bytes(size_t count) { return (count * sizeof(PassRound) + alignof(PassOp) - 1) / alignof(PassOp) * alignof(PassOp); }
 
     // operations that the kernel may read past a program's last one (it reads ahead)
     constexpr int kPassOpPad = 2;
@@ -59,7 +63,7 @@ namespace qsv
     // One sweep of a 2^n-amplitude state: every tile of 2^m amplitudes (m = kPassMinBits ..
     // kPassMaxBits; tile qubits tq[0..m-1] ascending; for n < m the whole state, tile qubits
     // 0..m-1) goes through the rounds.  rounds and ops are device memory (nrounds rounds, kPassOpPad
-    // operations past the last round's).
+    // operations past the last round's), each aligned as its type.
     template <class A>
     void launch_pass(hipStream_t s, A *state, int n, int m, const uint8_t *tq, const PassRound *rounds, int nrounds, const PassOp *ops);
 

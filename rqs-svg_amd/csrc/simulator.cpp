@@ -612,7 +612,7 @@ namespace qcore
         const std::vector<PassGate> low = lowering.finish();
         if (low.empty())
             return 0;
-        static_assert(sizeof(qsv::PassRound) % 16 == 0 && sizeof(qsv::PassOp) % 16 == 0, "pass program alignment");
+        static_assert((kPinnedResults * sizeof(double)) % alignof(qsv::PassOp) == 0 && (32 * sizeof(double)) % alignof(qsv::PassOp) == 0, "pass program alignment");
         // With 3 low qubits in each tile instead of 4 a tile has room for one more other qubit, but
         // a pass over a large complex128 state is 3 % slower.  Up to 23 qubits the tiles have 3 (20
         // qubits, 20 layers: 405 and 372 us; 23 qubits, QAOA: 280 and 246); above, the plan with 4
@@ -657,7 +657,7 @@ namespace qcore
         auto launch = [&](const PassPlan &P, bool last) {
             const uint32_t first_round = P.passes[done].first_round, first_op = P.rounds[first_round].first;
             const size_t nrounds = P.rounds.size() - first_round, nops = P.rounds.back().first + P.rounds.back().count - first_op;
-            const size_t rb = nrounds * sizeof(qsv::PassRound), ob = nops * sizeof(qsv::PassOp);
+            const size_t rb = qsv::pass_rounds_bytes(nrounds), ob = nops * sizeof(qsv::PassOp);
             const size_t pad = qsv::kPassOpPad * sizeof(qsv::PassOp); // read ahead, not used
             if (off + rb + ob + pad > cap)
             {
@@ -666,7 +666,7 @@ namespace qcore
                 area(std::max(rb + ob + pad, 2 * low.size() * sizeof(qsv::PassOp)));
             }
             auto *rounds = reinterpret_cast<qsv::PassRound *>(host + off);
-            std::memcpy(rounds, &P.rounds[first_round], rb);
+            std::memcpy(rounds, &P.rounds[first_round], nrounds * sizeof(qsv::PassRound));
             for (size_t i = 0; i < nrounds; ++i)
                 rounds[i].first -= first_op;
             std::memcpy(host + off + rb, &P.ops[first_op], ob);
