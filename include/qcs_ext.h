@@ -110,8 +110,9 @@ int qcs_ext_set_local_qubits(qcs_simulator *sim, bit_num_t num_local_qubits);
  * The state afterwards is what the same calls one by one leave, up to FP64 rounding (gates on
  * different qubits may be applied in another order), and all work is queued on the stream on
  * return.  Without measured qubits, complex128 states (precision 0) take runs of gates in
- * passes of several gates per sweep.  *num_applied: gates applied; on failure the gates
- * before the refused one have been. */
+ * passes of several gates per sweep.  *num_applied: gates applied; when a gate is refused
+ * the gates before it have been.  (Should the device itself fail, the state is undefined and
+ * the count is of gates whose passes were all launched.) */
 int qcs_ext_run_circuit(qcs_simulator *sim, int32_t count, const char *const *names, const int32_t *num_params,
                         const uint8_t *name_of, const uint8_t *num_targets, const uint8_t *num_negctrls,
                         const uint8_t *num_ctrls, const bit_num_t *targets, const bit_num_t *negctrls,

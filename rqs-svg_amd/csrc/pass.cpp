@@ -4,6 +4,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <iterator>
 #include <stdexcept>
 
 namespace qcore
@@ -540,6 +541,23 @@ namespace qcore
             rem.swap(merged);
         }
 
+        // Gates of a round: bounds its operations (at most two a gate, and the last flushes), so
+        // that a round always fits the memory that programs pass through.
+        constexpr size_t kRoundGates = (kProgramRoundOps - 2) / 2;
+
+        // Of more gates taken than a round holds, those past its end go back to rem.
+        void put_back_rest(std::vector<int> &taken, std::vector<int> &rem)
+        {
+            if (taken.size() <= kRoundGates)
+                return;
+            std::vector<int> back(taken.begin() + kRoundGates, taken.end()), merged;
+            taken.resize(kRoundGates);
+            std::sort(back.begin(), back.end()); // the circuit's order again
+            merged.reserve(rem.size() + back.size());
+            std::merge(rem.begin(), rem.end(), back.begin(), back.end(), std::back_inserter(merged));
+            rem.swap(merged);
+        }
+
         // Emits one round: register qubits reg[0..3] (ascending tile bits), the gates `taken`.
         void emit_round(PassPlan &P, const std::vector<PassGate> &gates, const uint8_t *tq, int m, uint32_t regbits, const std::vector<int> &taken)
         {
@@ -729,6 +747,7 @@ namespace qcore
                 if (taken.empty())
                     throw std::runtime_error("pass: planning does not advance");
                 put_back_phases(gates, taken, rem);
+                put_back_rest(taken, rem);
                 if (first && (best & low))
                     emit_round(P, gates, tq, m, bits_of(top), {});
                 emit_round(P, gates, tq, m, bits_of(best), taken);
@@ -872,5 +891,40 @@ namespace qcore
         }
         P.ops.resize(P.ops.size() + qsv::kPassOpPad, qsv::PassOp{});
         return P;
+    }
+
+    ProgramPart program_part(const PassPlan &P, uint32_t first, size_t room, bool split)
+    {
+        auto fits = [&](uint32_t end) { return ProgramPart{first, end}.bytes(P) + qsv::kPassOpPad * sizeof(qsv::PassOp) <= room; };
+        ProgramPart part{first, first};
+        for (const auto &ps : P.passes)
+            if (const uint32_t end = ps.first_round + ps.nrounds; end > first)
+            {
+                if (!fits(end))
+                    break;
+                part.end = end;
+            }
+        if (part.end == first && split) // not even one pass: as many of its rounds
+            while (part.end < P.rounds.size() && fits(part.end + 1))
+                ++part.end;
+        return part;
+    }
+
+    size_t ProgramPart::bytes(const PassPlan &P) const
+    {
+        return end == first ? 0 : qsv::pass_rounds_bytes(end - first) + (P.rounds[end - 1].first + P.rounds[end - 1].count - P.rounds[first].first) * sizeof(qsv::PassOp);
+    }
+
+    void ProgramPart::write(const PassPlan &P, char *to) const
+    {
+        const uint32_t first_op = P.rounds[first].first;
+        for (uint32_t r = first; r < end; ++r)
+        {
+            qsv::PassRound R = P.rounds[r];
+            R.first -= first_op;
+            std::memcpy(to + (r - first) * sizeof R, &R, sizeof R);
+        }
+        const size_t at = qsv::pass_rounds_bytes(end - first);
+        std::memcpy(to + at, P.ops.data() + first_op, bytes(P) - at);
     }
 } // namespace qcore

@@ -85,4 +85,18 @@ namespace qcore
     // `width` sequences kept, the `count` tiles that take most are tried (with the low_least to
     // low_most low qubits), and the sequences kept that leave least.  Empty if none is found.
     std::vector<uint64_t> search_tiles(const std::vector<PassGate> &gates, int n, int m, int low_least, int low_most, int width, int count);
+
+    // Programs reach the device in parts: consecutive rounds with their operations, numbered
+    // from the part's first.  Each round carries everything it needs, so a pass may be cut
+    // between two of its rounds into sweeps of their own.
+    struct ProgramPart
+    {
+        uint32_t first, end; // rounds
+        size_t bytes(const PassPlan &P) const;
+        void write(const PassPlan &P, char *to) const;
+    };
+    constexpr size_t kProgramRoundOps = 512; // operations of a round, at most
+    // The rounds of P from `first` on that fit `room` bytes with the padding behind them: whole
+    // passes, or (split) some rounds of one that does not fit; none if there is no room.
+    ProgramPart program_part(const PassPlan &P, uint32_t first, size_t room, bool split);
 } // namespace qcore

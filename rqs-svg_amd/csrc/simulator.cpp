@@ -77,7 +77,7 @@ namespace qcore
     {
         qsv::check(hipGetDevice(&device_), "hipGetDevice");
         qsv::check(hipStreamCreate(&stream_), "hipStreamCreate");
-        qsv::check(hipHostMalloc((void **)&pinned_, kPinnedResults * sizeof(double) + kSmallProgram, hipHostMallocDefault), "hipHostMalloc");
+        qsv::check(hipHostMalloc((void **)&pinned_, kPinnedResults * sizeof(double) + kRing, hipHostMallocDefault), "hipHostMalloc");
         std::random_device rd; // src/qcs.cu:1845-1852
         seed_ = rd();
         engine_.seed(seed_);
@@ -105,8 +105,9 @@ namespace qcore
             (void)hipEventDestroy(e);
         if (open_a_)
             (void)hipEventDestroy(open_a_);
-        if (prog_copied_)
-            (void)hipEventDestroy(prog_copied_);
+        for (auto e : ring_read_)
+            if (e)
+                (void)hipEventDestroy(e);
         if (pinned_)
             (void)hipHostFree(pinned_);
         if (stream_)
@@ -224,9 +225,9 @@ namespace qcore
             fused_->set_check(planner_check_ != 0);
         }
         work_len_ = std::max(qsv::reduce_workspace(count), qsv::expz_workspace(count)) + 16;
-        // the reductions' workspace, and behind it the device copy of a small pass program
+        // the reductions' workspace, and behind it the device's copies of pass programs
         work_len_ = (work_len_ + 31) & ~uint64_t(31);
-        qsv::check(hipMalloc((void **)&work_, work_len_ * sizeof(double) + kSmallProgram), "hipMalloc workspace");
+        qsv::check(hipMalloc((void **)&work_, work_len_ * sizeof(double) + kRing), "hipMalloc workspace");
         allocated_ = true;
         set_zero_state();
     }
@@ -249,12 +250,6 @@ namespace qcore
             (void)hipFree(work_);
             work_ = nullptr;
         }
-        if (prog_dev_)
-            (void)hipFree(prog_dev_);
-        if (prog_host_)
-            (void)hipHostFree(prog_host_);
-        prog_dev_ = prog_host_ = nullptr;
-        prog_cap_ = 0;
         if (shots_)
             (void)hipHostFree(shots_);
         shots_ = nullptr;
@@ -565,32 +560,23 @@ namespace qcore
         }
     }
 
-    void Simulator::reserve_program(size_t bytes)
+    void Simulator::leave_segment(size_t segment)
     {
-        if (!prog_copied_)
-            qsv::check(hipEventCreateWithFlags(&prog_copied_, hipEventDisableTiming), "hipEventCreate");
-        else if (prog_pending_) // the last program's copy still reads the staging area
-            qsv::check(hipEventSynchronize(prog_copied_), "hipEventSynchronize");
-        prog_pending_ = false;
-        if (bytes <= kSmallProgram || bytes <= prog_cap_)
-            return;
-        // queued passes may still read the device copy
-        qsv::check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
-        if (prog_dev_)
-            (void)hipFree(prog_dev_);
-        if (prog_host_)
-            (void)hipHostFree(prog_host_);
-        prog_dev_ = prog_host_ = nullptr;
-        prog_cap_ = 0;
-        size_t cap = kSmallProgram;
-        while (cap < bytes)
-            cap *= 2;
-        if (hipMalloc(&prog_dev_, cap) != hipSuccess || hipHostMalloc(&prog_host_, cap, hipHostMallocDefault) != hipSuccess)
-        {
-            (void)hipGetLastError();
-            throw std::bad_alloc();
-        }
-        prog_cap_ = cap;
+        if (!ring_read_[segment])
+            qsv::check(hipEventCreateWithFlags(&ring_read_[segment], hipEventDisableTiming), "hipEventCreate");
+        qsv::check(hipEventRecord(ring_read_[segment], stream_), "hipEventRecord");
+        ring_pending_[segment] = true;
+    }
+
+    void Simulator::enter_segments(size_t bytes)
+    {
+        // the segments that begin inside the part
+        for (size_t i = (ring_at_ + kSegment - 1) / kSegment; i * kSegment < ring_at_ + bytes; ++i)
+            if (ring_pending_[i])
+            {
+                qsv::check(hipEventSynchronize(ring_read_[i]), "hipEventSynchronize");
+                ring_pending_[i] = false;
+            }
     }
 
     int Simulator::run_passes(const std::vector<ResolvedGate> &gates)
@@ -642,76 +628,70 @@ namespace qcore
         // Passes are copied and launched in groups as they are planned, the first of 2 and each of
         // two more than all before it, so that they run while others are planned and there are
         // few copies (20 qubits, 20 layers in 13 passes: 905 -> 761 us a call; 13 qubits, 6 layers:
-        // 222 -> 200).
-        char *host = nullptr, *dev = nullptr;
-        size_t cap = 0, off = 0;
-        auto area = [&](size_t want) {
-            reserve_program(want);
-            const bool small = want <= kSmallProgram;
-            host = small ? reinterpret_cast<char *>(pinned_ + kPinnedResults) : static_cast<char *>(prog_host_);
-            dev = small ? reinterpret_cast<char *>(work_ + work_len_) : static_cast<char *>(prog_dev_);
-            cap = small ? kSmallProgram : prog_cap_;
-            off = 0;
+        // 222 -> 200).  Nothing is allocated once a pass has been launched, since a run that ends
+        // between its passes is a state that no gates leave: the ring is there before, a group
+        // longer than what is free of it goes in parts, and a pass longer than the ring in several
+        // sweeps.
+        static_assert(kRing >= qsv::pass_rounds_bytes(1) + (kProgramRoundOps + qsv::kPassOpPad) * sizeof(qsv::PassOp), "the ring holds every round");
+        char *const host = reinterpret_cast<char *>(pinned_ + kPinnedResults), *const dev = reinterpret_cast<char *>(work_ + work_len_);
+        uint32_t done = 0; // rounds launched
+        int sweeps = 0;
+        auto launch = [&](const PassPlan &P) {
+            while (done < P.rounds.size())
+            {
+                const ProgramPart part = program_part(P, done, kRing - ring_at_, ring_at_ == 0);
+                if (part.end == done)
+                {
+                    if (ring_at_ == 0)
+                        throw std::runtime_error("pass: a round does not fit the program ring");
+                    if (ring_at_ < kRing)
+                        leave_segment(ring_at_ / kSegment);
+                    ring_at_ = 0;
+                    continue;
+                }
+                const size_t bytes = part.bytes(P), from = ring_at_;
+                enter_segments(bytes);
+                part.write(P, host + from);
+                qsv::launch_program_copy(stream_, dev + from, host + from, bytes);
+                ring_at_ += bytes;
+                for (size_t i = from / kSegment; i < ring_at_ / kSegment; ++i)
+                    leave_segment(i);
+                const auto *rounds = reinterpret_cast<const qsv::PassRound *>(dev + from);
+                const auto *ops = reinterpret_cast<const qsv::PassOp *>(dev + from + qsv::pass_rounds_bytes(part.end - part.first));
+                for (const auto &ps : P.passes)
+                {
+                    const uint32_t a = std::max(ps.first_round, part.first), b = std::min(ps.first_round + ps.nrounds, part.end);
+                    if (a >= b)
+                        continue;
+                    prof_begin(QCS_EXT_K_FUSED, 2.0 * amp_bytes * (1ull << n_));
+                    with_state([&](auto *st) { qsv::launch_pass(stream_, st, n_, m, ps.tq, rounds + (a - part.first), int(b - a), ops); });
+                    prof_end();
+                    ++sweeps;
+                }
+                done = part.end;
+            }
         };
-        size_t done = 0; // passes launched
-        auto launch = [&](const PassPlan &P, bool last) {
-            const uint32_t first_round = P.passes[done].first_round, first_op = P.rounds[first_round].first;
-            const size_t nrounds = P.rounds.size() - first_round, nops = P.rounds.back().first + P.rounds.back().count - first_op;
-            const size_t rb = qsv::pass_rounds_bytes(nrounds), ob = nops * sizeof(qsv::PassOp);
-            const size_t pad = qsv::kPassOpPad * sizeof(qsv::PassOp); // read ahead, not used
-            if (off + rb + ob + pad > cap)
-            {
-                if (off > 0) // the groups before are still in it
-                    qsv::check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
-                area(std::max(rb + ob + pad, 2 * low.size() * sizeof(qsv::PassOp)));
-            }
-            auto *rounds = reinterpret_cast<qsv::PassRound *>(host + off);
-            std::memcpy(rounds, &P.rounds[first_round], nrounds * sizeof(qsv::PassRound));
-            for (size_t i = 0; i < nrounds; ++i)
-                rounds[i].first -= first_op;
-            std::memcpy(host + off + rb, &P.ops[first_op], ob);
-            qsv::launch_program_copy(stream_, dev + off, host + off, rb + ob);
-            if (last)
-            {
-                qsv::check(hipEventRecord(prog_copied_, stream_), "hipEventRecord");
-                prog_pending_ = true;
-            }
-            for (; done < P.passes.size(); ++done)
-            {
-                const auto &ps = P.passes[done];
-                prof_begin(QCS_EXT_K_FUSED, 2.0 * amp_bytes * (1ull << n_));
-                with_state([&](auto *st) {
-                    qsv::launch_pass(stream_, st, n_, m, ps.tq, reinterpret_cast<const qsv::PassRound *>(dev + off) + (ps.first_round - first_round), int(ps.nrounds), reinterpret_cast<const qsv::PassOp *>(dev + off + rb));
-                });
-                prof_end();
-            }
-            off += rb + ob;
-        };
+        size_t launched = 0; // passes
         PassPlan P;
         try
         {
             P = plan_passes(
                 low, n_, m, amp_bytes, low_bits,
                 [&](const PassPlan &so_far, bool last) {
-                    if (!last && so_far.passes.size() >= 2 * (done + 1))
-                        launch(so_far, false);
+                    if (last || so_far.passes.size() < 2 * (launched + 1))
+                        return;
+                    launch(so_far);
+                    launched = so_far.passes.size();
                 },
                 tiles);
-            launch(P, true);
-        }
-        catch (const std::bad_alloc &)
-        {
-            (void)hipStreamSynchronize(stream_); // copies may be on their way
-            if (done > 0)
-                throw;
-            return -1; // nothing is launched, and gate by gate no memory is needed
+            launch(P);
         }
         catch (...)
         {
             (void)hipStreamSynchronize(stream_);
             throw;
         }
-        return int(P.passes.size());
+        return sweeps;
     }
 
     void Simulator::apply_run(const std::vector<ResolvedGate> &gates)

@@ -28,3 +28,8 @@ def check(source, folder, *args):
 
 def test_misaligned_programs_are_refused(tmp_path):
     check("pass_align_check.cpp", tmp_path)
+
+
+@pytest.mark.parametrize("seed", [1, 2])
+def test_programs_in_parts(tmp_path, seed):
+    check("pass_parts_check.cpp", tmp_path, seed)
