@@ -396,9 +396,106 @@ namespace qcore
 
     namespace
     {
-        // Which gates of `rem` (indices, in order) can be applied with 2x2 targets in `targets`
-        // only; `no_control`: qubits that a 2x2 other than a flip may not be controlled by.
-        // Calls take(i) for each; stops once no target is left that a later 2x2 could use.
+        // Gates still to be planned, by index and in order.  They are taken from the front part that
+        // a scan covers: what stays of it moves up to the rest, so that a round costs what it scans
+        // and not what is left of the circuit.
+        class Remaining
+        {
+        public:
+            Remaining() = default;
+            explicit Remaining(const std::vector<PassGate> &gates) : Remaining(gates, all(gates.size())) {}
+            Remaining(const std::vector<PassGate> &gates, std::vector<int> indices) : v_(std::move(indices))
+            {
+                for (int i : v_)
+                    count(gates[i], 1);
+            }
+            const int *data() const { return v_.data() + head_; }
+            size_t size() const { return v_.size() - head_; }
+            bool empty() const { return size() == 0; }
+            // qubits that a remaining 2x2 has as its target; a scan need not wait for others
+            uint64_t targets() const { return targets_; }
+            bool phases_only() const { return targets_ == 0; }
+
+            // Goes through the gates until more(gate) is false; those that ok(gate) chooses are
+            // appended to taken, the others stay.
+            template <class Ok, class More>
+            void take(const std::vector<PassGate> &gates, std::vector<int> &taken, Ok ok, More more)
+            {
+                stay_.clear();
+                size_t i = head_;
+                for (bool go = true; go && i < v_.size(); ++i)
+                {
+                    const PassGate &g = gates[v_[i]];
+                    if (ok(g))
+                    {
+                        taken.push_back(v_[i]);
+                        count(g, -1);
+                    }
+                    else
+                        stay_.push_back(v_[i]);
+                    go = more(g);
+                }
+                head_ = i - stay_.size();
+                std::copy(stay_.begin(), stay_.end(), v_.begin() + long(head_));
+            }
+            // the first ones, phases or not
+            void take_front(const std::vector<PassGate> &gates, std::vector<int> &taken, size_t most)
+            {
+                for (; most > 0 && !empty(); --most, ++head_)
+                {
+                    taken.push_back(*data());
+                    count(gates[*data()], -1);
+                }
+            }
+            // takes gates back in, `back` in order
+            void put_back(const std::vector<PassGate> &gates, const std::vector<int> &back)
+            {
+                for (int i : back)
+                    count(gates[i], 1);
+                if (back.size() > head_)
+                {
+                    std::vector<int> merged;
+                    merged.reserve(size() + back.size());
+                    std::merge(v_.begin() + long(head_), v_.end(), back.begin(), back.end(), std::back_inserter(merged));
+                    v_.swap(merged);
+                    head_ = 0;
+                    return;
+                }
+                size_t to = head_ - back.size(), from = head_;
+                head_ = to;
+                for (int b : back)
+                {
+                    while (from < v_.size() && v_[from] < b)
+                        v_[to++] = v_[from++];
+                    v_[to++] = b;
+                }
+            }
+
+        private:
+            std::vector<int> v_, stay_;
+            size_t head_ = 0;
+            uint64_t targets_ = 0;
+            int left_[64] = {}; // 2x2s by target
+
+            static std::vector<int> all(size_t n)
+            {
+                std::vector<int> v(n);
+                for (size_t i = 0; i < n; ++i)
+                    v[i] = int(i);
+                return v;
+            }
+            void count(const PassGate &g, int by)
+            {
+                if (g.t < 0)
+                    return;
+                left_[g.t] += by;
+                targets_ = left_[g.t] ? targets_ | bit(g.t) : targets_ & ~bit(g.t);
+            }
+        };
+
+        // Which gates of `rem` can be applied with 2x2 targets in `targets` only; `no_control`: qubits
+        // that a 2x2 other than a flip may not be controlled by.  Scans stop once no target is left
+        // that a later 2x2 could use, or `most` gates are taken.
         struct Frontier
         {
             uint64_t x = 0, z = 0; // qubits with a deferred 2x2 target, a deferred control or phase
@@ -425,13 +522,15 @@ namespace qcore
         }
 
         // weight of the 2x2s of rem that a fixed target set takes
-        int count_take(const std::vector<PassGate> &gates, const int *rem, size_t nrem, uint64_t targets, uint64_t no_control)
+        int count_take(const std::vector<PassGate> &gates, const Remaining &rem, uint64_t targets, uint64_t no_control, size_t most = ~size_t(0))
         {
             Frontier f;
             int w = 0;
-            for (size_t i = 0; i < nrem; ++i)
+            const int *at = rem.data();
+            targets &= rem.targets();
+            for (size_t i = 0; i < rem.size(); ++i)
             {
-                const PassGate &g = gates[rem[i]];
+                const PassGate &g = gates[at[i]];
                 const bool ok = f.free(g) && (g.t < 0 || ((targets >> g.t) & 1)) && !(is_dense(g) && (g.cmask & no_control));
                 if (!ok)
                 {
@@ -439,21 +538,27 @@ namespace qcore
                     if (!(targets & ~(f.x | f.z)))
                         break;
                 }
-                else if (g.t >= 0)
-                    w += weight(g);
+                else
+                {
+                    if (g.t >= 0)
+                        w += weight(g);
+                    if (--most == 0)
+                        break;
+                }
             }
             return w;
         }
 
         // a target set of at most `room` more qubits, grown over the gates in order
-        uint64_t grow(const std::vector<PassGate> &gates, const int *rem, size_t nrem, uint64_t allowed, uint64_t start, int room, bool avoid_controls, uint64_t &avoid)
+        uint64_t grow(const std::vector<PassGate> &gates, const Remaining &rem, uint64_t allowed, uint64_t start, int room, bool avoid_controls, uint64_t &avoid, size_t most = ~size_t(0))
         {
             Frontier f;
             uint64_t set = start;
             avoid = 0;
-            for (size_t i = 0; i < nrem; ++i)
+            const int *at = rem.data();
+            for (size_t i = 0; i < rem.size(); ++i)
             {
-                const PassGate &g = gates[rem[i]];
+                const PassGate &g = gates[at[i]];
                 bool ok = f.free(g);
                 if (ok && g.t >= 0)
                 {
@@ -476,50 +581,41 @@ namespace qcore
                 if (!ok)
                 {
                     f.defer(g);
-                    if (room == 0 && !(set & ~(f.x | f.z)))
+                    if (!((room > 0 ? set | (allowed & ~avoid) : set) & rem.targets() & ~(f.x | f.z)))
                         break;
                 }
+                else if (--most == 0)
+                    break;
             }
             return set;
         }
 
         // moves the gates that the target set takes from rem to taken
-        void take(const std::vector<PassGate> &gates, std::vector<int> &rem, uint64_t targets, uint64_t no_control, std::vector<int> &taken)
+        void take(const std::vector<PassGate> &gates, Remaining &rem, uint64_t targets, uint64_t no_control, std::vector<int> &taken, size_t most = ~size_t(0))
         {
             Frontier f;
-            size_t keep = 0;
-            for (size_t i = 0; i < rem.size(); ++i)
-            {
-                const int gi = rem[i];
-                const PassGate &g = gates[gi];
-                const bool ok = f.free(g) && (g.t < 0 || ((targets >> g.t) & 1)) && !(is_dense(g) && (g.cmask & no_control));
-                if (ok)
-                {
-                    taken.push_back(gi);
-                    continue;
-                }
-                f.defer(g);
-                rem[keep++] = gi;
-                if (!(targets & ~(f.x | f.z)))
-                { // nothing but phases could follow
-                    std::copy(rem.begin() + i + 1, rem.end(), rem.begin() + keep);
-                    keep += rem.size() - i - 1;
-                    break;
-                }
-            }
-            rem.resize(keep);
+            targets &= rem.targets();
+            rem.take(
+                gates, taken,
+                [&](const PassGate &g) {
+                    const bool ok = f.free(g) && (g.t < 0 || ((targets >> g.t) & 1)) && !(is_dense(g) && (g.cmask & no_control));
+                    if (!ok)
+                        f.defer(g);
+                    return ok;
+                },
+                // with every target blocked nothing but phases could follow
+                [&](const PassGate &) { return taken.size() < most && (targets & ~(f.x | f.z)); });
         }
 
         // A phase can wait until a 2x2 needs one of its qubits: of the gates just taken, the phases
-        // that no later taken 2x2 waits for go back to rem (in order), unless only phases are
-        // left.  They then join that 2x2's own phase instead of being multiplied in at the end
+        // that no later taken 2x2 waits for go back to rem (in order), unless nothing else was taken
+        // or is left.  They then join that 2x2's own phase instead of being multiplied in at the end
         // of each round.
-        void put_back_phases(const std::vector<PassGate> &gates, std::vector<int> &taken, std::vector<int> &rem)
+        void put_back_phases(const std::vector<PassGate> &gates, std::vector<int> &taken, Remaining &rem, size_t most = ~size_t(0))
         {
-            if (std::none_of(rem.begin(), rem.end(), [&](int i) { return gates[i].t >= 0; }))
+            if (rem.phases_only())
             {
-                taken.insert(taken.end(), rem.begin(), rem.end());
-                rem.clear();
+                rem.take_front(gates, taken, most - taken.size());
                 return;
             }
             uint64_t needed = 0;
@@ -531,32 +627,17 @@ namespace qcore
                     needed |= bit(g.t);
                 (g.t >= 0 || (g.cmask & needed) ? keep : back).push_back(taken[i]);
             }
-            if (back.empty())
+            if (back.empty() || keep.empty())
                 return;
             std::reverse(keep.begin(), keep.end());
             std::reverse(back.begin(), back.end());
             taken.swap(keep);
-            std::vector<int> merged(rem.size() + back.size());
-            std::merge(rem.begin(), rem.end(), back.begin(), back.end(), merged.begin());
-            rem.swap(merged);
+            rem.put_back(gates, back);
         }
 
         // Gates of a round: bounds its operations (at most two a gate, and the last flushes), so
         // that a round always fits the memory that programs pass through.
         constexpr size_t kRoundGates = (kProgramRoundOps - 2) / 2;
-
-        // Of more gates taken than a round holds, those past its end go back to rem.
-        void put_back_rest(std::vector<int> &taken, std::vector<int> &rem)
-        {
-            if (taken.size() <= kRoundGates)
-                return;
-            std::vector<int> back(taken.begin() + kRoundGates, taken.end()), merged;
-            taken.resize(kRoundGates);
-            std::sort(back.begin(), back.end()); // the circuit's order again
-            merged.reserve(rem.size() + back.size());
-            std::merge(rem.begin(), rem.end(), back.begin(), back.end(), std::back_inserter(merged));
-            rem.swap(merged);
-        }
 
         // Emits one round: register qubits reg[0..3] (ascending tile bits), the gates `taken`.
         void emit_round(PassPlan &P, const std::vector<PassGate> &gates, const uint8_t *tq, int m, uint32_t regbits, const std::vector<int> &taken)
@@ -693,7 +774,7 @@ namespace qcore
         }
 
         // the rounds of one sweep over the tile tq[0..m-1]
-        void plan_rounds(PassPlan &P, const std::vector<PassGate> &gates, std::vector<int> rem, const uint8_t *tq, int n, int m, int line_bits)
+        void plan_rounds(PassPlan &P, const std::vector<PassGate> &gates, Remaining rem, const uint8_t *tq, int n, int m, int line_bits)
         {
             uint64_t tile = 0;
             for (int b = 0; b < m; ++b)
@@ -722,11 +803,11 @@ namespace qcore
                 taken.clear();
                 uint64_t best = 0;
                 int best_w = -1;
-                const bool phases_only = std::none_of(rem.begin(), rem.end(), [&](int i) { return gates[i].t >= 0; });
+                const bool phases_only = rem.phases_only();
                 auto consider = [&](uint64_t set) {
                     if (!set)
                         return;
-                    int w = 4 * count_take(gates, rem.data(), rem.size(), set, set);
+                    int w = 4 * count_take(gates, rem, set, set, kRoundGates);
                     if (w == 0 && !phases_only)
                         return;
                     if (first && !(set & low))
@@ -737,17 +818,16 @@ namespace qcore
                         best_w = w, best = set;
                 };
                 uint64_t avoid = 0;
-                const uint64_t g0 = grow(gates, rem.data(), rem.size(), tile, 0, 4, true, avoid);
+                const uint64_t g0 = grow(gates, rem, tile, 0, 4, true, avoid, kRoundGates);
                 consider(fill(g0, avoid));
                 for (int b = 0; b + 4 <= std::min(m, n); ++b)
                     consider(bit(tq[b]) | bit(tq[b + 1]) | bit(tq[b + 2]) | bit(tq[b + 3]));
                 if (best_w <= 0 && !fill(g0, avoid))
                     throw std::runtime_error("pass: no register set for a gate");
-                take(gates, rem, best, best, taken);
+                take(gates, rem, best, best, taken, kRoundGates);
                 if (taken.empty())
                     throw std::runtime_error("pass: planning does not advance");
-                put_back_phases(gates, taken, rem);
-                put_back_rest(taken, rem);
+                put_back_phases(gates, taken, rem, kRoundGates);
                 if (first && (best & low))
                     emit_round(P, gates, tq, m, bits_of(top), {});
                 emit_round(P, gates, tq, m, bits_of(best), taken);
@@ -774,15 +854,13 @@ namespace qcore
     {
         struct Kept
         {
-            std::vector<int> rem;
+            Remaining rem;
             std::vector<uint64_t> tiles;
             long left = 0; // weight of rem
         };
-        std::vector<Kept> kept(1), next;
+        std::vector<Kept> kept(1, Kept{Remaining(gates), {}, 0}), next;
         if (n <= m || width < 1 || count < 1 || low_least < 3 || low_most > 4)
             return {};
-        for (size_t i = 0; i < gates.size(); ++i)
-            kept[0].rem.push_back(int(i));
         std::vector<int> taken;
         std::vector<std::pair<int, uint64_t>> tries;
         while (!gates.empty())
@@ -794,13 +872,13 @@ namespace qcore
                 auto add = [&](uint64_t set) {
                     set = fill_tile(set, n, m);
                     if (std::none_of(tries.begin(), tries.end(), [&](auto &t) { return t.second == set; }))
-                        tries.push_back({count_take(gates, k.rem.data(), k.rem.size(), set, 0), set});
+                        tries.push_back({count_take(gates, k.rem, set, 0), set});
                 };
                 for (int low_bits = low_least; low_bits <= low_most; ++low_bits)
                 {
                     const uint64_t low = bit(low_bits) - 1;
                     uint64_t avoid;
-                    add(grow(gates, k.rem.data(), k.rem.size(), bit(n) - 1, low, m - low_bits, false, avoid));
+                    add(grow(gates, k.rem, bit(n) - 1, low, m - low_bits, false, avoid));
                     for (int a = low_bits; a + (m - low_bits) <= n; ++a)
                         add(low | ((bit(m - low_bits) - 1) << a));
                 }
@@ -816,8 +894,8 @@ namespace qcore
                     x.tiles.push_back(tries[t].second);
                     if (x.rem.empty())
                         return x.tiles;
-                    for (int gi : x.rem)
-                        x.left += weight(gates[gi]);
+                    for (size_t i = 0; i < x.rem.size(); ++i)
+                        x.left += weight(gates[x.rem.data()[i]]);
                     // one of those that leave as much: mostly the same tiles in another order
                     if (std::none_of(next.begin(), next.end(), [&](auto &o) { return o.left == x.left && o.rem.size() == x.rem.size(); }))
                         next.push_back(std::move(x));
@@ -839,9 +917,7 @@ namespace qcore
             throw std::runtime_error("passes: state or tile size out of range");
         PassPlan P;
         P.m = m;
-        std::vector<int> rem(gates.size());
-        for (size_t i = 0; i < rem.size(); ++i)
-            rem[i] = int(i);
+        Remaining rem(gates);
         const int line_bits = n < 18 ? 0 : amp_bytes == 16 ? 3 : 4;
         std::vector<int> taken;
         while (!rem.empty())
@@ -851,22 +927,22 @@ namespace qcore
             {
                 for (int b = 0; b < m; ++b)
                     ps.tq[b] = uint8_t(b);
-                taken.swap(rem);
-                rem.clear();
+                taken.clear();
+                rem.take_front(gates, taken, rem.size());
             }
             else
             {
                 // the low qubits (contiguous runs of amplitudes) and m - low_bits others: those of
                 // the 2x2s in order, or the run of qubits that takes most
                 const uint64_t low = bit(low_bits) - 1, all = (bit(n) - 1);
-                uint64_t avoid, best = P.passes.size() < tiles.size() ? tiles[P.passes.size()] : grow(gates, rem.data(), rem.size(), all, low, m - low_bits, false, avoid);
+                uint64_t avoid, best = P.passes.size() < tiles.size() ? tiles[P.passes.size()] : grow(gates, rem, all, low, m - low_bits, false, avoid);
                 if (tiles.empty())
                 {
-                    int best_w = count_take(gates, rem.data(), rem.size(), best, 0);
+                    int best_w = count_take(gates, rem, best, 0);
                     for (int a = low_bits; a + (m - low_bits) <= n; ++a)
                     {
                         const uint64_t w = low | ((bit(m - low_bits) - 1) << a);
-                        const int c = count_take(gates, rem.data(), rem.size(), w, 0);
+                        const int c = count_take(gates, rem, w, 0);
                         if (c > best_w)
                             best_w = c, best = w;
                     }
@@ -883,7 +959,7 @@ namespace qcore
                 put_back_phases(gates, taken, rem);
             }
             ps.first_round = uint32_t(P.rounds.size());
-            plan_rounds(P, gates, taken, ps.tq, n, m, line_bits);
+            plan_rounds(P, gates, Remaining(gates, taken), ps.tq, n, m, line_bits);
             ps.nrounds = uint32_t(P.rounds.size()) - ps.first_round;
             P.passes.push_back(ps);
             if (planned)

@@ -604,7 +604,8 @@ namespace qcore
         // qubits, 20 layers: 405 and 372 us; 23 qubits, QAOA: 280 and 246); above, the plan with 4
         // is taken unless one with 3 has fewer passes (30 qubits, brick depth 3: 5 passes 33.2 ms,
         // 4 passes 27.5 ms; QFT: 7 either way, 56.2 and 58.0 ms), and from 28 qubits on, where a
-        // pass takes longer than the search (0.2 to 1 ms), more sequences of tiles are tried (30
+        // pass takes longer (1.4 ms at 28, 5.5 at 30) than the search for it (0.05 to 0.15 ms in plans
+        // of up to 10 passes, 0.2 to 0.3 in those of 100), more sequences of tiles are tried (30
         // qubits, 4 RY/RZ/CNOT layers: 6 passes 54.2 ms, 4 passes 42.3 ms; brick depth 24: 15 and
         // 13, 179 and 162 ms; 28 qubits, two-qubit gates: 6 and 5, 10.2 and 8.8 ms).
         // Complex64 lines are 16 amplitudes, and its passes are bound by arithmetic: 25 qubits, 6

@@ -1,4 +1,5 @@
-"""Pass programs on the CPU: how they are laid out for the device (tests/pass_align_check.cpp)."""
+"""Pass programs on the CPU: how they are laid out for the device, how they
+go there in parts, and what planning them takes (the programs tests/pass_*_check.cpp)."""
 import os
 import shutil
 import subprocess
@@ -33,3 +34,7 @@ def test_misaligned_programs_are_refused(tmp_path):
 @pytest.mark.parametrize("seed", [1, 2])
 def test_programs_in_parts(tmp_path, seed):
     check("pass_parts_check.cpp", tmp_path, seed)
+
+
+def test_planning_time_grows_with_the_circuit(tmp_path):
+    check("pass_time_check.cpp", tmp_path)
