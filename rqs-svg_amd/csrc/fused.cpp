@@ -577,7 +577,7 @@ namespace qcore
             // 30 -> 6.0 ms.  BF16x3 products (mode 3) are a choice of arithmetic and stay.
             if (passes_)
             {
-                const int passes = sim_.run_passes(gates);
+                const int passes = sim_.run_passes(gates.data(), gates.size());
                 if (passes >= 0)
                 {
                     blocks_applied_ += passes;

@@ -579,21 +579,28 @@ namespace qcore
             }
     }
 
-    int Simulator::run_passes(const std::vector<ResolvedGate> &gates)
+    // Whether a gate may be in a pass: a controlled 2x2 needs 4 register bits clear of its
+    // controls.
+    bool Simulator::pass_takes(const ResolvedGate &g) const { return int(g.pphys.size() + g.nphys.size() + g.tphys.size()) <= pass_tile_bits(n_) - 4; }
+
+    // What a kernel of its own for the gate moves, in sweeps of the state.
+    static double sweeps_alone(const ResolvedGate &g)
+    {
+        const Kind kd = g.spec.kind;
+        return kd == Kind::Identity ? 0.0 : std::ldexp(kd == Kind::PhaseOne || kd == Kind::PairSub ? 0.5 : 1.0, -int(g.pphys.size() + g.nphys.size()));
+    }
+
+    int Simulator::run_passes(const ResolvedGate *gates, size_t count)
     {
         const int m = pass_tile_bits(n_);
         const int amp_bytes = fused_ && !fused_->f64() ? 8 : 16;
         PassLowering lowering(n_);
         double bytes = 0; // what one kernel per gate would move, in sweeps of the state
-        for (const ResolvedGate &g : gates)
+        for (size_t i = 0; i < count; ++i)
         {
-            const int nc = int(g.pphys.size() + g.nphys.size());
-            // a controlled 2x2 needs 4 register bits clear of its controls
-            if (nc + int(g.tphys.size()) > m - 4 || !lowering.add(g))
+            if (!pass_takes(gates[i]) || !lowering.add(gates[i]))
                 return -1;
-            const Kind kd = g.spec.kind;
-            if (kd != Kind::Identity)
-                bytes += std::ldexp(kd == Kind::PhaseOne || kd == Kind::PairSub ? 0.5 : 1.0, -nc);
+            bytes += sweeps_alone(gates[i]);
         }
         const std::vector<PassGate> low = lowering.finish();
         if (low.empty())
@@ -622,7 +629,7 @@ namespace qcore
                     tiles = std::move(four);
             }
             // A pass moves the whole state once, so few gates with many controls are cheaper one
-            // by one; on smaller states the launches count, not the bytes.
+            // by one.
             if (bytes < double(tiles.size()))
                 return -1;
         }
@@ -700,10 +707,34 @@ namespace qcore
         if (gates.empty())
             return;
         state_changed();
-        if (gates.size() > 1 && run_passes(gates) >= 0)
-            return;
-        for (const auto &g : gates)
-            apply_resolved(g);
+        // Up to 22 qubits a pass is worth its program's copy and its sweep where the gates' own
+        // kernels take longer, in us: 3.4 a launch, or on larger states twice their share of a sweep
+        // (they touch parts of lines), against 6.5 more for the first pass, 0.5 a gate, and of the
+        // sweep what its launch does not cover.  (Calls that are waited for, gates' kernels and
+        // passes: 10 qubits, 2 Hadamards 21.1 and 22.9 us, 3 23.4 and 23.7, 5 30.4 and 23.4; 22
+        // qubits, X with 6 controls, 2 24.6 and 41.2, 6 37.6 and 43.6, 8 44.0 and 45.9, 12 57.9 and
+        // 48.4, with 2 controls, 2 32.4 and 37.4, 3 52.0 and 41.0, Hadamards, 2 54.7 and 51.9.)
+        const double sweep = std::ldexp(32.0, n_) / 6.2e6;
+        auto worth = [&](size_t first, size_t end) {
+            if (n_ > 22)
+                return end - first > 1;
+            double alone = 0;
+            for (size_t i = first; i < end; ++i)
+                if (const double share = sweeps_alone(gates[i]))
+                    alone += std::max(3.4, std::min(1.0, 2 * share) * sweep);
+            return alone > 6.5 + 0.5 * double(end - first) + std::max(0.0, sweep - 5.0);
+        };
+        for (size_t i = 0; i < gates.size();)
+        {
+            // the next gates that passes take, and those that they don't
+            size_t end = i;
+            while (end < gates.size() && pass_takes(gates[end]))
+                ++end;
+            if (end > i && worth(i, end) && run_passes(&gates[i], end - i) >= 0)
+                i = end;
+            for (; i < end || (i < gates.size() && !pass_takes(gates[i])); ++i)
+                apply_resolved(gates[i]);
+        }
     }
 
     void Simulator::apply_resolved(const ResolvedGate &r)

@@ -120,7 +120,8 @@ namespace qcore
         void apply_run(const std::vector<ResolvedGate> &gates);
         // Applies gates as circuit passes and returns how many sweeps that took, or returns -1 with
         // nothing done where they have no such form or would not pay for their sweeps.
-        int run_passes(const std::vector<ResolvedGate> &gates);
+        int run_passes(const ResolvedGate *gates, size_t count);
+        bool pass_takes(const ResolvedGate &g) const;
         void ensure_levels();
         uint64_t stage_len() const;
         void ensure_stage();
