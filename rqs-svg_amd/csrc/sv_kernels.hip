@@ -606,16 +606,21 @@ namespace qsv
                 p = prob(lda(s + u));
         }
 
-        template <class A>
-        __global__ __launch_bounds__(kBlock) void k_reduce_probs(const A *__restrict__ s, uint64_t count, double *__restrict__ out)
+        // SIGNED: p negated where index bit zbit is set
+        template <class A, bool SIGNED>
+        __global__ __launch_bounds__(kBlock) void k_reduce_probs(const A *__restrict__ s, uint64_t count, uint64_t zbit, double *__restrict__ out)
         {
             double y[1][16];
             uint64_t base = uint64_t(blockIdx.x) * kTile + threadIdx.x;
 #pragma unroll
             for (int j = 0; j < 16; ++j)
             {
-                double e;
-                unit_probs<A>(s, count, base + uint64_t(j) * kBlock, y[0][j], e);
+                const uint64_t u = base + uint64_t(j) * kBlock;
+                double p, e;
+                unit_probs<A>(s, count, u, p, e);
+                if (SIGNED)
+                    p = zbit < reduce_per_unit<A>() ? e : (u * reduce_per_unit<A>()) & zbit ? -p : p;
+                y[0][j] = p;
             }
             tile_tree<1>(y, out + blockIdx.x, 0);
         }
@@ -1662,20 +1667,21 @@ namespace qsv
     }
 
     template <class A>
-    void reduce_probs(hipStream_t s, const A *state, uint64_t count, double *work, double *out)
+    void reduce_probs(hipStream_t s, const A *state, uint64_t count, double *work, double *out, uint64_t zbit)
     {
+        const auto first = zbit ? k_reduce_probs<A, true> : k_reduce_probs<A, false>;
         if (reduce_per_unit<A>() == 2 && (count & 1))
             throw std::runtime_error("reduce: complex64 states have an even amplitude count");
         uint64_t g = (count / reduce_per_unit<A>() + kTile - 1) / kTile;
         double *lvl = work; // level arrays
         if (g == 1)
         {
-            hipLaunchKernelGGL(k_reduce_probs<A>, dim3(1), dim3(kBlock), 0, s, state, count, out);
+            hipLaunchKernelGGL(first, dim3(1), dim3(kBlock), 0, s, state, count, zbit, out);
             after_launch("reduce kernel");
         }
         else
         {
-            hipLaunchKernelGGL(k_reduce_probs<A>, dim3(g), dim3(kBlock), 0, s, state, count, lvl);
+            hipLaunchKernelGGL(first, dim3(g), dim3(kBlock), 0, s, state, count, zbit, lvl);
             after_launch("reduce kernel");
             finish_tiles<1>(s, lvl, g, g, lvl + g, out);
         }
@@ -1713,6 +1719,12 @@ namespace qsv
         for (int i = 0; i < nbits; ++i)
             if (bits[i] < 0 || bits[i] >= n)
                 throw std::runtime_error("expect_z: qubit out of range");
+        if (nbits == 1)
+        { // one signed reduction: 29 qubits 1.28 ms, with the differences of all qubits 1.45
+            reduce_probs(s, state, count, work, pinned, uint64_t(1) << bits[0]);
+            out[0] = pinned[0];
+            return;
+        }
         const uint64_t g = (count / P + kTile - 1) / kTile;
         const int nv1 = 1 + kTileBits + (P == 2 ? 1 : 0);
         // value of unit bit b: array 1 + b for b < 12, then 12 more arrays per level
@@ -1767,12 +1779,12 @@ namespace qsv
         double *lvl = work + 2;
         if (g == 1)
         {
-            hipLaunchKernelGGL(k_reduce_probs<A>, dim3(1), dim3(kBlock), 0, s, state, count, dev_out);
+            hipLaunchKernelGGL((k_reduce_probs<A, false>), dim3(1), dim3(kBlock), 0, s, state, count, uint64_t(0), dev_out);
             after_launch("reduce kernel");
         }
         else
         {
-            hipLaunchKernelGGL(k_reduce_probs<A>, dim3(g), dim3(kBlock), 0, s, state, count, lvl);
+            hipLaunchKernelGGL((k_reduce_probs<A, false>), dim3(g), dim3(kBlock), 0, s, state, count, uint64_t(0), lvl);
             after_launch("reduce kernel");
             finish_tiles<1>(s, lvl, g, g, lvl + g, dev_out);
         }
@@ -2157,7 +2169,7 @@ namespace qsv
     template void launch_fill_random<A>(hipStream_t, A *, uint64_t, uint64_t);                                                                          \
     template void launch_set_one<A>(hipStream_t, A *, uint64_t);                                                                                        \
     template void reduce_pair_probs<A>(hipStream_t, const A *, const Subspace &, uint64_t, uint64_t, double *, double *);                               \
-    template void reduce_probs<A>(hipStream_t, const A *, uint64_t, double *, double *);                                                                \
+    template void reduce_probs<A>(hipStream_t, const A *, uint64_t, double *, double *, uint64_t);                                                      \
     template void expect_z<A>(hipStream_t, const A *, int, double *, double *, const int *, int, double *);                                            \
     template void launch_collapse<A>(hipStream_t, A *, int, int, int, double, const int *, int, uint64_t);                                               \
     template void renormalize_async<A>(hipStream_t, A *, uint64_t, double *);                                                                           \

@@ -104,9 +104,9 @@ namespace qsv
     // {p0,p1} over the subspace `sub` (p1 at index | tbit)
     template <class A>
     void reduce_pair_probs(hipStream_t s, const A *state, const Subspace &sub, uint64_t tbit, uint64_t nitems, double *work, double *out);
-    // canonical sum of p(i) over all amplitudes
+    // canonical sum of p(i) over all amplitudes, negated where index bit zbit (if any) is set
     template <class A>
-    void reduce_probs(hipStream_t s, const A *state, uint64_t count, double *work, double *out);
+    void reduce_probs(hipStream_t s, const A *state, uint64_t count, double *work, double *out, uint64_t zbit = 0);
     // out[i] = canonical sum of p negated where physical bit bits[i] is set, i < nbits, all
     // from one read of the 2^n amplitudes; work holds expz_workspace(2^n) doubles, pinned 64
     // doubles of pinned host memory (the last kernel writes there).  Synchronises `s`.
