@@ -108,6 +108,9 @@ namespace qcore
         for (auto e : ring_read_)
             if (e)
                 (void)hipEventDestroy(e);
+        for (auto e : shots_there_)
+            if (e)
+                (void)hipEventDestroy(e);
         if (pinned_)
             (void)hipHostFree(pinned_);
         if (stream_)
@@ -1240,28 +1243,41 @@ namespace qcore
         if (shots == 0)
             return;
         // through pinned memory that the search writes: an allocation, a copy and a release each
-        // call took 40 us
-        const uint64_t cap = std::min(shots, kShotChunk);
-        if (cap > shots_cap_)
+        // call took 40 us.  More outcomes than one fetch come in turn to its two halves, and
+        // one is searched while the other is copied out (8388608 outcomes of 10 qubits: 8.2 ms
+        // one after the other, 5.3 so).
+        const uint64_t cap = std::min(shots, kShotChunk), halves = shots > cap ? 2 : 1;
+        if (halves * cap > shots_cap_)
         {
             if (shots_)
                 (void)hipHostFree(shots_);
             shots_ = nullptr;
             shots_cap_ = 0;
             uint64_t want = 1024;
-            while (want < cap)
+            while (want < halves * cap)
                 want *= 2;
             qsv::check(hipHostMalloc((void **)&shots_, want * sizeof(uint64_t), hipHostMallocDefault), "hipHostMalloc outcomes");
             shots_cap_ = want;
         }
-        for (uint64_t first = 0; first < shots; first += cap)
-        {
-            const uint64_t n = std::min(cap, shots - first);
+        auto search = [&](uint64_t chunk) {
+            const uint64_t first = chunk * cap;
             prof_begin(QCS_EXT_K_SAMPLE, 0.0);
-            with_state([&](auto *st) { qsv::launch_sample_search(stream_, st, uint64_t(1) << n_, levels_, total, seed, first, n, p2l_.data(), n_, shots_); });
+            with_state([&](auto *st) { qsv::launch_sample_search(stream_, st, uint64_t(1) << n_, levels_, total, seed, first, std::min(cap, shots - first), p2l_.data(), n_, shots_ + chunk % 2 * cap); });
             prof_end();
-            qsv::check(hipStreamSynchronize(stream_), "sync");
-            std::memcpy(out + first, shots_, n * sizeof(uint64_t));
+            if (halves == 1)
+                return;
+            hipEvent_t &e = shots_there_[chunk % 2];
+            if (!e)
+                qsv::check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
+            qsv::check(hipEventRecord(e, stream_), "hipEventRecord");
+        };
+        search(0);
+        for (uint64_t chunk = 0, first = 0; first < shots; ++chunk, first += cap)
+        {
+            if (first + cap < shots)
+                search(chunk + 1);
+            qsv::check(halves == 1 ? hipStreamSynchronize(stream_) : hipEventSynchronize(shots_there_[chunk % 2]), "sync");
+            std::memcpy(out + first, shots_ + chunk % 2 * cap, std::min(cap, shots - first) * sizeof(uint64_t));
         }
     }
 

@@ -165,6 +165,7 @@ namespace qcore
         static constexpr uint64_t kShotChunk = 65536; // outcomes fetched at a time
         uint64_t *shots_ = nullptr;                   // pinned, kept until free_memory
         uint64_t shots_cap_ = 0;
+        hipEvent_t shots_there_[2] = {};
         double levels_total_ = 0.0;
         void state_changed() { levels_valid_ = false; }
         // every amplitude that contradicts a measured qubit's value is zero
