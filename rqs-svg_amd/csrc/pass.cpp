@@ -230,11 +230,26 @@ namespace qcore
         return std::move(out_);
     }
 
+    static bool finite(const GateSpec &s)
+    {
+        double zero = 0.0;
+        auto look = [&](const cd *z, int count) {
+            for (int i = 0; i < count; ++i)
+                zero += 0.0 * z[i].real() + 0.0 * z[i].imag();
+        };
+        look(s.phase, 4);
+        look(s.m, s.kind == Kind::Dense4 ? 16 : 4);
+        look(s.coef, s.nrows);
+        return zero == 0.0;
+    }
+
     bool PassLowering::add(const ResolvedGate &g)
     {
-        if (g.mmask)
-            return false;
         const GateSpec &s = g.spec;
+        // multiplied into others, an angle that is no number would reach amplitudes that its gate
+        // leaves alone
+        if (g.mmask || !finite(s))
+            return false;
         uint64_t c1 = 0, c0 = 0;
         for (int q : g.pphys)
             c1 |= bit(q);

@@ -32,7 +32,7 @@ namespace qcore
     {
     public:
         explicit PassLowering(int n) : one_(n) {}
-        // false, with nothing changed, for a gate that has no such form
+        // false, with nothing changed, for a gate that has no such form (or holds no numbers)
         bool add(const ResolvedGate &g);
         // the operations of every gate added
         std::vector<PassGate> finish();
