@@ -45,9 +45,10 @@ namespace qcore
                 m[i] = u[i];
         }
 
-        // f(0) .. f(count - 1), each once, on up to 16 threads of at least 8 calls each
-        template <class F>
-        void for_each_circuit(size_t count, F f)
+        // f(0) .. f(count - 1), each once, on up to `threads` threads; first meanwhile(), on this one
+        // beside the others
+        template <class F, class M>
+        void for_each_circuit(size_t count, size_t threads, F f, M meanwhile)
         {
             std::exception_ptr err;
             std::mutex err_mu;
@@ -64,7 +65,7 @@ namespace qcore
                     err = std::current_exception();
                 }
             };
-            const size_t threads = std::min<size_t>({size_t(16), std::max(1u, std::thread::hardware_concurrency()), count / 8});
+            threads = std::min<size_t>({threads, std::max(1u, std::thread::hardware_concurrency()), count});
             std::vector<std::thread> pool;
             pool.reserve(threads);
             try
@@ -74,6 +75,15 @@ namespace qcore
             }
             catch (const std::exception &)
             { // fewer threads, then
+            }
+            try
+            {
+                meanwhile();
+            }
+            catch (...)
+            {
+                std::lock_guard<std::mutex> lock(err_mu);
+                err = std::current_exception();
             }
             work();
             for (auto &th : pool)
@@ -196,7 +206,16 @@ namespace qcore
             return;
         if (circuits_.empty())
             throw std::runtime_error("batch: no circuits");
+        release(); // what a preparation that failed left
         const BatchTuning &T = tuning_;
+        auto make_streams = [&](int count) {
+            while ((int)streams_.size() < std::clamp(count, 1, T.streams))
+            {
+                hipStream_t s;
+                qsv::check(hipStreamCreateWithFlags(&s, hipStreamNonBlocking), "hipStreamCreate");
+                streams_.push_back(s);
+            }
+        };
         // ---- small circuits: op lists for the persistent kernel ----
         std::vector<qsv::BatchCircuit> small;
         std::vector<qsv::BatchOp> ops;
@@ -208,11 +227,21 @@ namespace qcore
             PassPlan plan;
         };
         std::vector<Passed> passed;
-        // The circuits' pass plans, on up to 16 host threads: 50 us a circuit, 256 circuits would
-        // wait 13 ms for their first run (no passes: a circuit without such a plan).
+        // The circuits' pass plans (no passes: a circuit without such a plan), on up to 16 host threads
+        // of at least 512 gates each, some 200 us of work.  The streams are created beside them,
+        // one a kind of circuit as far as the sizes tell: several take 0.3 to 2 ms.  (First run,
+        // before passes, with 8 circuits a thread and the streams afterwards, and so: 8 circuits of
+        // 4-6 qubits and 150 layers 2.4, 4.0 and 1.8 ms; 256 of 8-14 and 6 layers 4.7, 6.1 and 4.5.)
         std::vector<PassPlan> plans(circuits_.size());
+        size_t gates = 0;
+        int kinds[4] = {}; // up to 10, 11, 12 and more qubits
+        for (const Circuit &C : circuits_)
+        {
+            gates += C.gates.size();
+            ++kinds[std::clamp(C.n, qsv::kPassMinBits, qsv::kPassMaxBits + 1) - qsv::kPassMinBits];
+        }
         if (passes_)
-            for_each_circuit(circuits_.size(), [&](size_t ci) {
+            for_each_circuit(circuits_.size(), std::min<size_t>(16, gates / 512), [&](size_t ci) {
                 const Circuit &C = circuits_[ci];
                 if (x3_ && C.n > T.lds_max_qubits)
                     return;
@@ -229,7 +258,7 @@ namespace qcore
                 const auto low = lowering.finish();
                 if (!low.empty())
                     plans[ci] = plan_passes(low, C.n, std::clamp(C.n, qsv::kPassMinBits, qsv::kPassMaxBits), 8);
-            });
+            }, [&] { make_streams(std::min(kinds[0], 1) + std::min(kinds[1], 1) + std::min(kinds[2], 1) + std::min(kinds[3], 2)); });
         for (int ci = 0; ci < (int)circuits_.size(); ++ci)
         {
             const Circuit &C = circuits_[ci];
@@ -364,9 +393,6 @@ namespace qcore
             const int na = circuits_[a.ci].n, nb = circuits_[b.ci].n;
             return na != nb ? na > nb : a.plan.work > b.plan.work;
         });
-        std::vector<qsv::PassRound> prounds;
-        std::vector<qsv::PassOp> pops;
-        std::vector<qsv::PassZ> pz;
         struct PassLaunch
         {
             int m;
@@ -412,26 +438,35 @@ namespace qcore
             qsv::check(hipMalloc((void **)&d_partials_, partial_total * sizeof(double)), "hipMalloc batch");
         if (sums_total)
             qsv::check(hipMalloc((void **)&d_sums_, sums_total * sizeof(double)), "hipMalloc batch");
-        size_t nrounds_total = 0, nops_total = 0;
+        // the program, written once: rounds, padding, operations, tasks of each launch, <Z> entries
+        // (all multiples of 16 bytes)
+        static_assert(sizeof(qsv::PassRound) % 16 == 0 && sizeof(qsv::PassOp) % 16 == 0 && sizeof(qsv::PassTask) % 16 == 0 && sizeof(qsv::PassZ) % 16 == 0, "pass program alignment");
+        size_t nrounds = 0, nops = 0, ntasks = 0, nz = 0;
         for (const auto &pc : passed)
         {
-            nrounds_total += pc.plan.rounds.size();
-            nops_total += pc.plan.ops.size();
+            nrounds += pc.plan.rounds.size();
+            nops += pc.plan.ops.size();
+            ntasks += pc.plan.passes.size();
+            nz += one_launch ? 0 : size_t(circuits_[pc.ci].n);
         }
-        prounds.reserve(nrounds_total);
-        pops.reserve(nops_total);
+        const size_t pops_off = qsv::pass_rounds_bytes(nrounds), tasks_off = pops_off + nops * sizeof(qsv::PassOp), pz_off = tasks_off + ntasks * sizeof(qsv::PassTask);
+        // (one small circuit's task and entries are less than the padding of its operations)
+        const size_t prog_bytes = passed.empty() ? 0 : std::max(pz_off + nz * sizeof(qsv::PassZ), pops_off + (nops + qsv::kPassOpPad) * sizeof(qsv::PassOp));
+        const std::unique_ptr<char[]> prog(new char[prog_bytes]);
+        auto put = [&](size_t at, const void *src, size_t bytes) { std::memcpy(prog.get() + at, src, bytes); };
+        uint32_t first_round = 0, first_op = 0, pz_count = 0;
         for (size_t i = 0; i < passed.size(); ++i)
         {
             const Circuit &C = circuits_[passed[i].ci];
             const PassPlan &P = passed[i].plan;
             const int n = C.n, m = P.m;
             const uint32_t tiles = n > m ? uint32_t(1) << (n - m) : 1;
-            const uint32_t first_op = uint32_t(pops.size()), first_round = uint32_t(prounds.size());
-            pops.insert(pops.end(), P.ops.begin(), P.ops.end());
-            for (auto r : P.rounds)
+            put(pops_off + first_op * sizeof(qsv::PassOp), P.ops.data(), P.ops.size() * sizeof(qsv::PassOp));
+            for (size_t k = 0; k < P.rounds.size(); ++k)
             {
+                qsv::PassRound r = P.rounds[k];
                 r.first += first_op;
-                prounds.push_back(r);
+                put((first_round + k) * sizeof r, &r, sizeof r);
             }
             for (size_t p = 0; p < P.passes.size(); ++p)
             {
@@ -467,33 +502,24 @@ namespace qcore
                         z.ntiles = tiles;
                         z.slot = b < m ? 1 + b : 0;
                         z.sign = b < m ? 0 : uint32_t(1) << outside++;
-                        pz.push_back(z);
+                        put(pz_off + pz_count++ * sizeof z, &z, sizeof z);
                     }
                 }
                 L.tiles += tiles;
                 L.tasks.push_back(t);
             }
             large_passed += n > m;
+            first_round += uint32_t(P.rounds.size());
+            first_op += uint32_t(P.ops.size());
         }
-        // rounds, padding, operations, tasks of each launch, <Z> entries (all multiples of 16 bytes)
-        std::vector<char> prog;
-        auto put = [&](const void *src, size_t bytes) {
-            const size_t off = prog.size();
-            prog.insert(prog.end(), static_cast<const char *>(src), static_cast<const char *>(src) + bytes);
-            return off;
-        };
-        static_assert(sizeof(qsv::PassRound) % 16 == 0 && sizeof(qsv::PassOp) % 16 == 0 && sizeof(qsv::PassTask) % 16 == 0 && sizeof(qsv::PassZ) % 16 == 0, "pass program alignment");
-        prog.reserve(qsv::pass_rounds_bytes(prounds.size()) + pops.size() * sizeof(qsv::PassOp) + pz.size() * sizeof(qsv::PassZ) + (2 * passed.size() + plaunch.size()) * sizeof(qsv::PassTask));
-        put(prounds.data(), prounds.size() * sizeof(qsv::PassRound));
-        prog.resize(qsv::pass_rounds_bytes(prounds.size()));
-        const size_t pops_off = put(pops.data(), pops.size() * sizeof(qsv::PassOp));
+        size_t at = tasks_off;
         for (auto &L : plaunch)
-            L.offset = put(L.tasks.data(), L.tasks.size() * sizeof(qsv::PassTask));
-        const size_t pz_off = put(pz.data(), pz.size() * sizeof(qsv::PassZ));
-        const uint32_t pz_count = uint32_t(pz.size());
-        if (!pops.empty()) // one small circuit's task and entries are less than the padding
-            prog.resize(std::max(prog.size(), pops_off + (pops.size() + qsv::kPassOpPad) * sizeof(qsv::PassOp)));
-        upload(&d_prog_, prog.data(), prog.size());
+        {
+            L.offset = at;
+            put(at, L.tasks.data(), L.tasks.size() * sizeof(qsv::PassTask));
+            at += L.tasks.size() * sizeof(qsv::PassTask);
+        }
+        upload(&d_prog_, prog.get(), prog_bytes);
         // states within the 256 MB memory-side cache keep cached accesses
         const bool pass_nt = state_total * sizeof(qsv::c64) > (uint64_t(256) << 20);
         // ---- staged circuits: task arrays of the rounds, the fill and the reduction ----
@@ -587,7 +613,7 @@ namespace qcore
         }
         for (const auto &L : plaunch)
             launches_ += L.tasks.empty() ? 0 : 1;
-        launches_ += pz.empty() ? 0 : 1;
+        launches_ += pz_count > 0;
         int grid = 0;
         if (!small.empty())
         {
@@ -595,17 +621,12 @@ namespace qcore
             grid = std::min<int>(qsv::batch_lds_grid(T.block_size, small_max_n), (int)small.size());
         }
         // ---- streams and graph capture ----
-        // no more streams than chains of launches: each takes 30 us to create
+        // no more streams than chains of launches
         int chains = int(!small.empty()) + int(!staged.empty()) + (blocked.empty() ? 0 : T.streams) + int(std::min<size_t>(large_passed, 2));
         for (int i = 0; i < 3; ++i)
             chains += int(!plaunch[i].tasks.empty());
         const int ns = std::clamp(chains, 1, T.streams);
-        for (int i = 0; i < ns; ++i)
-        {
-            hipStream_t s;
-            qsv::check(hipStreamCreateWithFlags(&s, hipStreamNonBlocking), "hipStreamCreate");
-            streams_.push_back(s);
-        }
+        make_streams(ns);
         for (int i = 0; i < 2 * ns; ++i)
         {
             hipEvent_t e;
