@@ -217,8 +217,12 @@ namespace qsv
     QSV_TURN1(i)                                      \
     ".Lqsv_tu" #i "_%=:\n\t"
 #define QSV_TURN_IF(i, j) QSV_TURN1_IF(i) QSV_TURN1_IF(j)
+        // Each operation begins a line of instructions: a wave that is alone on its SIMD waits for
+        // their fetch, and without this its time changes with the length of the code before (8
+        // circuits of 4-6 qubits and 150 layers, the touch above written three ways: 570, 576 and
+        // 605 us, on lines 547 and 562).
 #define QSV_CASE(n, body)                             \
-    ".Lqsv_c" #n "_%=:\n\t"                           \
+    ".p2align 6\n.Lqsv_c" #n "_%=:\n\t"               \
     body                                              \
     "s_branch .Lqsv_end_%=\n\t"
 #define QSV_CASES(n0, n1, n2, n3, F)                                                      \
