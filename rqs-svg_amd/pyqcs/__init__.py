@@ -288,7 +288,7 @@ class Simulator:
     def run(self, circuit):
         """Apply a list of (name, targets, params, ctrls, negctrls) tuples: as one call, or gate by
         gate where `gate` is overridden."""
-        own = "gate" in self.__dict__ or type(self).gate is not Simulator.gate  # sees every gate
+        own = "gate" in self.__dict__ or type(self).gate is not __class__.gate  # sees every gate
         packed = _pack_circuit(circuit) if not own and type(circuit) in (list, tuple) and not self._few(circuit) else None
         if packed is None:
             for op in circuit:
