@@ -52,6 +52,18 @@ def log(msg):
     print(msg, file=sys.stderr, flush=True)
 
 
+def brief(x):
+    """The result with its numbers to 6 digits (those near 1, the fidelities, to 12), so that the
+    line stays short of 16000 characters, the length that is kept of a run's output."""
+    if isinstance(x, dict):
+        return {k: brief(v) for k, v in x.items()}
+    if isinstance(x, (list, tuple)):
+        return [brief(v) for v in x]
+    if isinstance(x, float):
+        return float(f"{x:.12g}" if abs(x - 1) < 1e-3 else f"{x:.6g}")
+    return x
+
+
 def traffic_from_profiles():
     """HBM bytes per pass measured with rocprofv3 PMC counters, if committed."""
     f = REPO / "profiles" / "pass_kernel_brick30_traffic.json"
@@ -347,8 +359,7 @@ def _class_rate(sim, cls):
         return None
     avg = v["seconds"] / v["launches"]
     gbs = v["bytes"] / v["seconds"] / 1e9
-    return {"launches": v["launches"], "avg_ms": avg * 1e3, "GBps": gbs, "frac": gbs / (HBM_PEAK / 1e9),
-            "bytes_per_launch": v["bytes"] / v["launches"]}
+    return {"launches": v["launches"], "avg_ms": avg * 1e3, "GBps": gbs, "frac": gbs / (HBM_PEAK / 1e9)}
 
 
 SUBSYSTEM_GATES = (
@@ -402,6 +413,7 @@ def subsystem_leg(n=30, reps=4):
                 sim.gate(name, tg, params, ctrls=ctl)
             r = _class_rate(sim, cls)
             sim.profile(False)
+            del r["launches"]  # reps
             r["operands"] = list(tg)
             if ctl:
                 r["controls"] = list(ctl)
@@ -806,7 +818,9 @@ def main():
                                                             fixed_sweep=args.planner_fixed_sweep)
     if not args.no_cpu_baseline:
         result["cpu_baseline"] = cpu_baseline(n, circ, args.cpu_budget)
-    print(json.dumps(result), flush=True)
+    line = json.dumps({**brief(result), "value": result["value"], "ms_per_step": result["ms_per_step"]}, separators=(",", ":"))
+    log(f"result line: {len(line)} characters")
+    print(line, flush=True)
 
 
 if __name__ == "__main__":
