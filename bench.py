@@ -512,11 +512,12 @@ def planner_leg(n, depth, record_count, k=4, fixed_sweep=False):
     the plan the model picks (taken only when its predicted gain
     over the default exceeds the model's error; one run each, so an override runs as the
     model picked it, before the planner's measured check has compared it with the default)
-    -- and each output compared with the plain complex128 method on a second state in HBM."""
+    -- and each output compared with a second state in HBM, whose gates are called one by
+    one: a kernel per gate, which shares no code with passes or stages."""
     lib = pyqcs.gpu_library()
     model, info = pyqcs.train_cost_model(lib, 2, k, (26, 28, 30, 32), record_count, (26, 28, 30), log=log)
     out = {"config": f"complex128 fused blocks (k<={k}), {n}-qubit QFT on a random brick layer and "
-                     f"{n}-qubit brick depth {depth}; outputs against the plain complex128 method",
+                     f"{n}-qubit brick depth {depth}; outputs against complex128 gate by gate",
            "cost_model": info}
     prep_qft = circuits.brick(n, 1, seed=CIRCUIT_SEED + 9)
     work = {"qft": (prep_qft, circuits.qft(n)), "brick": ((), circuits.brick(n, depth, seed=CIRCUIT_SEED + 5))}
@@ -536,10 +537,12 @@ def planner_leg(n, depth, record_count, k=4, fixed_sweep=False):
         for name, (prep, circ) in work.items():
             res = {"gates": len(circ)}
             plain.call("set_zero_state")
-            plain.run(prep)
+            for op in prep:
+                plain.gate(*op)
             plain.norm()
             t0 = time.perf_counter()
-            plain.run(circ)
+            for op in circ:
+                plain.gate(*op)
             plain.norm()
             res["plain_per_gate_s"] = time.perf_counter() - t0
             for mode in ("greedy", "stages", "passes", "learned"):
@@ -565,7 +568,7 @@ def planner_leg(n, depth, record_count, k=4, fixed_sweep=False):
                     res["learned_choices"] = st1["learned_choices"] - st0["learned_choices"]
                     res["flushes"] = st1["flushes"] - st0["flushes"]
                     res["learned_plan"] = list(pyqcs.planner_last_choice(fused))
-                log(f"planner leg: {name} {mode}: {dt:.3f}s, {b1 - b0} sweeps, fidelity vs plain "
+                log(f"planner leg: {name} {mode}: {dt:.3f}s, {b1 - b0} sweeps, fidelity vs per-gate "
                     f"{fid:.15f}, max|d| {maxdiff:.2e}")
             pyqcs.set_planner(fused, None)
             if fixed_sweep:
@@ -584,7 +587,7 @@ def planner_leg(n, depth, record_count, k=4, fixed_sweep=False):
             res["learned_vs_greedy"] = res["greedy_s"] / res["learned_s"]
             res["stages_vs_greedy"] = res["greedy_s"] / res["stages_s"]
             log(f"planner leg: {name}: learned vs default stages {res['learned_vs_stages']:.3f}x, "
-                f"vs greedy {res['learned_vs_greedy']:.2f}x; plain {res['plain_per_gate_s']:.2f}s")
+                f"vs greedy {res['learned_vs_greedy']:.2f}x; per gate {res['plain_per_gate_s']:.2f}s")
             out[name] = res
     finally:
         pyqcs.set_planner(fused, None)
