@@ -142,6 +142,10 @@ namespace qcore
 
     void PassLowering::phase(uint64_t cmask, uint64_t cval, cl p)
     {
+        // Entries of a gate lie off the unit circle by their rounding to double.  A ratio of several
+        // of them would add that up (RZZ as the phase of both its qubits' |1>: four times); scaled
+        // to modulus 1 it keeps their angles' errors only, as the gate has them.
+        p = unit(p);
         if (p == cl(1.0))
             return;
         if (!cmask)
