@@ -109,10 +109,13 @@ int qcs_ext_set_local_qubits(qcs_simulator *sim, bit_num_t num_local_qubits);
  * and num_ctrls[i] entries of targets, negctrls and ctrls (params must not be NULL).
  * The state afterwards is what the same calls one by one leave, up to FP64 rounding (gates on
  * different qubits may be applied in another order), and all work is queued on the stream on
- * return.  Without measured qubits, complex128 states (precision 0) take runs of gates in
- * passes of several gates per sweep.  *num_applied: gates applied; when a gate is refused
- * the gates before it have been.  (Should the device itself fail, the state is undefined and
- * the count is of gates whose passes were all launched.) */
+ * return.  Without measured qubits and a window of local ones, complex128 states (precision 0)
+ * take runs of gates in passes of several gates per sweep where those are faster than the
+ * gates' own kernels; a run ends at a gate with too many controls for a pass (controls +
+ * targets > 6 to 8, by the state's size), and one with an angle that is no number goes gate by
+ * gate.  *num_applied: gates applied; when a gate is refused the gates before it have been.
+ * (Should the device itself fail, the state is undefined and the count is of gates whose passes
+ * were all launched.) */
 int qcs_ext_run_circuit(qcs_simulator *sim, int32_t count, const char *const *names, const int32_t *num_params,
                         const uint8_t *name_of, const uint8_t *num_targets, const uint8_t *num_negctrls,
                         const uint8_t *num_ctrls, const bit_num_t *targets, const bit_num_t *negctrls,
@@ -230,7 +233,9 @@ int qcs_ext_batch_run_direct(qcs_ext_batch *batch, double *expz, uint64_t count,
  * default plan's by the model's own typical error: a factor 2^-rms, rms = the root mean
  * squared error (log2 microseconds) of the model's last qcs_ext_mlp_train on its data,
  * within [0.75, 0.97] (0.97 for parameters set by qcs_ext_mlp_set_params).  Without a model
- * the default plan is used.  With the measured check (qcs_ext_planner_set_check, on by
+ * mode 3 uses the default plan, and modes 1 and 2 run circuit passes: a model there chooses
+ * among blocks and stages only, which take several times as long (33-qubit QFT in mode 2: 2.5 s
+ * with a model, 0.47 s as passes).  With the measured check (qcs_ext_planner_set_check, on by
  * default) the default plan also checks each override by measurement: a flush structure
  * keeps the model's choice only if it ran faster than the default plan.  The caller keeps
  * the model alive while it is attached. */

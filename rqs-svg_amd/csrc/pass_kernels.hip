@@ -530,7 +530,7 @@ namespace qsv
 
         // One tile of one of several circuits per workgroup (PassTask).  Bound by FP64 arithmetic
         // like k_pass: 96 circuits of 10-20 qubits run 8 rounds of up to 4172 tiles, 35 to 400 us
-        // each, and the whole circuits of up to 12 qubits beside the first; the batch takes 1.25
+        // each, and the whole circuits of up to 12 qubits beside the first; the batch takes 1.14
         // ms where per-block launches, stage rounds and the LDS kernel took 2.7.
         template <int M, bool NT>
         __global__ __launch_bounds__(1 << (M - 4), QSV_PASS_WAVES) void k_pass_tasks(const PassTask *__restrict__ tasks_, int ntasks, const PassRound *__restrict__ rounds, const PassOp *__restrict__ ops)
