@@ -514,7 +514,7 @@ namespace qcore
 
         // Which gates of `rem` can be applied with 2x2 targets in `targets` only; `no_control`: qubits
         // that a 2x2 other than a flip may not be controlled by.  Scans stop once no target is left
-        // that a later 2x2 could use, or `most` gates are taken.
+        // that a later 2x2 could use, or `most` 2x2s are taken.
         struct Frontier
         {
             uint64_t x = 0, z = 0; // qubits with a deferred 2x2 target, a deferred control or phase
@@ -557,10 +557,9 @@ namespace qcore
                     if (!(targets & ~(f.x | f.z)))
                         break;
                 }
-                else
+                else if (g.t >= 0)
                 {
-                    if (g.t >= 0)
-                        w += weight(g);
+                    w += weight(g);
                     if (--most == 0)
                         break;
                 }
@@ -603,7 +602,7 @@ namespace qcore
                     if (!((room > 0 ? set | (allowed & ~avoid) : set) & rem.targets() & ~(f.x | f.z)))
                         break;
                 }
-                else if (--most == 0)
+                else if (g.t >= 0 && --most == 0)
                     break;
             }
             return set;
@@ -620,21 +619,23 @@ namespace qcore
                     const bool ok = f.free(g) && (g.t < 0 || ((targets >> g.t) & 1)) && !(is_dense(g) && (g.cmask & no_control));
                     if (!ok)
                         f.defer(g);
+                    else if (g.t >= 0)
+                        --most;
                     return ok;
                 },
                 // with every target blocked nothing but phases could follow
-                [&](const PassGate &) { return taken.size() < most && (targets & ~(f.x | f.z)); });
+                [&](const PassGate &) { return most > 0 && (targets & ~(f.x | f.z)); });
         }
 
         // A phase can wait until a 2x2 needs one of its qubits: of the gates just taken, the phases
-        // that no later taken 2x2 waits for go back to rem (in order), unless nothing else was taken
-        // or is left.  They then join that 2x2's own phase instead of being multiplied in at the end
+        // that no later taken 2x2 waits for go back to rem (in order), unless only phases are
+        // left.  They then join that 2x2's own phase instead of being multiplied in at the end
         // of each round.
-        void put_back_phases(const std::vector<PassGate> &gates, std::vector<int> &taken, Remaining &rem, size_t most = ~size_t(0))
+        void put_back_phases(const std::vector<PassGate> &gates, std::vector<int> &taken, Remaining &rem)
         {
             if (rem.phases_only())
             {
-                rem.take_front(gates, taken, most - taken.size());
+                rem.take_front(gates, taken, rem.size());
                 return;
             }
             uint64_t needed = 0;
@@ -646,7 +647,7 @@ namespace qcore
                     needed |= bit(g.t);
                 (g.t >= 0 || (g.cmask & needed) ? keep : back).push_back(taken[i]);
             }
-            if (back.empty() || keep.empty())
+            if (back.empty())
                 return;
             std::reverse(keep.begin(), keep.end());
             std::reverse(back.begin(), back.end());
@@ -657,6 +658,17 @@ namespace qcore
         // Gates of a round: bounds its operations (at most two a gate, and the last flushes), so
         // that a round always fits the memory that programs pass through.
         constexpr size_t kRoundGates = (kProgramRoundOps - 2) / 2;
+
+        // Of more gates taken than a round holds, those past its end go back to rem.
+        void put_back_rest(const std::vector<PassGate> &gates, std::vector<int> &taken, Remaining &rem)
+        {
+            if (taken.size() <= kRoundGates)
+                return;
+            std::vector<int> back(taken.begin() + kRoundGates, taken.end());
+            taken.resize(kRoundGates);
+            std::sort(back.begin(), back.end()); // the circuit's order again
+            rem.put_back(gates, back);
+        }
 
         // Emits one round: register qubits reg[0..3] (ascending tile bits), the gates `taken`.
         void emit_round(PassPlan &P, const std::vector<PassGate> &gates, const uint8_t *tq, int m, uint32_t regbits, const std::vector<int> &taken)
@@ -846,7 +858,8 @@ namespace qcore
                 take(gates, rem, best, best, taken, kRoundGates);
                 if (taken.empty())
                     throw std::runtime_error("pass: planning does not advance");
-                put_back_phases(gates, taken, rem, kRoundGates);
+                put_back_phases(gates, taken, rem);
+                put_back_rest(gates, taken, rem);
                 if (first && (best & low))
                     emit_round(P, gates, tq, m, bits_of(top), {});
                 emit_round(P, gates, tq, m, bits_of(best), taken);

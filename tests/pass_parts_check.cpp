@@ -61,11 +61,12 @@ int main(int argc, char **argv)
     struct Case
     {
         int n, m, gates;
-        enum { Any, Phases, Flips } kind;
+        enum { Any, Phases, Flips, PhasesFirst } kind;
     };
     // one tile and many; any gates, doubly controlled phases, and Hadamards
-    // and CNOTs, which all run in one round where 4 qubits are all there are
-    for (const Case &k : {Case{4, 10, 1500, Case::Flips}, {4, 10, 1500, Case::Any}, {9, 10, 2500, Case::Any}, {5, 10, 1400, Case::Phases}, {12, 12, 1200, Case::Any}, {12, 12, 6000, Case::Flips}, {13, 11, 1500, Case::Any}, {14, 11, 700, Case::Phases}})
+    // and CNOTs, which all run in one round where 4 qubits are all there are; 400 phases before 100
+    // other gates, and 400 after them
+    for (const Case &k : {Case{4, 10, 1500, Case::Flips}, {4, 10, 1500, Case::Any}, {9, 10, 2500, Case::Any}, {5, 10, 1400, Case::Phases}, {12, 12, 1200, Case::Any}, {12, 12, 6000, Case::Flips}, {13, 11, 1500, Case::Any}, {14, 11, 700, Case::Phases}, {6, 10, 900, Case::PhasesFirst}, {14, 11, 900, Case::PhasesFirst}})
     {
         const int c = k.n;
         PassLowering lowering(k.n);
@@ -76,8 +77,9 @@ int main(int argc, char **argv)
             for (double &p : prm)
                 p = 6.283 * unif(seed) - 3.14;
             ResolvedGate g;
-            const int nc = k.kind == Case::Phases ? 2 : int(mix(seed) % 2);
-            g.spec = make_gate(k.kind == Case::Phases ? "p" : k.kind == Case::Flips ? (nc ? "x" : "h") : kNames[mix(seed) % 21], prm);
+            const bool phase = k.kind == Case::Phases || (k.kind == Case::PhasesFirst && (i < 400 || i >= 500));
+            const int nc = phase ? 2 : int(mix(seed) % 2);
+            g.spec = make_gate(phase ? "p" : k.kind == Case::Flips ? (nc ? "x" : "h") : kNames[mix(seed) % 21], prm);
             int qs[64];
             for (int q = 0; q < k.n; ++q)
                 qs[q] = q;
