@@ -234,11 +234,11 @@ namespace qcore
         // 4-6 qubits and 150 layers 2.4, 4.0 and 1.8 ms; 256 of 8-14 and 6 layers 4.7, 6.1 and 4.5.)
         std::vector<PassPlan> plans(circuits_.size());
         size_t gates = 0;
-        int kinds[4] = {}; // up to 10, 11, 12 and more qubits
+        int kinds[5] = {}; // up to 10, 11, 12 and more qubits, and those that run as stages
         for (const Circuit &C : circuits_)
         {
             gates += C.gates.size();
-            ++kinds[std::clamp(C.n, qsv::kPassMinBits, qsv::kPassMaxBits + 1) - qsv::kPassMinBits];
+            ++kinds[x3_ && C.n > T.lds_max_qubits ? 4 : std::clamp(C.n, qsv::kPassMinBits, qsv::kPassMaxBits + 1) - qsv::kPassMinBits];
         }
         if (passes_)
             for_each_circuit(circuits_.size(), std::min<size_t>(16, gates / 512), [&](size_t ci) {
@@ -262,7 +262,7 @@ namespace qcore
                 // 255), 64 of 13-18 396 (418), 256 of 13-15 380 (415).
                 if (!low.empty())
                     plans[ci] = plan_passes(low, C.n, std::clamp(C.n, qsv::kPassMinBits, qsv::kPassMaxBits), 8);
-            }, [&] { make_streams(std::min(kinds[0], 1) + std::min(kinds[1], 1) + std::min(kinds[2], 1) + std::min(kinds[3], 2)); });
+            }, [&] { make_streams(std::min(kinds[0], 1) + std::min(kinds[1], 1) + std::min(kinds[2], 1) + std::min(kinds[3], 2) + std::min(kinds[4], 1)); });
         for (int ci = 0; ci < (int)circuits_.size(); ++ci)
         {
             const Circuit &C = circuits_[ci];
