@@ -336,6 +336,7 @@ namespace qcore
         std::vector<Blocked> blocked;
         std::vector<float> mats;
         ComposeList compose;
+        compose.apart = true;
         for (int ci : large)
         {
             const Circuit &C = circuits_[ci];
@@ -587,8 +588,18 @@ namespace qcore
             };
             zsum_offset = append(zt.data(), zt.size() * sizeof(qsv::ZsumTask));
         }
-        compose.append(mats);
-        upload((void **)&d_mats_, mats.data(), mats.size() * sizeof(float));
+        const size_t room_at = compose.append(mats);
+        for (const auto &sc : staged)
+            for (const auto &st : sc.stages)
+                move_matrices(st, room_at, mats);
+        for (auto &bc : blocked)
+            for (auto &b : bc.blocks)
+                b.matrix_offset += room_at;
+        if (!mats.empty())
+        {
+            qsv::check(hipMalloc((void **)&d_mats_, (compose.room > 0 ? room_at + compose.room : mats.size()) * sizeof(float)), "hipMalloc batch");
+            qsv::check(hipMemcpy(d_mats_, mats.data(), mats.size() * sizeof(float), hipMemcpyHostToDevice), "batch upload");
+        }
         // algorithmic traffic and launches of one run (see qcs_ext_batch_traffic)
         hbm_bytes_ = 0;
         launches_ = small.empty() ? 0 : 2;

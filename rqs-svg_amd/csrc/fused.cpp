@@ -303,10 +303,20 @@ namespace qcore
         }
     }
 
-    void ComposeList::append(std::vector<float> &mats)
+    size_t ComposeList::place(std::vector<float> &mats, size_t count)
+    {
+        const size_t at = apart ? room : mats.size();
+        if (apart)
+            room += count;
+        else
+            mats.resize(at + count);
+        return at;
+    }
+
+    size_t ComposeList::append(std::vector<float> &mats)
     {
         if (jobs.empty())
-            return;
+            return 0;
         auto put = [&](const void *src, size_t bytes) {
             while (mats.size() % 4)
                 mats.push_back(0.f);
@@ -316,10 +326,20 @@ namespace qcore
                 std::memcpy(mats.data() + off, src, bytes);
             return off;
         };
-        jobs_at_ = put(jobs.data(), jobs.size() * sizeof(qsv::ComposeJob));
         gates_at_ = put(gates.data(), gates.size() * sizeof(qsv::ComposeGate));
         diagonals_at_ = put(diagonals.data(), diagonals.size() * sizeof(qsv::ComposeDiagonal));
         coefs_at_ = put(coefs.data(), coefs.size() * sizeof(cd));
+        jobs_at_ = put(jobs.data(), jobs.size() * sizeof(qsv::ComposeJob));
+        if (room == 0)
+            return 0;
+        const size_t base = (mats.size() + 63) & ~size_t(63);
+        if (base + room > size_t(1) << 32)
+            throw std::runtime_error("compose: block or buffer too large");
+        for (auto &j : jobs)
+            if (j.kind != qsv::kComposeTable)
+                j.dst += uint32_t(base);
+        std::memcpy(mats.data() + jobs_at_, jobs.data(), jobs.size() * sizeof(qsv::ComposeJob));
+        return base;
     }
 
     void ComposeList::launch(hipStream_t s, float *mats_dev) const
@@ -1144,12 +1164,17 @@ namespace qcore
             PreparedBlock b;
             b.kq = kq;
             b.gates = (int)pb.gates.size();
-            b.matrix_offset = mats.size();
-            mats.resize(mats.size() + per);
             if (compose)
+            {
+                b.matrix_offset = compose->place(mats, per);
                 compose->matrix(gates, pb, lay, b.matrix_offset, x3);
+            }
             else
+            {
+                b.matrix_offset = mats.size();
+                mats.resize(mats.size() + per);
                 write_matrix(block_matrix(gates, pb, lay), kq, x3, mats.data() + b.matrix_offset);
+            }
             std::vector<int> outside = lay.pos_out;
             outside.insert(outside.end(), lay.neg_out.begin(), lay.neg_out.end());
             uint64_t setb = 0;
@@ -1539,12 +1564,18 @@ namespace qcore
         {
             if (first_trail == 0 && compose)
                 break; // the table alone is read
-            desc[i].matrix = uint32_t(mats.size());
-            mats.resize(mats.size() + per);
             if (compose)
-                compose->matrix(sub, plan[i], lays[i], desc[i].matrix, x3);
+            {
+                const size_t at = compose->place(mats, per);
+                desc[i].matrix = uint32_t(at);
+                compose->matrix(sub, plan[i], lays[i], at, x3);
+            }
             else
+            {
+                desc[i].matrix = uint32_t(mats.size());
+                mats.resize(mats.size() + per);
                 write_matrix(block_matrix(sub, plan[i], lays[i]), kq, x3, mats.data() + desc[i].matrix);
+            }
         }
         static_assert(sizeof(qsv::StageBlock) % 16 == 0, "StageBlock keeps 16-B alignment");
         PreparedStage p;
@@ -1600,6 +1631,18 @@ namespace qcore
         mats.resize(mats.size() + desc.size() * sizeof(qsv::StageBlock) / sizeof(float));
         std::memcpy(mats.data() + p.desc_offset, desc.data(), desc.size() * sizeof(qsv::StageBlock));
         return p;
+    }
+
+    void move_matrices(const PreparedStage &p, size_t by, std::vector<float> &mats)
+    {
+        for (int i = 0; i < p.nblocks; ++i)
+        {
+            qsv::StageBlock sb;
+            float *at = mats.data() + p.desc_offset + size_t(i) * (sizeof sb / sizeof(float));
+            std::memcpy(&sb, at, sizeof sb);
+            sb.matrix += uint32_t(by);
+            std::memcpy(at, &sb, sizeof sb);
+        }
     }
 
     int stage64_lds_blocks(const std::vector<ResolvedGate> &gates, int kq) { return stage128_lds_blocks(gates, kq); }

@@ -44,8 +44,15 @@ namespace qcore
 
     // Matrices and tables of a flush that the device composes: filled by prepare_blocks and
     // prepare_stage, which then only leave room for them in `mats`.
+    // apart: the matrices' room (not the tables') is behind `mats`, where the host neither holds
+    // nor uploads it; their offsets count from its start until append says where that is.  For
+    // batches, whose matrices are tens of MB: host memory for them is mapped page by page at each
+    // growth.  (First run of 256 circuits of 6-16 qubits in BF16x3: 14.5 ms with that memory from
+    // malloc's heap, 20 to 27 where malloc maps it, 13.0 so.)
     struct ComposeList
     {
+        bool apart = false;
+        size_t room = 0; // floats taken apart
         std::vector<qsv::ComposeJob> jobs;
         std::vector<qsv::ComposeGate> gates;
         std::vector<qsv::ComposeDiagonal> diagonals;
@@ -54,8 +61,11 @@ namespace qcore
         void matrix(const std::vector<ResolvedGate> &gates, const PlannedBlock &b, const BlockLayout &lay, size_t dst, bool x3);
         // the product table of diagonals over 2^m indices; bpos[i]: tile bits of diagonal i's bits
         void table(const std::vector<std::vector<cd>> &diags, const std::vector<std::vector<int>> &bpos, int m, size_t dst);
-        // Appends the list to `mats`, and launches it on the uploaded copy.
-        void append(std::vector<float> &mats);
+        // the place of a matrix of `count` floats
+        size_t place(std::vector<float> &mats, size_t count);
+        // Appends the list to `mats`, and launches it on the uploaded copy.  Returns where the room
+        // apart begins in the buffer (floats; 0 if there is none), for move_matrices.
+        size_t append(std::vector<float> &mats);
         void launch(hipStream_t s, float *mats_dev) const;
 
     private:
@@ -146,6 +156,8 @@ namespace qcore
     // blocks only then runs as that table alone, another applies it as its tiles are stored.
     // compose: as for prepare_blocks, the table too.
     PreparedStage prepare_stage(const std::vector<ResolvedGate> &gates, const PlannedStage &st, int kq, int m, int n, std::vector<float> &mats, bool x3, bool table = false, ComposeList *compose = nullptr);
+    // Adds `by` to the stage's matrix offsets, in its descriptors in `mats`.
+    void move_matrices(const PreparedStage &p, size_t by, std::vector<float> &mats);
     // Blocks a complex64 stage with tables runs through LDS (as stage128_lds_blocks).
     int stage64_lds_blocks(const std::vector<ResolvedGate> &gates, int kq);
     // The stage's task on `state` as the launch's tiles from tile_begin on (checked).
